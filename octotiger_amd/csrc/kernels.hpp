@@ -19,20 +19,46 @@ namespace octofmm {
 // ---------------------------------------------------------------------------
 // Pair arithmetic
 //
-// Partner records carry the multiplicity factors of the contraction folded
-// into the multipole: m4, m7, m9 are stored halved (factor_half) and the
-// octupole m10..m19 scaled by factor_sixth = {1,3,3,3,6,3,1,3,3,1}/6, so every
-// term of the contraction is one fused multiply-add.  The target's own
-// octupole used by the angular-momentum correction carries the same scaling,
-// which makes the scaled octupole difference directly the correction weight.
+// The derivatives of -1/r are harmonic, so every trace over two of their
+// indices vanishes: at separation x, with d1 = 1/r^3, d2 = -3/r^5, d3 = 15/r^7,
+// 3 d1 + d2 r^2 = 0 and 5 d2 + d3 r^2 = 0.  The pair functions therefore never
+// form the tensors D_ab and D_abc.  They contract the partner's moments with
+// the separation (vectors Q x, scalars x Q x, p x, B x x x) and accumulate
+// sums of a few radial powers times those, from which a target's expansion is
+// formed once, after its last pair (acc_finish):
+//   - only the trace-free parts of the quadrupole Q and of the octupole B act
+//     on L, so the staged record holds those;
+//   - L_ab and L_abc are the trace-free parts of the sums R_ab (Acc::hd, ho)
+//     and T_abc (Acc::t), which leave out every term that only adds a trace;
+//   - the angular-momentum correction uses the order-4 derivatives without
+//     their d4 term, -[d2 tau_d + d3 (B_dbc x_b x_c + x_d tau x)] with tau the
+//     trace of B.  Split into trace-free part and trace, the d2 term cancels:
+//     -d3 [B0_dbc x_b x_c + 7/5 x_d tau x];
+//   - the target's own octupole enters the correction linearly, as the mass
+//     ratio m0 / mc0 times the same form, so its part needs only the sums
+//     W_bc = sum m0 d3 x_b x_c.
+// FP64 VALU issue bounds the level kernels, so the instructions per pair are
+// what counts: 115 (RHO) and 102 (DRHODT) per far pair, where forming the
+// tensors took 177 and 132.  A pass over 4096 sub-grids went 2.97 -> 2.19 ms
+// (RHO) and 2.42 -> 2.00 ms (DRHODT), over 512 0.386 -> 0.293 ms, with the
+// errors against 64-bit sums no larger.  The identities hold for separations
+// above the floor r^2 >= 1e-20, which exists so that a pair of coincident
+// empty cells gives zero, not NaN.
+//
+// Powers: one Newton step of the hardware estimate gives P = 2/r (rsqrt2), and
+// d1' = P^3, e2 = P^5, e3 = P^7 carry the factors 8, 32, 128, which the
+// record's scales and acc_finish take back.
+//
+// Record of one partner cell, 24 doubles:
+//   0      m0
+//   1..3   5/4 p
+//   4..8   15/32 of the trace-free M_ab: xx xy xz yy yz
+//   9..20  RHO: 5/64 of the trace-free part of M_abc, xxx xyy xzz xxy yyy yzz
+//          xxz yyz xyz, then 7/10 of the trace of 5/64 M_abc
+//          DRHODT: the same trace-free part as the coefficients of the 8 cubic
+//          monomials of cubic_monomials (9..16), zeros
+//   21..23 centre of mass
 // ---------------------------------------------------------------------------
-__host__ __device__ constexpr double record_scale(int c) {
-    return (c == 4 || c == 7 || c == 9) ? 0.5
-        : (c == 10 || c == 16 || c == 19) ? 1.0 / 6.0
-        : (c == 14) ? 1.0
-        : (c >= 11 && c <= 18) ? 0.5
-        : 1.0;
-}
 
 // Sum over the 8 lanes of an aligned group, by three DPP lane moves (VALU ops,
 // no LDS round trip): the pair of xor 1, the pair of xor 2 within each quad,
@@ -55,166 +81,180 @@ __device__ __forceinline__ double sum8(double v) {
     return v;
 }
 
-struct DTensor {
-    double D[20];
-    double d2, d3;
-    // d3 times monomials of the separation, shared with the correction
-    double d3x00, d3x11, d3x22, d3x01, d3x02, d3x12;
+// 2/sqrt(x): the hardware estimate (relative error <= 5.2e-8, measured on
+// MI355X over x in [1e-12, 1e6]) refined by one Newton step, which squares the
+// error: <= 4.1e-15 (a second step would give 1.4e-16).  The expansion's
+// highest power scales it by at most 7, far inside the 1e-12 gate.  Without
+// the step's factor 1/2 it is one instruction shorter.
+__device__ __forceinline__ double rsqrt2(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    return y * fma(-(x * y), y, 3.0);
+}
+
+// Running sums of one target cell over its partners (see the top of the
+// file); scales as acc_finish takes them.
+template <bool RHO>
+struct Acc {
+    double a0, aq;      // potential
+    double l[3];        // gradient
+    double hd[3], ho[3];   // second order: diagonal xx yy zz, off-diagonal xy xz yz
+    double t[8];        // third order
+    double u[RHO ? 9 : 3];   // RHO: W xx yy zz xy xz yz, correction; DRHODT: dipole rows
 };
 
-// 1/sqrt(x): the hardware estimate (relative error <= 5.2e-8, measured on
-// MI355X over x in [1e-12, 1e6]) refined by one Newton step, which squares the
-// error: <= 4.1e-15 measured (a second step would give 1.4e-16).  The
-// derivative tensor scales it by at most 7 (d3 ~ r^-7), far inside the 1e-12
-// gate, and the step saves three instructions per pair.
-__device__ __forceinline__ double rsqrt_nr(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-((0.5 * x) * y), y, 0.5);
-    return fma(y, e, y);
+template <bool RHO>
+__device__ __forceinline__ void acc_clear(Acc<RHO>& s) {
+    s.a0 = s.aq = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) s.l[i] = s.hd[i] = s.ho[i] = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s.t[i] = 0.0;
+#pragma unroll
+    for (int i = 0; i < (RHO ? 9 : 3); ++i) s.u[i] = 0.0;
 }
 
-// Derivatives of -1/r up to order 3 at dX (compute_d_factors), with the
+// Squares of the separation and the radial powers of a pair, with the
 // reference's floor r^2 >= 1e-20.
-__device__ __forceinline__ void d_tensor(double x, double y, double z, DTensor& t) {
-    const double x00 = x * x;
-    double r2 = fma(z, z, fma(y, y, x00));
-    r2 = fmax(r2, 1.0e-20);   // one v_max_f64; r2 of finite separations is never NaN
-    const double ri = rsqrt_nr(r2);           // 1/r
-    const double r2inv = ri * ri;
-    const double d1 = ri * r2inv;             // 1/r^3
-    const double d2 = (-3.0 * r2inv) * d1;    // -3/r^5
-    const double d3 = (-5.0 * r2inv) * d2;    // 15/r^7
-    t.d2 = d2;
-    t.d3 = d3;
-    double* D = t.D;
-    D[0] = -ri;
-    D[1] = x * d1;
-    D[2] = y * d1;
-    D[3] = z * d1;
-    const double d2x = d2 * x, d2y = d2 * y, d2z = d2 * z;
-    // second order from the d2 x_a products the order-3 terms need anyway
-    D[4] = fma(d2, x00, d1);
-    D[5] = d2x * y;
-    D[6] = d2x * z;
-    D[7] = fma(d2y, y, d1);
-    D[8] = d2y * z;
-    D[9] = fma(d2z, z, d1);
-    const double d3x = d3 * x, d3y = d3 * y;
-    const double d3x00 = d3x * x, d3x11 = d3y * y, d3x22 = (d3 * z) * z;
-    const double d3x01 = d3x * y, d3x02 = d3x * z, d3x12 = d3y * z;
-    t.d3x00 = d3x00;
-    t.d3x11 = d3x11;
-    t.d3x22 = d3x22;
-    t.d3x01 = d3x01;
-    t.d3x02 = d3x02;
-    t.d3x12 = d3x12;
-    D[10] = fma(d3x00, x, 3.0 * d2x);
-    D[11] = fma(d3x00, y, d2y);
-    D[12] = fma(d3x00, z, d2z);
-    D[13] = fma(d3x11, x, d2x);
-    D[14] = d3x12 * x;
-    D[15] = fma(d3x22, x, d2x);
-    D[16] = fma(d3x11, y, 3.0 * d2y);
-    D[17] = fma(d3x11, z, d2z);
-    D[18] = fma(d3x22, y, d2y);
-    D[19] = fma(d3x22, z, 3.0 * d2z);
+struct Radial {
+    double xx, yy, zz;
+    double P, d1, e2, e3;   // 2/r and its powers 3, 5, 7
+};
+
+__device__ __forceinline__ void radial_powers(double P, Radial& g) {
+    const double rho = P * P;
+    g.P = P;
+    g.d1 = P * rho;
+    g.e2 = rho * g.d1;
+    g.e3 = rho * g.e2;
 }
 
-// Order-2/3 part of the contraction (compute_interaction_multipole_non_rho)
-// with factor-scaled partner components m.  NCOMP == 4: potential and
-// gradient rows only (p2m targets).
-template <int NCOMP>
-__device__ __forceinline__ void contract_high(const double* m, const double* D, double* L) {
-    double l0 = L[0], l1 = L[1], l2 = L[2], l3 = L[3];
-    l0 = fma(m[4], D[4], l0);   l1 = fma(m[4], D[10], l1);  l2 = fma(m[4], D[11], l2);  l3 = fma(m[4], D[12], l3);
-    l0 = fma(m[5], D[5], l0);   l1 = fma(m[5], D[11], l1);  l2 = fma(m[5], D[13], l2);  l3 = fma(m[5], D[14], l3);
-    l0 = fma(m[6], D[6], l0);   l1 = fma(m[6], D[12], l1);  l2 = fma(m[6], D[14], l2);  l3 = fma(m[6], D[15], l3);
-    l0 = fma(m[7], D[7], l0);   l1 = fma(m[7], D[13], l1);  l2 = fma(m[7], D[16], l2);  l3 = fma(m[7], D[17], l3);
-    l0 = fma(m[8], D[8], l0);   l1 = fma(m[8], D[14], l1);  l2 = fma(m[8], D[17], l2);  l3 = fma(m[8], D[18], l3);
-    l0 = fma(m[9], D[9], l0);   l1 = fma(m[9], D[15], l1);  l2 = fma(m[9], D[18], l2);  l3 = fma(m[9], D[19], l3);
-#pragma unroll
-    for (int k = 10; k < 20; ++k) l0 = fma(-m[k], D[k], l0);
-    L[0] = l0; L[1] = l1; L[2] = l2; L[3] = l3;
-    if constexpr (NCOMP == 20) {
-        // L_ab += m0 D_ab - m_c D_abc
-        L[4] = fma(m[0], D[4], L[4]); L[4] = fma(-m[1], D[10], L[4]); L[4] = fma(-m[2], D[11], L[4]); L[4] = fma(-m[3], D[12], L[4]);
-        L[5] = fma(m[0], D[5], L[5]); L[5] = fma(-m[1], D[11], L[5]); L[5] = fma(-m[2], D[13], L[5]); L[5] = fma(-m[3], D[14], L[5]);
-        L[6] = fma(m[0], D[6], L[6]); L[6] = fma(-m[1], D[12], L[6]); L[6] = fma(-m[2], D[14], L[6]); L[6] = fma(-m[3], D[15], L[6]);
-        L[7] = fma(m[0], D[7], L[7]); L[7] = fma(-m[1], D[13], L[7]); L[7] = fma(-m[2], D[16], L[7]); L[7] = fma(-m[3], D[17], L[7]);
-        L[8] = fma(m[0], D[8], L[8]); L[8] = fma(-m[1], D[14], L[8]); L[8] = fma(-m[2], D[17], L[8]); L[8] = fma(-m[3], D[18], L[8]);
-        L[9] = fma(m[0], D[9], L[9]); L[9] = fma(-m[1], D[15], L[9]); L[9] = fma(-m[2], D[18], L[9]); L[9] = fma(-m[3], D[19], L[9]);
-#pragma unroll
-        for (int i = 10; i < 20; ++i) L[i] = fma(m[0], D[i], L[i]);
-    }
+__device__ __forceinline__ void radial(double x, double y, double z, Radial& g) {
+    g.xx = x * x;
+    g.yy = y * y;
+    g.zz = z * z;
+    const double r2 = fmax(g.xx + g.yy + g.zz, 1.0e-20);   // one v_max_f64; r2 of finite separations is never NaN
+    radial_powers(rsqrt2(r2), g);
+}
+
+// Record fields by index from the 12 double2 of a record.
+__device__ __forceinline__ double rec_at(const double2* v, int i) { return (i & 1) ? v[i >> 1].y : v[i >> 1].x; }
+
+// Potential and gradient rows of mass and quadrupole.
+template <bool RHO>
+__device__ __forceinline__ void add_gradient(const double2* v, double x, double y, double z, const Radial& g, double e2x,
+    Acc<RHO>& s) {
+    const double m0 = rec_at(v, 0);
+    const double qxx = rec_at(v, 4), qxy = rec_at(v, 5), qxz = rec_at(v, 6), qyy = rec_at(v, 7), qyz = rec_at(v, 8);
+    const double qzz = -(qxx + qyy);
+    const double qx = fma(qxz, z, fma(qxy, y, qxx * x));
+    const double qy = fma(qyz, z, fma(qyy, y, qxy * x));
+    const double qz = fma(qzz, z, fma(qyz, y, qxz * x));
+    const double sq = fma(qz, z, fma(qy, y, qx * x));
+    s.a0 = fma(m0, g.P, s.a0);
+    s.aq = fma(g.e2, sq, s.aq);
+    const double e = fma(g.e3, sq, m0 * g.d1);
+    s.l[0] = fma(-e2x, qx, fma(e, x, s.l[0]));
+    s.l[1] = fma(-e2x, qy, fma(e, y, s.l[1]));
+    s.l[2] = fma(-e2x, qz, fma(e, z, s.l[2]));
+}
+
+// z_a x_b + z_b x_a of the second-order sums (z_a x_a on the diagonal).
+template <bool RHO>
+__device__ __forceinline__ void add_second(double zx, double zy, double zz, double x, double y, double z, Acc<RHO>& s) {
+    s.hd[0] = fma(zx, x, s.hd[0]);
+    s.hd[1] = fma(zy, y, s.hd[1]);
+    s.hd[2] = fma(zz, z, s.hd[2]);
+    s.ho[0] = fma(zy, x, fma(zx, y, s.ho[0]));
+    s.ho[1] = fma(zz, x, fma(zx, z, s.ho[1]));
+    s.ho[2] = fma(zz, y, fma(zy, z, s.ho[2]));
+}
+
+// Quadratic monomials of the trace-free octupole forms, B_dbc x_b x_c / 2 =
+// B_dxx h1 + B_dyy h2 + B_dxy xy + B_dxz xz + B_dyz yz.
+struct Quadratic {
+    double h1, h2, xy, xz, yz;
+};
+
+__device__ __forceinline__ Quadratic quadratic(double x, double y, double z, const Radial& g) {
+    Quadratic q;
+    const double h = 0.5 * g.zz;
+    q.h1 = fma(0.5, g.xx, -h);
+    q.h2 = fma(0.5, g.yy, -h);
+    q.xy = x * y;
+    q.xz = x * z;
+    q.yz = y * z;
+    return q;
+}
+
+// b: xxx xyy xzz xxy yyy yzz xxz yyz xyz
+__device__ __forceinline__ void octupole_vector(const double* b, const Quadratic& q, double* v) {
+    v[0] = fma(b[8], q.yz, fma(b[6], q.xz, fma(b[3], q.xy, fma(b[1], q.h2, b[0] * q.h1))));
+    v[1] = fma(b[7], q.yz, fma(b[8], q.xz, fma(b[1], q.xy, fma(b[4], q.h2, b[3] * q.h1))));
+    v[2] = fma(b[5], q.yz, fma(b[2], q.xz, fma(b[8], q.xy, fma(b[7], q.h2, b[6] * q.h1))));
+}
+
+// Partner part of the correction (and, with the potential a0, the partner's
+// octupole on it): c += e3 (v + x tau x).
+__device__ __forceinline__ void add_correction(const double* b, const double* tau, double x, double y, double z,
+    const Quadratic& q, double e3, double* a0, double* c) {
+    double v[3];
+    octupole_vector(b, q, v);
+    if (a0) *a0 = fma(e3, fma(v[2], z, fma(v[1], y, v[0] * x)), *a0);
+    const double tx = fma(tau[2], z, fma(tau[1], y, tau[0] * x));
+    c[0] = fma(e3, fma(x, tx, v[0]), c[0]);
+    c[1] = fma(e3, fma(y, tx, v[1]), c[1]);
+    c[2] = fma(e3, fma(z, tx, v[2]), c[2]);
+}
+
+// W += m0 e3 x x, the sums the target's own octupole meets.
+__device__ __forceinline__ void add_w(double g3, const Radial& g, const Quadratic& q, double* w) {
+    w[0] = fma(g3, g.xx, w[0]);
+    w[1] = fma(g3, g.yy, w[1]);
+    w[2] = fma(g3, g.zz, w[2]);
+    w[3] = fma(g3, q.xy, w[3]);
+    w[4] = fma(g3, q.xz, w[4]);
+    w[5] = fma(g3, q.yz, w[5]);
+}
+
+// Third-order sums of the RHO kernels.
+__device__ __forceinline__ void add_third(double g3, double x, double y, double z, const Radial& g, const Quadratic& q,
+    double* t) {
+    const double gx = g3 * x, gy = g3 * y, gz = g3 * z;
+    t[0] = fma(gx, q.h1 - g.zz, t[0]);
+    t[1] = fma(gx, q.h2, t[1]);
+    t[2] = fma(gy, q.h1, t[2]);
+    t[3] = fma(gy, q.h2 - g.zz, t[3]);
+    t[4] = fma(gz, q.h1, t[4]);
+    t[5] = fma(gz, q.h2, t[5]);
+    t[6] = fma(gz, g.zz, t[6]);
+    t[7] = fma(gx, q.yz, t[7]);
+}
+
+// The 8 cubic monomials that both the third-order sums and the octupole's
+// potential of the DRHODT kernels use (twice those of add_third, but for the
+// last two).
+__device__ __forceinline__ void cubic_monomials(double x, double y, double z, const Radial& g, double* c) {
+    const double h1 = g.xx - g.zz, h2 = g.yy - g.zz;
+    c[0] = x * fma(-2.0, g.zz, h1);
+    c[1] = x * h2;
+    c[2] = y * h1;
+    c[3] = y * fma(-2.0, g.zz, h2);
+    c[4] = z * h1;
+    c[5] = z * h2;
+    c[6] = z * g.zz;
+    c[7] = x * (y * z);
 }
 
 // Dipole rows of the DRHODT kernels (compute_kernel_non_rho, :374-389).  The
 // reference subtracts the whole first row of the second-order tensor from
 // each gradient component; kept as is.
-__device__ __forceinline__ void dipole_rows(const double* m, const double* D, double* L) {
-    L[0] = fma(-m[1], D[1], L[0]);
-    L[0] = fma(-m[2], D[2], L[0]);
-    L[0] = fma(-m[3], D[3], L[0]);
-    L[1] = fma(-m[1], D[4] + D[5] + D[6], L[1]);
-    L[2] = fma(-m[2], D[5] + D[7] + D[8], L[2]);
-    L[3] = fma(-m[3], D[6] + D[8] + D[9], L[3]);
-}
-
-// Angular-momentum correction from the order-4 tensor (compute_interaction_multipole_rho,
-// :224-334; compute_interaction_p2m_rho, monopole_kernel_templates.hpp:69-187).
-// a[k] = factor-scaled octupole difference (M2L) or partner octupole (p2m).
-__device__ __forceinline__ void am_correction_t(double d2, double d3x00, double d3x11, double d3x22, double d3x01,
-    double d3x02, double d3x12, const double* a, double* C) {
-    // 6.0 in a scalar register pair: as a literal it makes the compiler use
-    // the two-operand FMA, whose tied destination costs a register copy for
-    // each of U0 and U10 (the three-operand form takes no 64-bit literal)
-    double six = 6.0;
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+s"(six));
-#endif
-    const double t2 = 3.0 * d2;
-    const double U0 = fma(six, d3x00, t2);
-    const double U1 = 3.0 * d3x01;
-    const double U2 = 3.0 * d3x02;
-    const double U3 = d2 + d3x11 + d3x00;
-    const double U4 = d3x12;
-    const double U5 = d2 + d3x22 + d3x00;
-    const double U7 = d3x02;
-    const double U8 = d3x01;
-    const double U10 = fma(six, d3x11, t2);
-    const double U12 = d2 + d3x22 + d3x11;
-    const double U13 = 3.0 * d3x12;
-    const double U14 = fma(six, d3x22, t2);
-    double c0 = C[0], c1 = C[1], c2 = C[2];
-    c0 = fma(-a[0], U0, c0);  c1 = fma(-a[0], U1, c1);  c2 = fma(-a[0], U2, c2);
-    c0 = fma(-a[1], U1, c0);  c1 = fma(-a[1], U3, c1);  c2 = fma(-a[1], U4, c2);
-    c0 = fma(-a[2], U2, c0);  c1 = fma(-a[2], U4, c1);  c2 = fma(-a[2], U5, c2);
-    c0 = fma(-a[3], U3, c0);  c1 = fma(-a[3], U1, c1);  c2 = fma(-a[3], U7, c2);
-    c0 = fma(-a[4], U4, c0);  c1 = fma(-a[4], U7, c1);  c2 = fma(-a[4], U8, c2);
-    c0 = fma(-a[5], U5, c0);  c1 = fma(-a[5], U8, c1);  c2 = fma(-a[5], U2, c2);
-    c0 = fma(-a[6], U1, c0);  c1 = fma(-a[6], U10, c1); c2 = fma(-a[6], U13, c2);
-    c0 = fma(-a[7], U7, c0);  c1 = fma(-a[7], U13, c1); c2 = fma(-a[7], U12, c2);
-    c0 = fma(-a[8], U8, c0);  c1 = fma(-a[8], U12, c1); c2 = fma(-a[8], U13, c2);
-    c0 = fma(-a[9], U2, c0);  c1 = fma(-a[9], U13, c1); c2 = fma(-a[9], U14, c2);
-    C[0] = c0; C[1] = c1; C[2] = c2;
-}
-
-// The same correction from the separation and d2, d3 (used where no
-// derivative tensor with the shared products is at hand).
-__device__ __forceinline__ void am_correction(double x, double y, double z, double d2, double d3,
-    const double* a, double* C) {
-    const double d3x = d3 * x, d3y = d3 * y;
-    am_correction_t(d2, d3x * x, d3y * y, (d3 * z) * z, d3x * y, d3x * z, d3y * z, a, C);
-}
-
-__device__ __forceinline__ void load_record20(const double* __restrict__ p, double* m) {
-    const double2* p2 = reinterpret_cast<const double2*>(p);
-#pragma unroll
-    for (int i = 0; i < 10; ++i) {
-        const double2 v = p2[i];
-        m[2 * i] = v.x;
-        m[2 * i + 1] = v.y;
-    }
+__device__ __forceinline__ void add_dipole_rows(const double2* v, double x, double y, double z, const Radial& g,
+    double px, Acc<false>& s) {
+    s.aq = fma(g.d1, px, s.aq);
+    const double es = -0.75 * (g.e2 * (x + y + z));
+    s.u[0] = fma(rec_at(v, 1), fma(es, x, g.d1), s.u[0]);
+    s.u[1] = fma(rec_at(v, 2), fma(es, y, g.d1), s.u[1]);
+    s.u[2] = fma(rec_at(v, 3), fma(es, z, g.d1), s.u[2]);
 }
 
 // A partner record held in registers (24 doubles as 12 double2).
@@ -228,31 +268,209 @@ __device__ __forceinline__ void load_rec(const double* __restrict__ p, Rec& r) {
     for (int i = 0; i < 12; ++i) r.v[i] = p2[i];
 }
 
-// One far M2L pair: partner record (m0, scaled M1..M19, Y, mon) onto the
-// target at X with mass reciprocal inv_mc0 and scaled octupole mc[0..9].
+// One far M2L pair: partner record r onto the target at X.
 template <bool RHO>
-__device__ __forceinline__ void m2l_far_rec(const Rec& r, double X0, double X1, double X2, double inv_mc0,
-    const double* mc, double* L, double* C) {
-    double m[20];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) {
-        m[2 * i] = r.v[i].x;
-        m[2 * i + 1] = r.v[i].y;
-    }
-    const double x = X0 - r.v[10].x, y = X1 - r.v[10].y, z = X2 - r.v[11].x;
-    DTensor t;
-    d_tensor(x, y, z, t);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) L[i] = fma(m[0], t.D[i], L[i]);
-    if constexpr (!RHO) dipole_rows(m, t.D, L);
-    contract_high<20>(m, t.D, L);
+__device__ __forceinline__ void m2l_far_rec(const Rec& r, double X0, double X1, double X2, Acc<RHO>& s) {
+    const double2* v = r.v;
+    const double x = X0 - rec_at(v, kRecY), y = X1 - rec_at(v, kRecY + 1), z = X2 - rec_at(v, kRecY + 2);
+    Radial g;
+    radial(x, y, z, g);
+    const double e2x = 1.6 * g.e2, m0 = rec_at(v, 0);
+    add_gradient<RHO>(v, x, y, z, g, e2x, s);
+    const double px = fma(rec_at(v, 3), z, fma(rec_at(v, 2), y, rec_at(v, 1) * x));
+    const double k = fma(g.e3, px, m0 * g.e2);
+    add_second<RHO>(fma(k, x, -(e2x * rec_at(v, 1))), fma(k, y, -(e2x * rec_at(v, 2))), fma(k, z, -(e2x * rec_at(v, 3))),
+        x, y, z, s);
+    const double g3 = m0 * g.e3;
     if constexpr (RHO) {
-        const double n0c = m[0] * inv_mc0;
-        double a[10];
+        const Quadratic q = quadratic(x, y, z, g);
+        add_third(g3, x, y, z, g, q, s.t);
+        add_w(g3, g, q, s.u);
+        double b[9], tau[3];
 #pragma unroll
-        for (int k = 0; k < 10; ++k) a[k] = fma(-mc[k], n0c, m[10 + k]);
-        am_correction_t(t.d2, t.d3x00, t.d3x11, t.d3x22, t.d3x01, t.d3x02, t.d3x12, a, C);
+        for (int i = 0; i < 9; ++i) b[i] = rec_at(v, 9 + i);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) tau[i] = rec_at(v, 18 + i);
+        add_correction(b, tau, x, y, z, q, g.e3, &s.a0, s.u + 6);
+    } else {
+        double c[8], o = 0.0;
+        cubic_monomials(x, y, z, g, c);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            s.t[i] = fma(g3, c[i], s.t[i]);
+            o = i == 0 ? rec_at(v, 9) * c[0] : fma(rec_at(v, 9 + i), c[i], o);
+        }
+        s.a0 = fma(g.e3, o, s.a0);
+        add_dipole_rows(v, x, y, z, g, px, s);
     }
+}
+
+// The same pair from a record in global memory.
+template <bool RHO>
+__device__ __forceinline__ void m2l_far(const double* __restrict__ p, double X0, double X1, double X2, Acc<RHO>& s) {
+    Rec r;
+    load_rec(p, r);
+    m2l_far_rec<RHO>(r, X0, X1, X2, s);
+}
+
+// One near pair with a monopole-only partner of mass mn at Y.
+template <bool RHO>
+__device__ __forceinline__ void m2l_near(double mn, double Y0, double Y1, double Y2, double X0, double X1,
+    double X2, Acc<RHO>& s) {
+    const double x = X0 - Y0, y = X1 - Y1, z = X2 - Y2;
+    Radial g;
+    radial(x, y, z, g);
+    s.a0 = fma(mn, g.P, s.a0);
+    const double e = mn * g.d1, k = mn * g.e2, g3 = mn * g.e3;
+    s.l[0] = fma(e, x, s.l[0]);
+    s.l[1] = fma(e, y, s.l[1]);
+    s.l[2] = fma(e, z, s.l[2]);
+    add_second<RHO>(k * x, k * y, k * z, x, y, z, s);
+    if constexpr (RHO) {
+        const Quadratic q = quadratic(x, y, z, g);
+        add_third(g3, x, y, z, g, q, s.t);
+        add_w(g3, g, q, s.u);
+    } else {
+        double c[8];
+        cubic_monomials(x, y, z, g, c);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s.t[i] = fma(g3, c[i], s.t[i]);
+    }
+}
+
+// The target's own octupole (its record trec, mass reciprocal inv_mc0) meets
+// the sums W; c = partner part in, whole correction out (scale of acc_finish).
+__device__ __forceinline__ void fold_w(const double* __restrict__ trec, double inv_mc0, const double* w, double* c) {
+    const Quadratic q = {0.5 * (w[0] - w[2]), 0.5 * (w[1] - w[2]), w[3], w[4], w[5]};
+    double b[9], v[3];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) b[i] = trec[9 + i];
+    octupole_vector(b, q, v);
+    const double t0 = trec[18], t1 = trec[19], t2 = trec[20];
+    v[0] = fma(t2, w[4], fma(t1, w[3], fma(t0, w[0], v[0])));
+    v[1] = fma(t2, w[5], fma(t1, w[1], fma(t0, w[3], v[1])));
+    v[2] = fma(t2, w[2], fma(t1, w[5], fma(t0, w[4], v[2])));
+#pragma unroll
+    for (int d = 0; d < 3; ++d) c[d] = fma(-inv_mc0, v[d], c[d]);
+}
+
+// Number of sums of a target after acc_fold.
+constexpr int kFolded = 21;
+
+// Folds a target's sums to the kFolded linear ones that partial sums of one
+// target add up in: potential, gradient 3, second order 6, third order 8,
+// correction 3 (zeros for DRHODT).
+template <bool RHO>
+__device__ __forceinline__ void acc_fold_expansion(const Acc<RHO>& s, double* f) {
+    f[0] = fma(0.2, s.aq, s.a0);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        f[1 + i] = RHO ? s.l[i] : fma(-0.8, s.u[i], s.l[i]);
+        f[4 + i] = s.hd[i];
+        f[7 + i] = s.ho[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[10 + i] = s.t[i];
+}
+
+template <bool RHO>
+__device__ __forceinline__ void acc_fold(const Acc<RHO>& s, const double* __restrict__ trec, double* f) {
+    acc_fold_expansion<RHO>(s, f);
+    if constexpr (RHO) {
+        double c[3] = {s.u[6], s.u[7], s.u[8]};
+        fold_w(trec, 1.0 / trec[0], s.u, c);
+        f[18] = c[0];
+        f[19] = c[1];
+        f[20] = c[2];
+    } else {
+        f[18] = f[19] = f[20] = 0.0;
+    }
+}
+
+constexpr double kCorrectionScale = -1.5;
+
+// Expansion and correction of a target from its folded sums.
+template <bool RHO>
+__device__ __forceinline__ void acc_finish(const double* f, double* L, double* C) {
+    L[0] = -0.5 * f[0];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) L[1 + i] = 0.125 * f[1 + i];
+    const double tr = (f[4] + f[5] + f[6]) * (1.0 / 3.0);
+    L[4] = -(3.0 / 32.0) * (f[4] - tr);
+    L[7] = -(3.0 / 32.0) * (f[5] - tr);
+    L[9] = -(3.0 / 32.0) * (f[6] - tr);
+    L[5] = -(3.0 / 64.0) * f[7];
+    L[6] = -(3.0 / 64.0) * f[8];
+    L[8] = -(3.0 / 64.0) * f[9];
+    const double k = 15.0 / 128.0, h = RHO ? 2.0 : 1.0;
+    const double* t = f + 10;
+    // T with its xzz, yzz components zero, less the trace part
+    const double xxx = h * t[0], xyy = h * t[1], xxy = h * t[2], yyy = h * t[3], xxz = h * t[4], yyz = h * t[5],
+                 zzz = -2.0 * t[6];
+    const double sx = 0.2 * (xxx + xyy), sy = 0.2 * (xxy + yyy), sz = 0.2 * (xxz + yyz + zzz);
+    L[10] = k * (xxx - 3.0 * sx);
+    L[11] = k * (xxy - sy);
+    L[12] = k * (xxz - sz);
+    L[13] = k * (xyy - sx);
+    L[14] = k * t[7];
+    L[15] = -k * sx;
+    L[16] = k * (yyy - 3.0 * sy);
+    L[17] = k * (yyz - sz);
+    L[18] = -k * sy;
+    L[19] = k * (zzz - 3.0 * sz);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) C[d] = RHO ? kCorrectionScale * f[18 + d] : 0.0;
+}
+
+// One p2m pair: refined-neighbour multipole record r onto a leaf cell at X
+// (compute_interaction_p2m_rho, monopole_kernel_templates.hpp:69-187): the
+// potential and gradient rows, and the partner part of the correction.
+template <bool RHO>
+__device__ __forceinline__ void p2m_pair_rec(const Rec& r, double X0, double X1, double X2, Acc<RHO>& s) {
+    const double2* v = r.v;
+    const double x = X0 - rec_at(v, kRecY), y = X1 - rec_at(v, kRecY + 1), z = X2 - rec_at(v, kRecY + 2);
+    Radial g;
+    radial(x, y, z, g);
+    add_gradient<RHO>(v, x, y, z, g, 1.6 * g.e2, s);
+    if constexpr (RHO) {
+        double b[9], tau[3];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) b[i] = rec_at(v, 9 + i);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) tau[i] = rec_at(v, 18 + i);
+        add_correction(b, tau, x, y, z, quadratic(x, y, z, g), g.e3, &s.a0, s.u + 6);
+    } else {
+        double c[8];
+        cubic_monomials(x, y, z, g, c);
+        double o = rec_at(v, 9) * c[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) o = fma(rec_at(v, 9 + i), c[i], o);
+        s.a0 = fma(g.e3, o, s.a0);
+        add_dipole_rows(v, x, y, z, g, fma(rec_at(v, 3), z, fma(rec_at(v, 2), y, rec_at(v, 1) * x)), s);
+    }
+}
+
+// L0..3 and the correction of a leaf target from its p2m sums.
+template <bool RHO>
+__device__ __forceinline__ void p2m_finish(const Acc<RHO>& s, double* L, double* C) {
+    L[0] = fma(-0.5, s.a0, -0.1 * s.aq);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        L[1 + i] = RHO ? 0.125 * s.l[i] : fma(-0.1, s.u[i], 0.125 * s.l[i]);
+        C[i] = RHO ? kCorrectionScale * s.u[6 + i] : 0.0;
+    }
+}
+
+// Multiplicity factors of the FP32 half of the mixed-precision pairs, folded
+// into the FP32 moments of the mixed record: m4, m7, m9 halved and the octupole
+// m10..m19 times {1,3,3,3,6,3,1,3,3,1}/6, so every term of its contraction is
+// one fused multiply-add.
+__host__ __device__ constexpr double record_scale(int c) {
+    return (c == 4 || c == 7 || c == 9) ? 0.5
+        : (c == 10 || c == 16 || c == 19) ? 1.0 / 6.0
+        : (c == 14) ? 1.0
+        : (c >= 11 && c <= 18) ? 0.5
+        : 1.0;
 }
 
 // FP32 half of a mixed-precision far pair: the derivative tensor of -1/r at
@@ -329,70 +547,47 @@ __device__ __forceinline__ float m2l_fp32_core(float x, float y, float z, const 
 
 // FP64 half of a mixed-precision far pair (RHO): the angular-momentum
 // correction at the FP64 separation, with 1/r refined from the FP32 estimate
-// ri by one FP64 Newton step, and the octupole difference formed from the
-// partner's FP64 mass m0 and scaled octupole oct[0..9].
-__device__ __forceinline__ void mixed_correction(double xd, double yd, double zd, float ri, double m0,
-    const double* oct, double inv_mc0, const double* mc, double* C) {
-    double r2d = fma(zd, zd, fma(yd, yd, xd * xd));
-    r2d = fmax(r2d, 1.0e-20);
-    double rid = (double)ri;
-    rid = fma(rid, fma(-(0.5 * r2d) * rid, rid, 0.5), rid);
-    const double r2i = rid * rid;
-    const double e1 = rid * r2i;
-    const double e2 = (-3.0 * r2i) * e1;
-    const double e3 = (-5.0 * r2i) * e2;
-    const double n0c = m0 * inv_mc0;
-    double a[10];
-#pragma unroll
-    for (int k = 0; k < 10; ++k) a[k] = fma(-mc[k], n0c, oct[k]);
-    am_correction(xd, yd, zd, e2, e3, a, C);
-}
-
-// Mixed precision far pair from an FP64 record (lane mapping 0): the
-// separation is formed in FP64 and rounded to FP32, the record's components
-// are rounded to FP32 for the derivative tensor and the 20-component
-// contraction, which accumulate into the FP32 partial sums Lf of the current
-// coarse offset (at most 8 pairs, added to the FP64 expansion by the caller).
-// The angular-momentum correction stays FP64 (mixed_correction).
-template <bool RHO>
-__device__ __forceinline__ void m2l_far_mixed(const Rec& r, double X0, double X1, double X2, double inv_mc0,
-    const double* mc, float* Lf, double* C) {
-    const double xd = X0 - r.v[10].x, yd = X1 - r.v[10].y, zd = X2 - r.v[11].x;
-    float m[20];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) {
-        m[2 * i] = (float)r.v[i].x;
-        m[2 * i + 1] = (float)r.v[i].y;
-    }
-    const float ri = m2l_fp32_core<RHO>((float)xd, (float)yd, (float)zd, m, Lf);
-    if constexpr (RHO) {
-        double oct[10];
-#pragma unroll
-        for (int k = 0; k < 10; ++k) oct[k] = (k & 1) ? r.v[5 + (k >> 1)].y : r.v[5 + (k >> 1)].x;
-        mixed_correction(xd, yd, zd, ri, r.v[0].x, oct, inv_mc0, mc, C);
-    }
+// ri by one FP64 Newton step.  b7 and tau: the partner's scaled FP64 octupole
+// without xzz and yzz, which its vanishing traces give.  Adds to the sums
+// W (s.u[0..5]) and the partner part of the correction (s.u[6..8]).
+__device__ __forceinline__ void mixed_correction(double x, double y, double z, float ri, double m0, const double* b7,
+    const double* tau, double* u) {
+    Radial g;
+    g.xx = x * x;
+    g.yy = y * y;
+    g.zz = z * z;
+    const double r2 = fmax(g.xx + g.yy + g.zz, 1.0e-20);
+    const double y0 = (double)ri;
+    radial_powers(y0 * fma(-(r2 * y0), y0, 3.0), g);
+    const Quadratic q = quadratic(x, y, z, g);
+    add_w(m0 * g.e3, g, q, u);
+    const double b[9] = {b7[0], b7[1], -(b7[0] + b7[1]), b7[2], b7[3], -(b7[2] + b7[3]), b7[4], b7[5], b7[6]};
+    add_correction(b, tau, x, y, z, q, g.e3, nullptr, u + 6);
 }
 
 // Mixed-precision partner record (192 bytes, 12 chunks of 16), written by the
 // staging kernel beside the FP64 record for mixed-precision plans: chunks 0-4
 // the factor-scaled multipole m0..m19 rounded to FP32, chunk 5 (Y0, Y1),
-// chunk 6 (Y2, m0), chunks 7-11 the factor-scaled octupole m10..m19 in FP64.
+// chunk 6 (Y2, m0), chunks 7-11 the FP64 octupole fields of the FP64 record
+// (xxx xyy xxy yyy xxz yyz xyz, trace 3).
 constexpr int kRecmY01 = 5;
 constexpr int kRecmY2M0 = 6;
 constexpr int kRecmOct = 7;
 
-// Mixed precision far pair from a mixed-precision record r (in LDS): no
-// conversion of the multipole, the separation formed in FP64 and rounded.
+// Mixed precision far pair from a mixed-precision record r (12 double2, in
+// LDS or registers): the separation is formed in FP64 and rounded to FP32 for
+// the derivative tensor and the 20-component contraction, which accumulate
+// into the FP32 partial sums Lf of the current image (at most 8 pairs, added
+// to the FP64 expansion by the caller).  The correction stays FP64, in u.
 template <bool RHO>
-__device__ __forceinline__ void m2l_far_m32(const double2* __restrict__ r, double X0, double X1, double X2,
-    double inv_mc0, const double* mc, float* Lf, double* C) {
+__device__ __forceinline__ void m2l_far_m32(const double2* __restrict__ r, double X0, double X1, double X2, float* Lf,
+    double* u) {
     const double2 y01 = r[kRecmY01], y2m = r[kRecmY2M0];
     const double xd = X0 - y01.x, yd = X1 - y01.y, zd = X2 - y2m.x;
     float m[20];
-    const float4* f4 = reinterpret_cast<const float4*>(r);
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
-        const float4 v = f4[i];
+        const float4 v = __builtin_bit_cast(float4, r[i]);
         m[4 * i] = v.x;
         m[4 * i + 1] = v.y;
         m[4 * i + 2] = v.z;
@@ -400,75 +595,15 @@ __device__ __forceinline__ void m2l_far_m32(const double2* __restrict__ r, doubl
     }
     const float ri = m2l_fp32_core<RHO>((float)xd, (float)yd, (float)zd, m, Lf);
     if constexpr (RHO) {
-        double oct[10];
+        double o[10];
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
             const double2 v = r[kRecmOct + k];
-            oct[2 * k] = v.x;
-            oct[2 * k + 1] = v.y;
+            o[2 * k] = v.x;
+            o[2 * k + 1] = v.y;
         }
-        mixed_correction(xd, yd, zd, ri, y2m.y, oct, inv_mc0, mc, C);
+        mixed_correction(xd, yd, zd, ri, y2m.y, o, o + 7, u);
     }
-}
-
-template <bool RHO>
-__device__ __forceinline__ void m2l_far(const double* __restrict__ p, double X0, double X1, double X2,
-    double inv_mc0, const double* mc, double* L, double* C) {
-    double m[20];
-    load_record20(p, m);
-    const double2 yv = reinterpret_cast<const double2*>(p)[10];
-    const double x = X0 - yv.x, y = X1 - yv.y, z = X2 - p[22];
-    DTensor t;
-    d_tensor(x, y, z, t);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) L[i] = fma(m[0], t.D[i], L[i]);
-    if constexpr (!RHO) dipole_rows(m, t.D, L);
-    contract_high<20>(m, t.D, L);
-    if constexpr (RHO) {
-        const double n0c = m[0] * inv_mc0;
-        double a[10];
-#pragma unroll
-        for (int k = 0; k < 10; ++k) a[k] = fma(-mc[k], n0c, m[10 + k]);
-        am_correction_t(t.d2, t.d3x00, t.d3x11, t.d3x22, t.d3x01, t.d3x02, t.d3x12, a, C);
-    }
-}
-
-// One near pair with a monopole-only partner of mass mn at Y.
-template <bool RHO>
-__device__ __forceinline__ void m2l_near(double mn, double Y0, double Y1, double Y2, double X0, double X1,
-    double X2, double inv_mc0, const double* mc, double* L, double* C) {
-    const double x = X0 - Y0, y = X1 - Y1, z = X2 - Y2;
-    DTensor t;
-    d_tensor(x, y, z, t);
-#pragma unroll
-    for (int i = 0; i < 20; ++i) L[i] = fma(mn, t.D[i], L[i]);
-    if constexpr (RHO) {
-        const double n0c = mn * inv_mc0;
-        double a[10];
-#pragma unroll
-        for (int k = 0; k < 10; ++k) a[k] = -(mc[k] * n0c);
-        am_correction_t(t.d2, t.d3x00, t.d3x11, t.d3x22, t.d3x01, t.d3x02, t.d3x12, a, C);
-    }
-}
-
-// One p2m pair: refined-neighbour multipole record r (held in registers)
-// onto a leaf cell at X.
-template <bool RHO>
-__device__ __forceinline__ void p2m_pair_rec(const Rec& r, double X0, double X1, double X2, double* L, double* C) {
-    double m[20];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) {
-        m[2 * i] = r.v[i].x;
-        m[2 * i + 1] = r.v[i].y;
-    }
-    const double x = X0 - r.v[10].x, y = X1 - r.v[10].y, z = X2 - r.v[11].x;
-    DTensor t;
-    d_tensor(x, y, z, t);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) L[i] = fma(m[0], t.D[i], L[i]);
-    if constexpr (!RHO) dipole_rows(m, t.D, L);
-    contract_high<4>(m, t.D, L);
-    if constexpr (RHO) am_correction_t(t.d2, t.d3x00, t.d3x11, t.d3x22, t.d3x01, t.d3x02, t.d3x12, m + 10, C);
 }
 
 // ---------------------------------------------------------------------------
@@ -486,6 +621,7 @@ struct StageArgs {
     const int32_t* list;    // slots to stage (null: all nslots)
     double dx;
     int32_t nslots;         // slots to stage (length of list when given)
+    int32_t rho;            // record form: RHO or DRHODT octupole fields
 };
 
 struct LevelArgs {
@@ -498,11 +634,13 @@ struct LevelArgs {
     const int2* items;      // (slot, flags)
     const Tables* tab;
     const uint64_t* mixbits;   // per coarse offset: byte k, bit j = far pair evaluated in FP32
-    // mixed-precision plans, lane mappings 3 and 7: the mixed-precision
-    // records, and per entry of the far schedule (Tables::sched) 1 where
-    // every far pair of the entry's offset is evaluated in FP32
+    // mixed-precision plans, lane mapping 7: the mixed-precision records, and
+    // the entries of the far schedule (Tables::sched) in the order they run,
+    // the first mix_n64 in FP64 and then those whose offset has every far pair
+    // evaluated in FP32
     const double* recm;
-    const uint8_t* mixoff;
+    const int32_t* mixorder;
+    int32_t mix_n64;
     const double* mon;      // [nslots][512] monopoles (p2p window of leaf targets)
     // leaf targets with refined neighbours: the p2m sums (L0..3, L_c, 0) of
     // each cell, [p2m item][512][8], written by p2m_kernel for leaf_kernel

@@ -61,16 +61,17 @@ __device__ __forceinline__ void store_stream(double2* p, double2 v) {
 
 // One block per 128 cells of a slot (two x-planes).  Those cells' records are
 // the 128 consecutive records of the block's coarse x-layer, so the block
-// loads the cells' M and centre-of-mass rows (contiguous) into LDS in 16-byte
-// pieces, then writes the 128 records as one contiguous range, consecutive
-// threads in consecutive 16-byte chunks.  Loads and stores are both
-// coalesced, where a lane per record spread every instruction over 64 rows.
+// loads the cells' M and centre-of-mass rows (contiguous) in 16-byte pieces
+// into LDS rows of 25 doubles (an odd stride: a wave that reads one column of
+// 64 rows hits every bank), two waves per 64 rows turn each row into its
+// record (one half the mass, dipole, quadrupole and centre, the other the
+// octupole), and the records leave as one contiguous range, consecutive
+// threads in consecutive 16-byte chunks.  Loads and stores are both coalesced,
+// where a lane per record spread every instruction over 64 rows.
+constexpr int kStageRow = 25;
+
 __global__ __launch_bounds__(256) void stage_records(StageArgs a) {
-    // leaf-cell centres are rounded operation by operation, as the reference does
-#pragma clang fp contract(off)
-    __shared__ double sM[128 * 20];
-    __shared__ double sC[128 * 3];
-    __shared__ double sm[128];
+    __shared__ double s_row[128 * kStageRow];
     const int si = blockIdx.x >> 2, q = blockIdx.x & 3;
     if (si >= a.nslots) return;                // uniform per block
     const int slot = a.list ? a.list[si] : si;
@@ -78,85 +79,146 @@ __global__ __launch_bounds__(256) void stage_records(StageArgs a) {
     const int c0 = q * 128;
     const int t = threadIdx.x;
     const size_t row0 = (size_t)slot * kCells + c0;
+    // cell c0 + t's row; thread t and t + 128 share cell t
+    const int cl = t & 127, octupole = t >> 7;   // octupole: uniform per wave
+    double* row = s_row + cl * kStageRow;
+    double v[12];                              // this half's record fields
+    float f32[10];                             // and its FP32 moments (mixed precision)
+#pragma unroll
+    for (int i = 0; i < 12; ++i) v[i] = 0.0;
     if (k == OCTOFMM_SLOT_NONLEAF) {
         const double2* srcM = reinterpret_cast<const double2*>(a.M + row0 * 20);
-        for (int i = t; i < 128 * 10; i += 256) reinterpret_cast<double2*>(sM)[i] = srcM[i];
+#pragma unroll
+        for (int r = 0; r < 5; ++r) {
+            const int i = t + 256 * r;
+            const double2 m = srcM[i];
+            double* d = s_row + (i / 10) * kStageRow + 2 * (i % 10);
+            d[0] = m.x;
+            d[1] = m.y;
+        }
         const double* srcC = a.com + row0 * 3;
-        for (int i = t; i < 128 * 3; i += 256) sC[i] = srcC[i];
-    } else if (k == OCTOFMM_SLOT_LEAF) {
-        if (t < 128) sm[t] = a.mon[row0 + t];
-    }
-    __syncthreads();
-    double2* dst = reinterpret_cast<double2*>(a.rec + row0 * kRecDoubles);
-    for (int ch = t; ch < 128 * 12; ch += 256) {
-        const int r = c0 + ch / 12, part = ch % 12;
-        // the cell of record r: coarse cell r >> 3 (x-major), child r & 7
-        const int co = r >> 3, ci = r & 7;
-        const int x = 2 * (co >> 4) + ((ci >> 2) & 1), y = 2 * ((co >> 2) & 3) + ((ci >> 1) & 1),
-                  z = 2 * (co & 3) + (ci & 1);
-        const int cl = x * 64 + y * 8 + z - c0;
-        double2 v = make_double2(0.0, 0.0);
-        if (k == OCTOFMM_SLOT_NONLEAF) {
-            if (part < 10) {
-                v.x = sM[cl * 20 + 2 * part] * record_scale(2 * part);
-                v.y = sM[cl * 20 + 2 * part + 1] * record_scale(2 * part + 1);
-            } else if (part == 10) {
-                v = make_double2(sC[cl * 3], sC[cl * 3 + 1]);
+        for (int i = t; i < 128 * 3; i += 256) s_row[(i / 3) * kStageRow + 20 + i % 3] = srcC[i];
+        __syncthreads();
+        if (!octupole) {
+            // fields 0..8 and the centre (v[9..11])
+            const double m4 = row[4], m7 = row[7], tr = (m4 + m7 + row[9]) * (1.0 / 3.0);
+            v[0] = row[0];
+#pragma unroll
+            for (int i = 1; i < 4; ++i) v[i] = 1.25 * row[i];
+            v[4] = (15.0 / 32.0) * (m4 - tr);
+            v[5] = (15.0 / 32.0) * row[5];
+            v[6] = (15.0 / 32.0) * row[6];
+            v[7] = (15.0 / 32.0) * (m7 - tr);
+            v[8] = (15.0 / 32.0) * row[8];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) v[9 + i] = row[20 + i];
+        } else {
+            // fields 9..20
+            double m[10];
+#pragma unroll
+            for (int i = 0; i < 10; ++i) m[i] = (5.0 / 64.0) * row[10 + i];
+            const double tx = m[0] + m[3] + m[5], ty = m[1] + m[6] + m[8], tz = m[2] + m[7] + m[9];
+            const double xxx = m[0] - 0.6 * tx, xyy = m[3] - 0.2 * tx, xzz = m[5] - 0.2 * tx;
+            const double xxy = m[1] - 0.2 * ty, yyy = m[6] - 0.6 * ty, yzz = m[8] - 0.2 * ty;
+            const double xxz = m[2] - 0.2 * tz, yyz = m[7] - 0.2 * tz, xyz = m[4];
+            if (a.rho) {
+                v[0] = xxx;
+                v[1] = xyy;
+                v[2] = xzz;
+                v[3] = xxy;
+                v[4] = yyy;
+                v[5] = yzz;
+                v[6] = xxz;
+                v[7] = yyz;
+                v[8] = xyz;
+                v[9] = 0.7 * tx;
+                v[10] = 0.7 * ty;
+                v[11] = 0.7 * tz;
             } else {
-                v = make_double2(sC[cl * 3 + 2], 0.0);
+                // coefficients of the cubic monomials
+                v[0] = 0.5 * xxx;
+                v[1] = 1.5 * xyy;
+                v[2] = 1.5 * xxy;
+                v[3] = 0.5 * yyy;
+                v[4] = 1.5 * xxz;
+                v[5] = 1.5 * yyz;
+                v[6] = xxz + yyz;
+                v[7] = 3.0 * xyz;
             }
-        } else if (k == OCTOFMM_SLOT_LEAF) {
-            const double m = sm[cl];
-            // geometric centre in the target's frame (multipole_interaction_interface.hpp:216-235)
+        }
+        if (a.recm) {
+#pragma unroll
+            for (int i = 0; i < 10; ++i)
+                f32[i] = (float)(row[10 * octupole + i] * (octupole ? record_scale(10 + i) : record_scale(i)));
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 10; ++i) f32[i] = 0.0f;
+        if (k == OCTOFMM_SLOT_LEAF && !octupole) {
+            // a monopole at the geometric cell centre in the target's frame
+            // (multipole_interaction_interface.hpp:216-235), rounded operation
+            // by operation as the reference does
+#pragma clang fp contract(off)
+            const int cell = c0 + cl;
             const int* fo = a.foff + 3 * slot;
             const double* fb = a.fxbase + 3 * slot;
-            if (part == 0) {
-                v.x = m;
-            } else if (part == 10) {
-                v.x = (double)(x + fo[0]) * a.dx + fb[0] - kInx * a.dx;
-                v.y = (double)(y + fo[1]) * a.dx + fb[1] - kInx * a.dx;
-            } else if (part == 11) {
-                v.x = (double)(z + fo[2]) * a.dx + fb[2] - kInx * a.dx;
-                v.y = m;
-            }
+            v[0] = a.mon[row0 + cl];
+            f32[0] = (float)v[0];
+            v[9] = (double)((cell >> 6) + fo[0]) * a.dx + fb[0] - kInx * a.dx;
+            v[10] = (double)(((cell >> 3) & 7) + fo[1]) * a.dx + fb[1] - kInx * a.dx;
+            v[11] = (double)((cell & 7) + fo[2]) * a.dx + fb[2] - kInx * a.dx;
         }
-        store_stream(dst + ch, v);
-        if (a.recm) {
-            // the mixed-precision record of the same cell: m0..m19 rounded to
-            // FP32 (4 per chunk), (Y0, Y1), (Y2, m0), the octupole in FP64
-            double2 w = make_double2(0.0, 0.0);
-            if (k == OCTOFMM_SLOT_NONLEAF) {
-                if (part < 5) {
-                    float4 f;
-                    f.x = (float)(sM[cl * 20 + 4 * part] * record_scale(4 * part));
-                    f.y = (float)(sM[cl * 20 + 4 * part + 1] * record_scale(4 * part + 1));
-                    f.z = (float)(sM[cl * 20 + 4 * part + 2] * record_scale(4 * part + 2));
-                    f.w = (float)(sM[cl * 20 + 4 * part + 3] * record_scale(4 * part + 3));
-                    w = __builtin_bit_cast(double2, f);
-                } else if (part == kRecmY01) {
-                    w = make_double2(sC[cl * 3], sC[cl * 3 + 1]);
-                } else if (part == kRecmY2M0) {
-                    w = make_double2(sC[cl * 3 + 2], sM[cl * 20]);
-                } else {
-                    const int c = 10 + 2 * (part - kRecmOct);
-                    w = make_double2(sM[cl * 20 + c] * record_scale(c), sM[cl * 20 + c + 1] * record_scale(c + 1));
-                }
-            } else if (k == OCTOFMM_SLOT_LEAF) {
-                const double m = sm[cl];
-                const int* fo = a.foff + 3 * slot;
-                const double* fb = a.fxbase + 3 * slot;
-                if (part == 0) {
-                    w = __builtin_bit_cast(double2, make_float4((float)m, 0.0f, 0.0f, 0.0f));
-                } else if (part == kRecmY01) {
-                    w.x = (double)(x + fo[0]) * a.dx + fb[0] - kInx * a.dx;
-                    w.y = (double)(y + fo[1]) * a.dx + fb[1] - kInx * a.dx;
-                } else if (part == kRecmY2M0) {
-                    w.x = (double)(z + fo[2]) * a.dx + fb[2] - kInx * a.dx;
-                    w.y = m;
-                }
-            }
-            store_stream(reinterpret_cast<double2*>(a.recm + row0 * kRecDoubles) + ch, w);
+    }
+    // the row of the block's r-th record: coarse cell r >> 3 of the layer,
+    // child r & 7
+    auto out = [&](double* rec) {
+        double2* dst = reinterpret_cast<double2*>(rec + row0 * kRecDoubles);
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            const int ch = t + 256 * i;
+            const int r = ch / 12, part = ch % 12;
+            const int co = r >> 3, ci = r & 7;
+            const int x = (ci >> 2) & 1, y = 2 * (co >> 2) + ((ci >> 1) & 1), z = 2 * (co & 3) + (ci & 1);
+            const double* src = s_row + (x * 64 + y * 8 + z) * kStageRow + 2 * part;
+            store_stream(dst + ch, make_double2(src[0], src[1]));
         }
+    };
+    __syncthreads();   // every row read before its record overwrites it
+    if (!octupole) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) row[i] = v[i];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) row[kRecY + i] = v[9 + i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 12; ++i) row[9 + i] = v[i];
+    }
+    __syncthreads();
+    out(a.rec);
+    if (a.recm) {   // uniform: the mixed-precision records of the same cells
+        __syncthreads();
+        double* d = row + 5 * octupole;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) d[i] = __builtin_bit_cast(double, make_float2(f32[2 * i], f32[2 * i + 1]));
+        if (!octupole) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) row[2 * kRecmY01 + i] = v[9 + i];
+            row[2 * kRecmY2M0 + 1] = v[0];
+        } else {
+            double* o = row + 2 * kRecmOct;
+            o[0] = v[0];
+            o[1] = v[1];
+            o[2] = v[3];
+            o[3] = v[4];
+            o[4] = v[6];
+            o[5] = v[7];
+            o[6] = v[8];
+            o[7] = v[9];
+            o[8] = v[10];
+            o[9] = v[11];
+        }
+        __syncthreads();
+        out(a.recm);
     }
 }
 
@@ -352,96 +414,132 @@ __device__ __forceinline__ void leaf_rows_coalesced(const LevelArgs& a, int slot
     store_stream(gg + 512 + t, bg[512 + t + ((512 + t) >> 5)]);
 }
 
+// Mixed-precision kernels: the expansion of a target's FP64 pairs, once they
+// are all in s, and after the FP32 ones the correction, whose sums go on.
+template <bool RHO>
+__device__ __forceinline__ void finish_fp64_part(const Acc<RHO>& s, double* L) {
+    double f[kFolded], C[3];
+    acc_fold_expansion<RHO>(s, f);
+    f[18] = f[19] = f[20] = 0.0;
+    acc_finish<RHO>(f, L, C);
+}
+
+template <bool RHO>
+__device__ __forceinline__ void finish_correction(const Acc<RHO>& s, const double* __restrict__ trec, double* C) {
+    if constexpr (RHO) {
+        double c[3] = {s.u[6], s.u[7], s.u[8]};
+        fold_w(trec, 1.0 / trec[0], s.u, c);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) C[d] = kCorrectionScale * c[d];
+    } else {
+        C[0] = C[1] = C[2] = 0.0;
+    }
+}
+
+// Near pairs of a target cell over the coarse offsets di = first, first + step,
+// ...: partners in leaf slots, which carry only their monopole.
+template <bool RHO>
+__device__ __forceinline__ void near_pairs(const LevelArgs& a, const LaneGeom& g, const int* s_nbr, const int* s_kind,
+    int first, int step, double X0, double X1, double X2, Acc<RHO>& s) {
+    const Tables* __restrict__ tab = a.tab;
+    for (int di = first; di < tab->ndelta; di += step) {
+        const int ax = tab->delta[di][0], ay = tab->delta[di][1], az = tab->delta[di][2];
+        unsigned nb = (unsigned)(tab->nearbits[di] >> (8 * g.k)) & 0xffu;
+        int ns, raw;
+        const int cb = partner_base(g, ax, ay, az, s_nbr, ns, raw);
+        if (ns < 0 || s_kind[raw] != OCTOFMM_SLOT_LEAF) nb = 0;
+        const double* pb = a.rec + ((size_t)(ns < 0 ? 0 : ns) * kCells + cb) * kRecDoubles;
+#pragma unroll 1
+        for (int j = 0; j < 8; ++j) {
+            if (nb & (1u << j)) {
+                const double* p = pb + j * kRecDoubles;
+                m2l_near<RHO>(p[0], p[kRecY], p[kRecY + 1], p[kRecY + 2], X0, X1, X2, s);
+            }
+        }
+    }
+}
+
+// Mapping 0.  MIXED: the FP64 pairs of every offset come first, then the FP32
+// ones (a.mixbits), so that the FP64 sums are done before the FP32 expansion
+// takes their registers.
 template <bool RHO, bool MIXED>
 __device__ void m2l_item(const LevelArgs& a, int slot, int flags, const int* s_nbr, const int* s_kind, int w) {
     const LaneGeom g = lane_geom(w);
     const Tables* __restrict__ tab = a.tab;
     const double* trec = a.rec + ((size_t)slot * kCells + g.rec) * kRecDoubles;
     const double X0 = trec[kRecY], X1 = trec[kRecY + 1], X2 = trec[kRecY + 2];
-    const double inv_mc0 = RHO ? 1.0 / trec[0] : 0.0;
-    double mc[10];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) mc[i] = RHO ? trec[10 + i] : 0.0;
-    double L[20], C[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int i = 0; i < 20; ++i) L[i] = 0.0;
-
+    Acc<RHO> s;
+    acc_clear(s);
     const int nd = tab->ndelta;
     // far pass, software-pipelined: the record of the next pair is loaded
     // (by every lane, from a valid address) while the current one is computed
-    auto far_base = [&](int di, unsigned& fb) -> const double* {
+    auto far_base = [&](int di, const double* rec, unsigned& fb) -> const double* {
         const int ax = tab->delta[di][0], ay = tab->delta[di][1], az = tab->delta[di][2];
         fb = (unsigned)(tab->farbits[di] >> (8 * g.k)) & 0xffu;
         int ns, raw;
         const int cb = partner_base(g, ax, ay, az, s_nbr, ns, raw);
         if (ns < 0) fb = 0;
-        return a.rec + ((size_t)(ns < 0 ? 0 : ns) * kCells + cb) * kRecDoubles;
+        return rec + ((size_t)(ns < 0 ? 0 : ns) * kCells + cb) * kRecDoubles;
     };
-    unsigned fb;
-    const double* pb = far_base(0, fb);
-    Rec nxt;
-    if constexpr (!MIXED) load_rec(pb, nxt);
-    float Lf[20];
-    if constexpr (MIXED) {
+    if constexpr (!MIXED) {
+        unsigned fb;
+        const double* pb = far_base(0, a.rec, fb);
+        Rec nxt;
+        load_rec(pb, nxt);
+        for (int di = 0; di < nd; ++di) {
+            unsigned fbn = 0;
+            const double* pbn = pb;
 #pragma unroll
-        for (int i = 0; i < 20; ++i) Lf[i] = 0.0f;
-    }
-    for (int di = 0; di < nd; ++di) {
-        unsigned fbn = 0;
-        const double* pbn = pb;
-        const unsigned mb = MIXED ? (unsigned)(a.mixbits[di] >> (8 * g.k)) & 0xffu : 0u;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            // FP64: the next record is prefetched while this pair computes;
-            // MIXED keeps a single record live (its FP32 partial sums need
-            // the registers)
-            Rec cur;
-            if constexpr (MIXED) {
-                load_rec(pb + j * kRecDoubles, cur);
-                if (j == 7 && di + 1 < nd) pbn = far_base(di + 1, fbn);
-            } else {
-                cur = nxt;
+            for (int j = 0; j < 8; ++j) {
+                const Rec cur = nxt;
                 if (j < 7) {
                     load_rec(pb + (j + 1) * kRecDoubles, nxt);
                 } else if (di + 1 < nd) {
-                    pbn = far_base(di + 1, fbn);
+                    pbn = far_base(di + 1, a.rec, fbn);
                     load_rec(pbn, nxt);
                 }
+                if (fb & (1u << j)) m2l_far_rec<RHO>(cur, X0, X1, X2, s);
             }
-            if (fb & (1u << j)) {
-                if (MIXED && (mb & (1u << j)))
-                    m2l_far_mixed<RHO>(cur, X0, X1, X2, inv_mc0, mc, Lf, C);
-                else
-                    m2l_far_rec<RHO>(cur, X0, X1, X2, inv_mc0, mc, L, C);
-            }
+            pb = pbn;
+            fb = fbn;
         }
-        if constexpr (MIXED) {
-            // the coarse offset's FP32 partial sums join the FP64 expansion
-#pragma unroll
-            for (int i = 0; i < 20; ++i) {
-                L[i] += (double)Lf[i];
-                Lf[i] = 0.0f;
-            }
-        }
-        pb = pbn;
-        fb = fbn;
-    }
-    if (flags & kItemNear) {
+    } else {
         for (int di = 0; di < nd; ++di) {
-            const int ax = tab->delta[di][0], ay = tab->delta[di][1], az = tab->delta[di][2];
-            unsigned nb = (unsigned)(tab->nearbits[di] >> (8 * g.k)) & 0xffu;
-            int ns, raw;
-            const int cb = partner_base(g, ax, ay, az, s_nbr, ns, raw);
-            if (ns < 0 || s_kind[raw] != OCTOFMM_SLOT_LEAF) nb = 0;
-            const double* pb = a.rec + ((size_t)(ns < 0 ? 0 : ns) * kCells + cb) * kRecDoubles;
+            unsigned fb;
+            const double* pb = far_base(di, a.rec, fb);
+            fb &= ~((unsigned)(a.mixbits[di] >> (8 * g.k)));
+#pragma unroll 1
+            for (int j = 0; j < 8; ++j)
+                if (fb & (1u << j)) m2l_far<RHO>(pb + j * kRecDoubles, X0, X1, X2, s);
+        }
+    }
+    if (flags & kItemNear) near_pairs<RHO>(a, g, s_nbr, s_kind, 0, 1, X0, X1, X2, s);
+    double f[kFolded], L[20], C[3];
+    if constexpr (!MIXED) {
+        acc_fold<RHO>(s, trec, f);
+        acc_finish<RHO>(f, L, C);
+    } else {
+        finish_fp64_part<RHO>(s, L);
+        for (int di = 0; di < nd; ++di) {
+            unsigned fb;
+            const double* pb = far_base(di, a.recm, fb);
+            fb &= (unsigned)(a.mixbits[di] >> (8 * g.k));
+            float Lf[20];
+#pragma unroll
+            for (int i = 0; i < 20; ++i) Lf[i] = 0.0f;
 #pragma unroll 1
             for (int j = 0; j < 8; ++j) {
-                if (nb & (1u << j)) {
-                    const double* p = pb + j * kRecDoubles;
-                    m2l_near<RHO>(p[kRecMon], p[kRecY], p[kRecY + 1], p[kRecY + 2], X0, X1, X2, inv_mc0, mc, L, C);
+                if (fb & (1u << j)) {
+                    Rec cur;
+                    load_rec(pb + j * kRecDoubles, cur);
+                    m2l_far_m32<RHO>(cur.v, X0, X1, X2, Lf, s.u);
                 }
             }
+            // the coarse offset's FP32 partial sums join the FP64 expansion
+#pragma unroll
+            for (int i = 0; i < 20; ++i) L[i] += (double)Lf[i];
         }
+        finish_correction<RHO>(s, trec, C);
     }
     finish_cell<RHO>(a, slot, g.cell, L, 20, C, true, false);
 }
@@ -460,13 +558,8 @@ __device__ void m2l_item_split(const LevelArgs& a, int slot, int flags, const in
     const Tables* __restrict__ tab = a.tab;
     const double* trec = a.rec + ((size_t)slot * kCells + g.rec) * kRecDoubles;
     const double X0 = trec[kRecY], X1 = trec[kRecY + 1], X2 = trec[kRecY + 2];
-    const double inv_mc0 = RHO ? 1.0 / trec[0] : 0.0;
-    double mc[10];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) mc[i] = RHO ? trec[10 + i] : 0.0;
-    double L[20], C[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int i = 0; i < 20; ++i) L[i] = 0.0;
+    Acc<RHO> s;
+    acc_clear(s);
     const int nd = tab->ndelta;
     for (int di = sl; di < nd; di += SPLIT) {
         const int ax = tab->delta[di][0], ay = tab->delta[di][1], az = tab->delta[di][2];
@@ -481,38 +574,26 @@ __device__ void m2l_item_split(const LevelArgs& a, int slot, int flags, const in
         for (int j = 0; j < 8; ++j) {
             const Rec cur = nxt;
             if (j < 7) load_rec(pb + (j + 1) * kRecDoubles, nxt);
-            if (fb & (1u << j)) m2l_far_rec<RHO>(cur, X0, X1, X2, inv_mc0, mc, L, C);
-        }
-        if (flags & kItemNear) {
-            unsigned nb = (unsigned)(tab->nearbits[di] >> (8 * g.k)) & 0xffu;
-            if (ns < 0 || s_kind[raw] != OCTOFMM_SLOT_LEAF) nb = 0;
-#pragma unroll 1
-            for (int j = 0; j < 8; ++j) {
-                if (nb & (1u << j)) {
-                    const double* p = pb + j * kRecDoubles;
-                    m2l_near<RHO>(p[kRecMon], p[kRecY], p[kRecY + 1], p[kRecY + 2], X0, X1, X2, inv_mc0, mc, L, C);
-                }
-            }
+            if (fb & (1u << j)) m2l_far_rec<RHO>(cur, X0, X1, X2, s);
         }
     }
+    if (flags & kItemNear) near_pairs<RHO>(a, g, s_nbr, s_kind, sl, SPLIT, X0, X1, X2, s);
+    double f[kFolded];
+    acc_fold<RHO>(s, trec, f);
     if (sl > 0) {
-        double* o = s_part + ((size_t)(sl - 1) * 64 + lane) * 23;
+        double* o = s_part + ((size_t)(sl - 1) * 64 + lane) * kFolded;
 #pragma unroll
-        for (int i = 0; i < 20; ++i) o[i] = L[i];
-        o[20] = C[0];
-        o[21] = C[1];
-        o[22] = C[2];
+        for (int i = 0; i < kFolded; ++i) o[i] = f[i];
     }
     __syncthreads();
     if (sl == 0) {
         for (int q = 0; q < SPLIT - 1; ++q) {
-            const double* o = s_part + ((size_t)q * 64 + lane) * 23;
+            const double* o = s_part + ((size_t)q * 64 + lane) * kFolded;
 #pragma unroll
-            for (int i = 0; i < 20; ++i) L[i] += o[i];
-            C[0] += o[20];
-            C[1] += o[21];
-            C[2] += o[22];
+            for (int i = 0; i < kFolded; ++i) f[i] += o[i];
         }
+        double L[20], C[3];
+        acc_finish<RHO>(f, L, C);
         finish_cell<RHO>(a, slot, g.cell, L, 20, C, true, false);
     }
 }
@@ -522,7 +603,7 @@ template <bool RHO, int SPLIT>
 __global__ __launch_bounds__(64 * SPLIT) void level_kernel_split(LevelArgs a) {
     __shared__ int s_nbr[27];
     __shared__ int s_kind[27];
-    __shared__ double s_part[(SPLIT - 1) * 64 * 23];
+    __shared__ double s_part[(SPLIT - 1) * 64 * kFolded];
     const int v = xcd_item(blockIdx.x, gridDim.x);
     const int item = v >> 3, w = v & 7;
     const int2 it = a.items[a.item0 + item];
@@ -594,7 +675,7 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T* as_const(c
 // run.
 //
 // MIXED (mixed-precision plans): a far offset all of whose far pairs are
-// evaluated in FP32 (a.mixoff) stages the mixed-precision records instead and
+// evaluated in FP32 (a.mixorder) stages the mixed-precision records instead and
 // runs m2l_far_m32 on them, with the offset's FP32 partial sums added to the
 // FP64 expansion after its 8 children; the other far offsets run in FP64.
 // The precision is uniform over the wave for each offset, so no lane waits
@@ -616,14 +697,8 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
     const int wu = __builtin_amdgcn_readfirstlane(w);
     const double* trec = a.rec + ((size_t)slot * kCells + lane_geom(wu).rec) * kRecDoubles;
     const double X0 = trec[kRecY], X1 = trec[kRecY + 1], X2 = trec[kRecY + 2];
-    const double inv_mc0 = RHO ? 1.0 / trec[0] : 0.0;
-    double mc[10];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) mc[i] = RHO ? trec[10 + i] : 0.0;
-    double L[20], C[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int i = 0; i < 20; ++i) L[i] = 0.0;
-    const int nd = tab->ndelta;
+    Acc<RHO> s;
+    acc_clear(s);
     const int bx = ((wu >> 2) & 1) * 2, by = ((wu >> 1) & 1) * 2, bz = (wu & 1) * 2;
     const auto* nbr_row = as_const(a.nbr + (size_t)__builtin_amdgcn_readfirstlane(slot) * 27);
     // record index (slot * 512 + first child) of the partner coarse cell of
@@ -639,6 +714,17 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
         if (ns < 0) empty |= 1u << gi;
         return (unsigned)(ns < 0 ? 0 : ns) * (unsigned)kCells + (unsigned)cb;
     };
+    // only the offsets with a far pair are staged (delta 0 is all near / self),
+    // in the order of the far schedule
+    const int nfd = tab->nsched;
+    const int q0 = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(sl);
+    // The wave's entries are those at positions q0, q0 + SPLIT, ... of the
+    // schedule; a mixed-precision plan orders it (a.mixorder) with its n64 FP64
+    // entries first, so that the FP64 sums are done before the FP32 expansion
+    // takes their registers.
+    const int n64 = MIXED ? a.mix_n64 : nfd;
+    const auto* mixorder = as_const(a.mixorder);
+    auto entry = [&](int i) -> int { return MIXED ? mixorder[i] : i; };
     // Group c (8 records = 96 chunks) is loaded by one full instruction
     // (chunks 0..63) and one on the lower 32 lanes (chunks 64..95): both are a
     // uniform base plus the lane's 16-byte offset, and the LDS destination is
@@ -647,12 +733,12 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
     // neighbour-slot loads in flight together (one wait, taken while the
     // current image is still arriving, instead of one wait per group).
     unsigned nrec[8];
-    const double* src_next = a.rec;   // the records the entry bases() last formed is staged from
+    int f32_next = 0;           // nonzero: that entry is staged from the mixed-precision records
     unsigned empty_next = 0;    // groups of that entry whose partner (a) slot is empty
     unsigned emptyb_next = 0;   // the same for offset b of a split entry (formed by issue())
     int entry_next = 0;         // the schedule entry bases() last formed
-    auto bases = [&](int q, const double* src) {
-        const int e = tab->sched[q];
+    auto bases = [&](int i) {
+        const int e = tab->sched[entry(i)];
         const int di = e & 0xff;
         const int ax = tab->delta[di][0], ay = tab->delta[di][1], az = tab->delta[di][2];
         unsigned empty = 0;
@@ -661,7 +747,7 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
         form_sgprs(nrec);
         empty_next = empty;
         entry_next = e;
-        src_next = src;
+        f32_next = i >= n64;
     };
     // The full-wave loads of all groups come first and the half-wave loads
     // follow in one branch of their own: with a full and a half load of one
@@ -684,7 +770,7 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
         asm volatile("" : "+s"(st));
         const int lo = lane();
         if (kind == 0) {
-            const char* rb = reinterpret_cast<const char*>(src_next);
+            const char* rb = reinterpret_cast<const char*>(MIXED && f32_next != 0 ? a.recm : a.rec);
             const unsigned loff = (unsigned)lo * 16u;
 #pragma unroll
             for (int gi = 0; gi < 8; ++gi)
@@ -727,108 +813,99 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
             }
         }
     };
-    // only the offsets with a far pair are staged (delta 0 is all near / self),
-    // in the order of the far schedule
-    const int nfd = tab->nsched;
-    const int q0 = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(sl);
-    const auto* mixoff = as_const(a.mixoff);
-    // the records entry q is staged from
-    auto source = [&](int q) -> const double* { return (MIXED && mixoff[q]) ? a.recm : a.rec; };
-    if (q0 < nfd) {
-        bases(q0, source(q0));
-        issue();
-    }
+    if (flags & kItemNear) near_pairs<RHO>(a, lane_geom(wu), s_nbr, s_kind, q0, SPLIT, X0, X1, X2, s);
     // the lane's group of 8 records in the image
     const double2* group = stage + (lane() >> 3) * kDirGroup;
-    for (int q = q0; q < nfd; q += SPLIT) {
+    // One image: image(lanes of step j, records) between the arrival of
+    // position i's records and the refill with those of position i + SPLIT.
+    auto walk = [&](int i, auto&& image) {
         // the lanes that read record j of the image: those of the classes in
         // byte j of the entry's step masks, unless their group's partner slot
         // is empty; kind 2 classes on the far side of the axis read records
         // 4..7 as their records 0..3.  The masks are formed in scalar
         // registers, one 64-bit lane mask per step (lane = group * 8 + class).
+        const int q = entry(i);
         const uint64_t ra = tab->sched_rowa[q], rb = tab->sched_rowb[q];
         // (emptyb_next is formed between the branches of issue(), after which
         // the compiler no longer knows it to be uniform)
         const uint64_t ea = spread_groups(empty_next);
         const uint64_t eb = spread_groups(__builtin_amdgcn_readfirstlane(emptyb_next));
-        auto step_mask = [&](int j) -> uint64_t { return step_lanes(ra, rb, ea, eb, j); };
         const double2* recs =
             __builtin_amdgcn_inverse_ballot_w64(repeat_bytes(tab->sched_half[q] & 0xffu)) ? group + 48 : group;
-        const bool f32 = MIXED && mixoff[q];   // uniform
-        if (q + SPLIT < nfd) bases(q + SPLIT, source(q + SPLIT));
+        if (i + SPLIT < nfd) bases(i + SPLIT);
         __builtin_amdgcn_s_waitcnt(0x3F70);   // vmcnt(0): this wave's image is in LDS
         __builtin_amdgcn_wave_barrier();
-        if (MIXED && f32) {
-            float Lf[20];
-#pragma unroll
-            for (int i = 0; i < 20; ++i) Lf[i] = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (__builtin_amdgcn_inverse_ballot_w64(step_mask(j)))
-                    m2l_far_m32<RHO>(recs + j * 12, X0, X1, X2, inv_mc0, mc, Lf, C);
-            // the offset's FP32 partial sums join the FP64 expansion
-#pragma unroll
-            for (int i = 0; i < 20; ++i) L[i] += (double)Lf[i];
-        } else {
+        image([&](int j) -> uint64_t { return step_lanes(ra, rb, ea, eb, j); }, recs);
+        lds_wave_sync();   // every read of the image done before it is refilled
+        if (i + SPLIT < nfd) issue();
+    };
+    int i = q0;
+    if (i < nfd) {
+        bases(i);
+        issue();
+    }
+    for (; i < n64; i += SPLIT)
+        walk(i, [&](auto&& step_mask, const double2* recs) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 if (__builtin_amdgcn_inverse_ballot_w64(step_mask(j))) {
                     Rec cur;
 #pragma unroll
-                    for (int i = 0; i < 12; ++i) cur.v[i] = recs[j * 12 + i];
-                    m2l_far_rec<RHO>(cur, X0, X1, X2, inv_mc0, mc, L, C);
+                    for (int c = 0; c < 12; ++c) cur.v[c] = recs[j * 12 + c];
+                    m2l_far_rec<RHO>(cur, X0, X1, X2, s);
                 }
             }
+        });
+    constexpr int kParts = MIXED ? 23 : kFolded;   // partial sums the waves hand over
+    double f[kParts];
+    if constexpr (!MIXED) {
+        acc_fold<RHO>(s, trec, f);
+    } else {
+        finish_fp64_part<RHO>(s, f);
+        for (; i < nfd; i += SPLIT)
+            walk(i, [&](auto&& step_mask, const double2* recs) {
+                float Lf[20];
+#pragma unroll
+                for (int c = 0; c < 20; ++c) Lf[c] = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (__builtin_amdgcn_inverse_ballot_w64(step_mask(j)))
+                        m2l_far_m32<RHO>(recs + j * 12, X0, X1, X2, Lf, s.u);
+                // the offset's FP32 partial sums join the FP64 expansion
+#pragma unroll
+                for (int c = 0; c < 20; ++c) f[c] += (double)Lf[c];
+            });
+        finish_correction<RHO>(s, trec, f + 20);
+    }
+    if constexpr (SPLIT > 1) {
+        // no refill is in flight and every read of the image is done, so the
+        // image can hold this wave's 64 x kParts partial sums (at most 11.5 KiB)
+        double* part = reinterpret_cast<double*>(stage) + (threadIdx.x & 63) * kParts;
+        if (q0 != 0) {
+#pragma unroll
+            for (int i = 0; i < kParts; ++i) part[i] = f[i];
         }
-        lds_wave_sync();   // every read of the image done before it is refilled
-        if (q + SPLIT < nfd) issue();
+        __syncthreads();
+        if (q0 != 0) return;
+        for (int o = 1; o < SPLIT; ++o) {
+            const double* po = reinterpret_cast<const double*>(s_stage + o * kDirWave) + (threadIdx.x & 63) * kParts;
+#pragma unroll
+            for (int i = 0; i < kParts; ++i) f[i] += po[i];
+        }
     }
     // The lane's geometry again, from an opaque copy of the thread index: the
     // far loop needs none of it, and formed here it is not held in registers
     // across that loop (where the RHO kernels run at the register limit).
     int t2;
     asm volatile("v_mov_b32 %0, %1" : "=v"(t2) : "v"((int)threadIdx.x));
-    const LaneGeom g = lane_geom(wu, t2);
-    if (flags & kItemNear) {
-        for (int di = q0; di < nd; di += SPLIT) {
-            const int ax = tab->delta[di][0], ay = tab->delta[di][1], az = tab->delta[di][2];
-            unsigned nb = (unsigned)(tab->nearbits[di] >> (8 * g.k)) & 0xffu;
-            int ns, raw;
-            const int cb = partner_base(g, ax, ay, az, s_nbr, ns, raw);
-            if (ns < 0 || s_kind[raw] != OCTOFMM_SLOT_LEAF) nb = 0;
-            const double* pb2 = a.rec + ((size_t)(ns < 0 ? 0 : ns) * kCells + cb) * kRecDoubles;
-#pragma unroll 1
-            for (int j = 0; j < 8; ++j) {
-                if (nb & (1u << j)) {
-                    const double* p = pb2 + j * kRecDoubles;
-                    m2l_near<RHO>(p[kRecMon], p[kRecY], p[kRecY + 1], p[kRecY + 2], X0, X1, X2, inv_mc0, mc, L, C);
-                }
-            }
-        }
+    const int cell = lane_geom(wu, t2).cell;
+    if constexpr (!MIXED) {
+        double L[20], C[3];
+        acc_finish<RHO>(f, L, C);
+        finish_cell<RHO>(a, slot, cell, L, 20, C, true, false);
+    } else {
+        finish_cell<RHO>(a, slot, cell, f, 20, f + 20, true, false);
     }
-    if constexpr (SPLIT > 1) {
-        // no refill is in flight and every read of the image is done, so the
-        // image can hold this wave's 64 x 23 partial sums (11.5 KiB)
-        double* part = reinterpret_cast<double*>(stage) + (threadIdx.x & 63) * 23;
-        if (q0 != 0) {
-#pragma unroll
-            for (int i = 0; i < 20; ++i) part[i] = L[i];
-            part[20] = C[0];
-            part[21] = C[1];
-            part[22] = C[2];
-        }
-        __syncthreads();
-        if (q0 != 0) return;
-        for (int o = 1; o < SPLIT; ++o) {
-            const double* po = reinterpret_cast<const double*>(s_stage + o * kDirWave) + (threadIdx.x & 63) * 23;
-#pragma unroll
-            for (int i = 0; i < 20; ++i) L[i] += po[i];
-            C[0] += po[20];
-            C[1] += po[21];
-            C[2] += po[22];
-        }
-    }
-    finish_cell<RHO>(a, slot, g.cell, L, 20, C, true, false);
 }
 
 // Leaf targets (monopole kernels): one 512-lane workgroup per leaf sub-grid.
@@ -996,7 +1073,8 @@ __device__ void p2m_item(const LevelArgs& a, int slot, int ordinal, int w, const
     const LaneGeom g = lane_geom(wu);
     const double* xc = a.com + ((size_t)slot * kCells + g.cell) * 3;
     const double X0 = xc[0], X1 = xc[1], X2 = xc[2];
-    double L[4] = {0.0, 0.0, 0.0, 0.0}, C[3] = {0.0, 0.0, 0.0};
+    Acc<RHO> s;
+    acc_clear(s);
     const int bx = ((wu >> 2) & 1) * 2, by = ((wu >> 1) & 1) * 2, bz = (wu & 1) * 2;
     // partner coarse cell of group gi at offset (ax, ay, az): its records, and
     // bit gi of `absent` where it is not in a refined neighbour slot
@@ -1056,13 +1134,15 @@ __device__ void p2m_item(const LevelArgs& a, int slot, int ordinal, int w, const
                 Rec cur;
 #pragma unroll
                 for (int i = 0; i < 12; ++i) cur.v[i] = group[j * 12 + i];
-                p2m_pair_rec<RHO>(cur, X0, X1, X2, L, C);
+                p2m_pair_rec<RHO>(cur, X0, X1, X2, s);
             }
         }
         lds_wave_sync();   // every read of the image done before it is refilled
         if (q + SPLIT < nlive) issue();
     }
     // waves 1..SPLIT-1 hand their sums to wave 0 through their own images
+    double L[4], C[3];
+    p2m_finish<RHO>(s, L, C);
     double* part = reinterpret_cast<double*>(stage) + l * 7;
     if (q0 != 0) {
 #pragma unroll
@@ -1335,21 +1415,19 @@ __global__ __launch_bounds__(512) void root_kernel(RootArgs a) {
     const int tx = t >> 6, ty = (t >> 3) & 7, tz = t & 7;
     const double* trec = a.rec + (size_t)record_of_cell(tx, ty, tz) * kRecDoubles;
     const double X0 = trec[kRecY], X1 = trec[kRecY + 1], X2 = trec[kRecY + 2];
-    const double inv_mc0 = RHO ? 1.0 / trec[0] : 0.0;
-    double mc[10];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) mc[i] = RHO ? trec[10 + i] : 0.0;
-    double L[20], C[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int i = 0; i < 20; ++i) L[i] = 0.0;
+    Acc<RHO> s;
+    acc_clear(s);
     const int p0 = blockIdx.x * a.per_chunk;
     for (int p = p0; p < p0 + a.per_chunk; ++p) {
         const int px = p >> 6, py = (p >> 3) & 7, pz = p & 7;
         const int dx = px - tx, dy = py - ty, dz = pz - tz;
         const bool inbox = dx >= -5 && dx <= 5 && dy >= -5 && dy <= 5 && dz >= -5 && dz <= 5;
         if (inbox && a.tab->root_excluded[(dx + 5) * 121 + (dy + 5) * 11 + (dz + 5)]) continue;
-        m2l_far<RHO>(a.rec + (size_t)record_of_cell(px, py, pz) * kRecDoubles, X0, X1, X2, inv_mc0, mc, L, C);
+        m2l_far<RHO>(a.rec + (size_t)record_of_cell(px, py, pz) * kRecDoubles, X0, X1, X2, s);
     }
+    double f[kFolded], L[20], C[3];
+    acc_fold<RHO>(s, trec, f);
+    acc_finish<RHO>(f, L, C);
     double* o = a.partial + ((size_t)blockIdx.x * kCells + t) * kRecDoubles;
 #pragma unroll
     for (int i = 0; i < 20; ++i) o[i] = L[i];
@@ -1763,9 +1841,11 @@ struct octofmm_plan {
     std::vector<int2> h_items;     // the work items (host copy, for the tuning key)
     uint64_t* d_mixbits = nullptr;
     // mixed precision, lane mappings 3 and 7: the mixed-precision records and
-    // the far-schedule entries evaluated in FP32 as a whole (Tables::sched order)
+    // the far schedule with the entries that stay FP64 (the first mix_n64) before
+    // those evaluated in FP32 as a whole
     double* d_recm = nullptr;
-    uint8_t* d_mixoff = nullptr;
+    int32_t* d_mixorder = nullptr;
+    int32_t mix_n64 = 0;
     uint32_t* d_queue = nullptr;   // per-XCD work counters of the persistent variants
     int32_t n_p2m = 0;             // leaf items with p2m: items [n_m2l, n_m2l + n_p2m)
     double* d_p2m_out = nullptr;   // their p2m sums [n_p2m][512][8]
@@ -1987,6 +2067,7 @@ static octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace&
     sa.foff = w.meta + kMetaFoff;
     sa.rec = w.rec;
     sa.recm = nullptr;
+    sa.rho = rho;
     sa.list = nullptr;
     sa.dx = dx;
     sa.nslots = 27;
@@ -2029,7 +2110,8 @@ static octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace&
         la.tab = c->d_tab;
         la.mixbits = nullptr;
         la.recm = nullptr;
-        la.mixoff = nullptr;
+        la.mixorder = nullptr;
+        la.mix_n64 = 0;
         la.queue = nullptr;
         la.mon = w.mon;
         la.p2m_out = w.p2m;
@@ -2248,7 +2330,7 @@ static void plan_free(octofmm_plan* p) {
     (void)hipFree(p->d_items);
     (void)hipFree(p->d_mixbits);
     (void)hipFree(p->d_recm);
-    (void)hipFree(p->d_mixoff);
+    (void)hipFree(p->d_mixorder);
     (void)hipFree(p->d_queue);
     (void)hipFree(p->d_p2m_out);
     (void)hipFree(p->d_partial);
@@ -2281,6 +2363,7 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         sa.foff = p->d_foff;
         sa.rec = p->d_rec;
         sa.recm = p->d_recm;
+        sa.rho = p->type == OCTOFMM_RHO;
         sa.list = p->d_stage_list;
         sa.dx = p->dx;
         sa.nslots = p->d_stage_list ? p->n_stage : p->nslots;
@@ -2322,7 +2405,8 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         la.tab = c->d_tab;
         la.mixbits = p->d_mixbits;
         la.recm = p->d_recm;
-        la.mixoff = p->d_mixoff;
+        la.mixorder = p->d_mixorder;
+        la.mix_n64 = p->mix_n64;
         la.queue = p->d_queue;
         la.mon = p->d_mon;
         la.p2m_out = p->d_p2m_out;
@@ -2837,16 +2921,19 @@ static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* 
         // split entries of opposite face offsets stage FP64 records only, so
         // their offsets stay FP64 (at mixed_far_d2 >= 4 they hold |d| = 2
         // pairs and would anyway)
-        std::vector<uint8_t> mo(T.nsched > 0 ? T.nsched : 1, 0);
+        std::vector<int32_t> order, fp32;
         std::vector<char> whole(T.ndelta > 0 ? T.ndelta : 1, 0);
         for (int q = 0; q < T.nsched; ++q) {
-            if ((T.sched[q] >> 16) & 0xff) continue;
             const int di = T.sched[q] & 0xff;
-            whole[di] = T.farbits[di] != 0 && mb[di] == T.farbits[di];
-            mo[q] = whole[di] ? 1 : 0;
+            const bool w = ((T.sched[q] >> 16) & 0xff) == 0 && T.farbits[di] != 0 && mb[di] == T.farbits[di];
+            if (w) whole[di] = 1;
+            (w ? fp32 : order).push_back(q);
         }
-        if (hipMalloc((void**)&p->d_mixoff, mo.size()) != hipSuccess ||
-            hipMemcpy(p->d_mixoff, mo.data(), mo.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        p->mix_n64 = (int32_t)order.size();
+        order.insert(order.end(), fp32.begin(), fp32.end());
+        if (order.empty()) order.push_back(0);
+        if (hipMalloc((void**)&p->d_mixorder, sizeof(int32_t) * order.size()) != hipSuccess ||
+            hipMemcpy(p->d_mixorder, order.data(), sizeof(int32_t) * order.size(), hipMemcpyHostToDevice) != hipSuccess ||
             hipMalloc((void**)&p->d_recm, (size_t)ns * kCells * kRecDoubles * sizeof(double) + kRecTailBytes) !=
                 hipSuccess)
             return cleanup(OCTOFMM_ERR_ALLOCATION, "mixed-precision record allocation failed");

@@ -11,10 +11,9 @@ namespace octofmm {
 
 constexpr int kInx = 8;
 constexpr int kCells = 512;
-constexpr int kRecDoubles = 24;       // partner record: m0, M1..M19, Y0..Y2, mon
+constexpr int kRecDoubles = 24;       // partner record: m0, scaled moments, Y0..Y2 (kernels.hpp)
 constexpr int kRecBytes = kRecDoubles * 8;
-constexpr int kRecY = 20;
-constexpr int kRecMon = 23;
+constexpr int kRecY = 21;
 constexpr int kMaxDelta = 125;        // coarse offsets in [-2, 2]^3 (theta >= 0.34)
 constexpr int kStencilInx = 11;       // stencil box edge (offsets -5..5)
 constexpr int kStencilBox = kStencilInx * kStencilInx * kStencilInx;

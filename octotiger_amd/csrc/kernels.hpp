@@ -701,30 +701,28 @@ __host__ __device__ constexpr int tmap3(int a, int b, int c) {
 }
 
 // taylor::operator>>= : B = A moved from its centre by X (X = old - new centre).
+// Each order takes the finished lower one as a factor: with T_ac = A_ac + A_a X_c,
+//   B_a = A_a + A X_a,  B_ab = A_ab + A_a X_b + X_a B_b,
+//   B_abc = A_abc + A_ab X_c + X_b T_ac + X_a B_bc,
+// 51 fused multiply-adds, where the expanded sums take about 190 operations.
 __device__ __forceinline__ void multipole_shift(const double* A, const double* X, double* B) {
+    B[0] = A[0];
 #pragma unroll
-    for (int i = 0; i < 20; ++i) B[i] = A[i];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) B[1 + a] += A[0] * X[a];
+    for (int a = 0; a < 3; ++a) B[1 + a] = fma(A[0], X[a], A[1 + a]);
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
-        for (int b = a; b < 3; ++b) {
-            B[tmap2(a, b)] += A[1 + a] * X[b] + X[a] * A[1 + b];
-            B[tmap2(a, b)] += A[0] * X[a] * X[b];
+        for (int b = a; b < 3; ++b) B[tmap2(a, b)] = fma(X[a], B[1 + b], fma(A[1 + a], X[b], A[tmap2(a, b)]));
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int c = a; c < 3; ++c) {
+            const double t = fma(A[1 + a], X[c], A[tmap2(a, c)]);
+#pragma unroll
+            for (int b = a; b <= c; ++b)
+                B[tmap3(a, b, c)] =
+                    fma(X[a], B[tmap2(b, c)], fma(X[b], t, fma(A[tmap2(a, b)], X[c], A[tmap3(a, b, c)])));
         }
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = a; b < 3; ++b)
-#pragma unroll
-            for (int c = b; c < 3; ++c) {
-                double t = B[tmap3(a, b, c)];
-                t += A[tmap2(a, b)] * X[c] + A[tmap2(b, c)] * X[a] + A[tmap2(c, a)] * X[b];
-                t += A[1 + a] * X[b] * X[c] + A[1 + b] * X[c] * X[a] + A[1 + c] * X[a] * X[b];
-                t += A[0] * X[a] * X[b] * X[c];
-                B[tmap3(a, b, c)] = t;
-            }
 }
 
 // multipole_shift for A = (m, 0, ..., 0), a cell that holds only its mass:
@@ -745,38 +743,31 @@ __device__ __forceinline__ void monopole_shift(double m, const double* X, double
             for (int c = b; c < 3; ++c) B[tmap3(a, b, c)] = m * X[a] * X[b] * X[c];
 }
 
-// taylor::operator<<= : B = local expansion A re-expanded at +X.
+// taylor::operator<<= : B = local expansion A re-expanded at +X.  With w_ab =
+// A_abc X_c, v_a = w_ab X_b and q_a = A_ab X_b,
+//   B_ab = A_ab + w_ab,  B_a = A_a + q_a + v_a / 2,
+//   B = A + X_a (A_a + q_a / 2 + v_a / 6),
+// 57 operations, where the expanded sums take about 280.
 __device__ __forceinline__ void local_shift(const double* A, const double* X, double* B) {
-#pragma unroll
-    for (int i = 0; i < 20; ++i) B[i] = A[i];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) B[0] += A[1 + a] * X[a];
+    double w[10];   // by tmap2
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
-        for (int b = 0; b < 3; ++b) B[0] += A[tmap2(a, b)] * X[a] * X[b] * 0.5;
+        for (int b = a; b < 3; ++b)
+            w[tmap2(a, b)] =
+                fma(A[tmap3(a, b, 2)], X[2], fma(A[tmap3(a, b, 1)], X[1], A[tmap3(a, b, 0)] * X[0]));
+    B[0] = A[0];
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+    for (int a = 0; a < 3; ++a) {
+        const double v = fma(w[tmap2(a, 2)], X[2], fma(w[tmap2(a, 1)], X[1], w[tmap2(a, 0)] * X[0]));
+        const double q = fma(A[tmap2(a, 2)], X[2], fma(A[tmap2(a, 1)], X[1], A[tmap2(a, 0)] * X[0]));
+        B[1 + a] = fma(0.5, v, A[1 + a] + q);
+        B[0] = fma(fma(1.0 / 6.0, v, fma(0.5, q, A[1 + a])), X[a], B[0]);
+    }
 #pragma unroll
-        for (int b = 0; b < 3; ++b) B[1 + a] += A[tmap2(a, b)] * X[b];
+    for (int i = 4; i < 10; ++i) B[i] = A[i] + w[i];
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) B[0] += A[tmap3(a, b, c)] * X[a] * X[b] * X[c] * (1.0 / 6.0);
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) B[1 + a] += A[tmap3(a, b, c)] * X[b] * X[c] * 0.5;
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-#pragma unroll
-            for (int c = a; c < 3; ++c) B[tmap2(a, c)] += A[tmap3(a, b, c)] * X[b];
+    for (int i = 10; i < 20; ++i) B[i] = A[i];
 }
 
 // parent cell holding coarse cell (ip, jp, kp) of a node in octant o

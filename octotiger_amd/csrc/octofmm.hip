@@ -361,59 +361,6 @@ __device__ __forceinline__ void finish_cell(const LevelArgs& a, int slot, int ce
     }
 }
 
-// Leaf epilogue of a whole-tree RHO solve, with the rows staged through LDS so
-// that the sub-grid's L, L_c and g blocks (contiguous: 512 rows of 20, 3 and 4
-// doubles) are written by consecutive lanes in consecutive 16-byte chunks.
-// Written straight from the class waves, each store instruction would touch
-// 64 rows two cells apart.  L goes in two halves of 256 cells (40 KiB of
-// LDS), then L_c and g together (28 KiB); without a.leaf_rows only L_c and
-// g.  Every thread of the workgroup calls it; buf is the kernel's dynamic
-// LDS, no longer in use.
-__device__ __forceinline__ void leaf_rows_coalesced(const LevelArgs& a, int slot, int cell, const double* Lf,
-    const double* Cf, const double* g4, double* __restrict__ buf) {
-    // Each staged row, L_c triple and g quadruple is shifted by one more
-    // element every 16 cells (c >> 4): the lanes of a wave hold cells 2 apart
-    // in z, 16 in y and 128 in x, and without the shift their rows fall on a
-    // quarter of the LDS banks (8-way conflicts on the row writes, 4-way on
-    // L_c, 8-way on g); with it each half-wave spreads over all of them.
-    const int t = threadIdx.x;
-    double2* b2 = reinterpret_cast<double2*>(buf);
-    for (int half = 0; half < (a.leaf_rows ? 2 : 0); ++half) {   // uniform
-        __syncthreads();
-        if ((cell >> 8) == half) {
-            const int c = cell & 255;
-            double2* row = b2 + c * 10 + (c >> 4);
-#pragma unroll
-            for (int j = 0; j < 10; ++j) row[j] = make_double2(Lf[2 * j], Lf[2 * j + 1]);
-        }
-        __syncthreads();
-        double2* dst = reinterpret_cast<double2*>(a.L + ((size_t)slot * kCells + half * 256) * 20);
-#pragma unroll
-        for (int r = 0; r < 5; ++r) {   // 256 rows x 10 chunks
-            const int ch = t + 512 * r;
-            store_stream(dst + ch, b2[ch + (ch / 10 >> 4)]);
-        }
-    }
-    __syncthreads();
-    buf[cell * 3 + (cell >> 4) + 0] = Cf[0];
-    buf[cell * 3 + (cell >> 4) + 1] = Cf[1];
-    buf[cell * 3 + (cell >> 4) + 2] = Cf[2];
-    double2* bg = b2 + 784;   // after the 1536 + 32 doubles of L_c
-    bg[cell * 2 + (cell >> 4)] = make_double2(g4[0], g4[1]);
-    bg[cell * 2 + (cell >> 4) + 1] = make_double2(g4[2], g4[3]);
-    __syncthreads();
-    double2* lc = reinterpret_cast<double2*>(a.Lc + (size_t)slot * kCells * 3);
-    double2* gg = reinterpret_cast<double2*>(a.g + (size_t)slot * kCells * 4);
-    auto lc_pair = [&](int ch) {   // doubles 2 ch and 2 ch + 1 of the L_c block
-        const int d0 = 2 * ch, d1 = d0 + 1;
-        return make_double2(buf[d0 + (d0 / 3 >> 4)], buf[d1 + (d1 / 3 >> 4)]);
-    };
-    store_stream(lc + t, lc_pair(t));                 // 768 chunks of L_c
-    if (t < 256) store_stream(lc + 512 + t, lc_pair(512 + t));
-    store_stream(gg + t, bg[t + (t >> 5)]);           // 1024 chunks of g (cell = chunk / 2)
-    store_stream(gg + 512 + t, bg[512 + t + ((512 + t) >> 5)]);
-}
-
 // Mixed-precision kernels: the expansion of a target's FP64 pairs, once they
 // are all in s, and after the FP32 ones the correction, whose sums go on.
 template <bool RHO>
@@ -908,7 +855,8 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
     }
 }
 
-// Leaf targets (monopole kernels): one 512-lane workgroup per leaf sub-grid.
+// Leaf targets (monopole kernels), list-driven for any opening angle: one
+// 512-lane workgroup per leaf sub-grid.
 // The monopoles of the sub-grid and of its leaf neighbours within the stencil
 // reach are staged once into an LDS window (zeros for refined or missing
 // neighbours, whose cells the monopole kernel does not see).  Wave w takes
@@ -921,25 +869,28 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
 // stencil, far and near alike (monopole_kernel_templates.hpp:69-239): those
 // sums come from p2m_kernel, launched before this kernel on the same stream.
 
-// LDS layout of the 14^3 monopole window of the theta = 0.5 leaf kernel: 8
-// parity planes (x & 1, y & 1, z & 1) of 7^3 cells each, row stride 12 and
-// plane stride 80 doubles.  At each partner offset a wave's 64 lanes read
-// cells 2C + const over the 4^3 coarse cells C, i.e. consecutive cells of
-// one parity plane: with strides 1, 12 and 80 (mod 32: 1, 12, 16) the 32
-// lanes of each half-wave hit 32 distinct 8-byte bank pairs.  In the plain
-// x-slowest layout the lanes' stride of 2 cells put 4 of them on every bank
-// pair in use.
-constexpr int kWinSY = 12, kWinSX = 80, kWinPlane = 7 * kWinSX;
-__device__ __forceinline__ int cube_win(int wx, int wy, int wz) {
-    return (((wx & 1) << 2) | ((wy & 1) << 1) | (wz & 1)) * kWinPlane + (wx >> 1) * kWinSX + (wy >> 1) * kWinSY + (wz >> 1);
+// The p2m sums (p2m_kernel) of cell `cell` of p2m item `ordinal` join the p2p
+// ones.  Leaf items with p2m come first among the leaf items, so the item's
+// place among them indexes p2m_out.
+__device__ __forceinline__ void add_p2m(const LevelArgs& a, int ordinal, int cell, double* L, double* C) {
+    const double2* ps = reinterpret_cast<const double2*>(a.p2m_out + ((size_t)ordinal * kCells + cell) * 8);
+    const double2 v0 = ps[0], v1 = ps[1], v2 = ps[2], v3 = ps[3];
+    L[0] += v0.x;
+    L[1] += v0.y;
+    L[2] += v1.x;
+    L[3] += v1.y;
+    C[0] = v2.x;
+    C[1] = v2.y;
+    C[2] = v3.x;
 }
 
-template <bool RHO, bool CUBE>
+template <bool RHO>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void leaf_kernel(LevelArgs a) {
     extern __shared__ double s_win[];
     __shared__ int s_nbr[27];
     __shared__ int s_kind[27];
-    const int2 it = a.items[a.item0 + xcd_item(blockIdx.x, gridDim.x)];
+    const int ordinal = xcd_item(blockIdx.x, gridDim.x);
+    const int2 it = a.items[a.item0 + ordinal];
     const int slot = it.x;
     if (threadIdx.x < 27) {
         const int n = a.nbr[(size_t)slot * 27 + threadIdx.x];
@@ -948,10 +899,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void l
     }
     __syncthreads();
     const Tables* __restrict__ tab = a.tab;
-    // window edge: 14 (halo 3) on the cube path, known at compile time, so the
-    // gather's index arithmetic folds and its loads are all in flight at once
-    const int h = CUBE ? 3 : tab->p2p_halo, W = kInx + 2 * h;
-    auto gather = [&](int i) {
+    const int h = tab->p2p_halo, W = kInx + 2 * h;
+    for (int i = threadIdx.x; i < W * W * W; i += 512) {
         const int x = i / (W * W) - h, y = (i / W) % W - h, z = i % W - h;
         const int raw = (x < 0 ? 0 : x < kInx ? 1 : 2) + 3 * (y < 0 ? 0 : y < kInx ? 1 : 2) +
             9 * (z < 0 ? 0 : z < kInx ? 1 : 2);
@@ -959,97 +908,354 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void l
         double m = 0.0;
         if (ns >= 0 && s_kind[raw] == OCTOFMM_SLOT_LEAF)
             m = a.mon[(size_t)ns * kCells + ((x + kInx) & 7) * 64 + ((y + kInx) & 7) * 8 + ((z + kInx) & 7)];
-        if constexpr (CUBE) {
-            const int wx = x + h, wy = y + h, wz = z + h;
-            s_win[cube_win(wx, wy, wz)] = m;
-        } else {
-            s_win[i] = m;
-        }
-    };
-    if constexpr (CUBE) {
-        constexpr int kWin = 14 * 14 * 14;
-#pragma unroll
-        for (int r = 0; r < (kWin + 511) / 512; ++r)
-            if (threadIdx.x + r * 512 < kWin) gather(threadIdx.x + r * 512);
-    } else {
-        for (int i = threadIdx.x; i < W * W * W; i += 512) gather(i);
+        s_win[i] = m;
     }
     __syncthreads();
     const int k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = threadIdx.x & 63;
-    const int Cx = l >> 4, Cy = (l >> 2) & 3, Cz = l & 3;
-    const int kx = (k >> 2) & 1, ky = (k >> 1) & 1, kz = k & 1;
-    const int tx = 2 * Cx + kx, ty = 2 * Cy + ky, tz = 2 * Cz + kz;
+    const int tx = 2 * (l >> 4) + ((k >> 2) & 1), ty = 2 * ((l >> 2) & 3) + ((k >> 1) & 1), tz = 2 * (l & 3) + (k & 1);
     const int cell = tx * 64 + ty * 8 + tz;
     double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-    if constexpr (CUBE) {
-        // the 6^3 block 2C - 2 .. 2C + 3 around the target's coarse cell C
-        // (the target itself included: four of offset 0 is zero), with the
-        // window offsets as LDS immediates and the constants of offset
-        // d = p - k at fixed offsets from one class base:
-        // box(d) = box(p) + 3 * 133 - (121 kx + 11 ky + kz) for p in [0, 6)^3
-        // window cell 2C + 1 + p lies in parity plane (1 + p) & 1 at index
-        // C + ((1 + p) >> 1): the lane's base plus a compile-time offset
-        const double* wc = s_win + Cx * kWinSX + Cy * kWinSY + Cz;
-        const double(*__restrict__ fb)[4] = tab->four + (3 * 133 - (121 * kx + 11 * ky + kz));
-#pragma unroll
-        for (int px = 0; px < 6; ++px)
-#pragma unroll
-            for (int py = 0; py < 6; ++py)
-#pragma unroll
-                for (int pz = 0; pz < 6; ++pz) {
-                    const double m = wc[cube_win(1 + px, 1 + py, 1 + pz)];
-                    const double* f = fb[px * 121 + py * 11 + pz];
-                    p0 = fma(f[0], m, p0);
-                    p1 = fma(f[1], m, p1);
-                    p2 = fma(f[2], m, p2);
-                    p3 = fma(f[3], m, p3);
-                }
-    } else {
-        const double* wp = s_win + ((tx + h) * W + (ty + h)) * W + (tz + h) - 2048;
-        const int32_t* __restrict__ list = tab->p2plist[k];
-        const char* __restrict__ fc = reinterpret_cast<const char*>(tab->p2pconst);
-        const int n = tab->np2p_k[k];
+    const double* wp = s_win + ((tx + h) * W + (ty + h)) * W + (tz + h) - 2048;
+    const int32_t* __restrict__ list = tab->p2plist[k];
+    const char* __restrict__ fc = reinterpret_cast<const char*>(tab->p2pconst);
+    const int n = tab->np2p_k[k];
 #pragma unroll 8
-        for (int q = 0; q < n; ++q) {
-            const int e = list[q];
-            const double* f = reinterpret_cast<const double*>(fc + (e & 0xffff));
-            const double m = wp[e >> 16];
-            p0 = fma(f[0], m, p0);
-            p1 = fma(f[1], m, p1);
-            p2 = fma(f[2], m, p2);
-            p3 = fma(f[3], m, p3);
-        }
+    for (int q = 0; q < n; ++q) {
+        const int e = list[q];
+        const double* f = reinterpret_cast<const double*>(fc + (e & 0xffff));
+        const double m = wp[e >> 16];
+        p0 = fma(f[0], m, p0);
+        p1 = fma(f[1], m, p1);
+        p2 = fma(f[2], m, p2);
+        p3 = fma(f[3], m, p3);
     }
     const double s1 = a.inv_dx * a.neg_inv_dx;
     double L[4] = {p0 * a.inv_dx, p1 * s1, p2 * s1, p3 * s1};
     double C[3] = {0.0, 0.0, 0.0};
     const bool p2m = (it.y & kItemP2M) != 0;
-    if (p2m) {
-        // refined neighbours: the p2m sums p2m_kernel formed for this leaf
-        // (leaf items with p2m come first among the leaf items, so the item's
-        // place among them indexes p2m_out)
-        const double2* ps = reinterpret_cast<const double2*>(
-            a.p2m_out + ((size_t)xcd_item(blockIdx.x, gridDim.x) * kCells + cell) * 8);
-        const double2 v0 = ps[0], v1 = ps[1], v2 = ps[2], v3 = ps[3];
-        L[0] += v0.x;
-        L[1] += v0.y;
-        L[2] += v1.x;
-        L[3] += v1.y;
-        C[0] = v2.x;
-        C[1] = v2.y;
-        C[2] = v3.x;
+    if (p2m) add_p2m(a, ordinal, cell, L, C);
+    finish_cell<RHO>(a, slot, cell, L, 4, C, p2m, true);
+}
+
+// Two consecutive doubles in one 16-byte load, from an address that need not
+// be 16-byte aligned.
+typedef double double2_a8 __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ void load2(const double* __restrict__ p, double* v) {
+    const double2_a8 d = *reinterpret_cast<const double2_a8*>(p);
+    v[0] = d.x;
+    v[1] = d.y;
+}
+
+// LDS layout of the 14^3 monopole window of leaf_cube_kernel: 8 parity planes
+// (x & 1, y & 1, z & 1) of 7^3 cells each, row stride 12 and plane stride 80
+// doubles.  At each partner offset a wave's 64 lanes read cells 2C + const
+// over the 4^3 coarse cells C, i.e. consecutive cells of one parity plane:
+// with strides 1, 12 and 80 (mod 32: 1, 12, 16) the 32 lanes of each half-wave
+// hit 32 distinct 8-byte bank pairs.  In the plain x-slowest layout the lanes'
+// stride of 2 cells put 4 of them on every bank pair in use.
+constexpr int kWinSY = 12, kWinSX = 80, kWinPlane = 7 * kWinSX;
+__device__ __forceinline__ int cube_win(int wx, int wy, int wz) {
+    return (((wx & 1) << 2) | ((wy & 1) << 1) | (wz & 1)) * kWinPlane + (wx >> 1) * kWinSX + (wy >> 1) * kWinSY + (wz >> 1);
+}
+
+// Sums of the p2p constants over one target's partners: potential, x, and the
+// odd y and z sums by |offset| 1, 2, 3.
+struct P2pSums {
+    double p, x, y[3], z[3];
+};
+
+// One row (or fold of two opposite rows) of a plane: even sums E[|dz|], odd
+// sums O[|dz|]; f = Tables::p2pfold[|dx|][|dy|].  Returns sum E / r^3.
+__device__ __forceinline__ double p2p_row(const __attribute__((address_space(4))) double* f, const double* E, const double* O, P2pSums& s) {
+    s.p = fma(f[3], E[3], fma(f[2], E[2], fma(f[1], E[1], fma(f[0], E[0], s.p))));
+#pragma unroll
+    for (int j = 0; j < 3; ++j) s.z[j] = fma(f[5 + j], O[1 + j], s.z[j]);
+    return fma(f[7], E[3], fma(f[6], E[2], fma(f[5], E[1], f[4] * E[0])));
+}
+
+// Forms the sums at this point (the constraint exists only in the device pass).
+__device__ __forceinline__ void form_vgprs(P2pSums& s) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(s.p), "+v"(s.x), "+v"(s.y[0]), "+v"(s.y[1]), "+v"(s.y[2]), "+v"(s.z[0]), "+v"(s.z[1]), "+v"(s.z[2]));
+#else
+    (void)s;
+#endif
+}
+
+// p2p of one lane's two targets, the children (0, ky, kz) and (1, ky, kz) of
+// coarse cell (Cx, Cy, Cz), over the 6^3 block of cells 2C - 2 .. 2C + 3, all
+// within one window.  Per axis a target of child bit 0 sees the offsets
+// -2 .. 3, of child bit 1 -3 .. 2: two opposite pairs, 0, and one end e = +-3.
+// 1/r and 1/r^3 are even in every offset, so opposite cells are added (for
+// the even sums) and subtracted (for the odd ones) before they meet their
+// constant, first along z for each row, then along y for each pair of rows.
+// The folded rows of a plane serve both targets.
+__device__ __forceinline__ void p2p_cube(const double* s_win, int Cx, int Cy, int Cz, int ky, int kz,
+    const Tables* tab, P2pSums* s) {
+    // window coordinate of the targets' row centre: 2C + 3 + k; "same" rows
+    // and columns (offsets 0, +-2) lie in its parity plane, "other" ones
+    // (+-1, and the end +-3) in the opposite one
+    const int zs = (1 - kz) * kWinPlane + Cz + kz;                 // offset -2
+    const int zo = kz * kWinPlane + Cz + 1;                         // offset -1
+    const int ze = zo + (kz ? -1 : 2);                              // the end
+    const int ys = (1 - ky) * 2 * kWinPlane + (Cy + ky) * kWinSY;   // offset -2
+    const int yo = ky * 2 * kWinPlane + (Cy + 1) * kWinSY;          // offset -1
+    const int ye = yo + (ky ? -1 : 2) * kWinSY;                     // the end
+    const double* w = s_win + Cx * kWinSX;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        s[t].p = s[t].x = 0.0;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) s[t].y[j] = s[t].z[j] = 0.0;
     }
-    if constexpr (RHO) {
-        if (a.l2l && a.g) {   // uniform: whole-tree RHO solve
-            double Lf[20], Cf[3], g4[4];
-            tree_final_row<RHO>(a, slot, cell, L, 4, C, p2m, Lf, Cf);
-            leaf_force<RHO>(a, Lf, Cf, g4);
-            leaf_rows_coalesced(a, slot, cell, Lf, Cf, g4, s_win);
-            return;
+#pragma unroll
+    for (int px = 0; px < 6; ++px) {   // plane x = 2C - 2 + px
+        const double* wx = w + ((1 + px) & 1) * 4 * kWinPlane + ((1 + px) >> 1) * kWinSX;
+        auto row = [&](int y, double* E, double* O) {
+            const double* r = wx + y;
+            const double a = r[zo], b = r[zo + 1], c = r[zs], d = r[zs + 2], e = r[ze];
+            E[0] = r[zs + 1];
+            E[1] = b + a;
+            O[1] = b - a;
+            E[2] = d + c;
+            O[2] = d - c;
+            E[3] = O[3] = e;
+        };
+        double u[2] = {0.0, 0.0};   // sum / r^3 over the plane, even in y and z
+        // constants of this plane by |dx| (the opaque pointer, the scheduling
+        // fences and form_vgprs keep each group of rows to its own loads and
+        // sums: without them all planes' rows and constants are held at once
+        // and spill)
+        const char* fold = uniform_ptr(reinterpret_cast<const char*>(&tab->p2pfold[0][0][0]));
+        auto consts = [&](int t, int ay) {
+            const int ax = px - 2 - t < 0 ? 2 + t - px : px - 2 - t;
+            return as_const(reinterpret_cast<const double*>(fold)) + (ax * 4 + ay) * 8;
+        };
+        __builtin_amdgcn_sched_barrier(0);
+        {
+            double E[4], O[4];
+            row(ys + kWinSY, E, O);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) u[t] += p2p_row(consts(t, 0), E, O, s[t]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        {
+            double E[4], O[4];
+            row(ye, E, O);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const double v = p2p_row(consts(t, 3), E, O, s[t]);
+                u[t] += v;
+                s[t].y[2] += v;
+            }
+        }
+#pragma unroll
+        for (int dy = 1; dy < 3; ++dy) {
+            __builtin_amdgcn_sched_barrier(0);
+            const int lo = dy == 1 ? yo : ys, step = dy == 1 ? kWinSY : 2 * kWinSY;
+            double E[4], O[4], F[4], P[4];
+            row(lo, E, O);
+            row(lo + step, F, P);
+            double D[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                D[j] = F[j] - E[j];
+                E[j] += F[j];
+            }
+#pragma unroll
+            for (int j = 1; j < 4; ++j) O[j] += P[j];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const auto* f = consts(t, dy);
+                u[t] += p2p_row(f, E, O, s[t]);
+                s[t].y[dy - 1] =
+                    fma(f[7], D[3], fma(f[6], D[2], fma(f[5], D[1], fma(f[4], D[0], s[t].y[dy - 1]))));
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+            if (px != 2 + t) s[t].x = fma((double)(px - 2 - t), u[t], s[t].x);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) form_vgprs(s[t]);
+    }
+    const double ey = ky ? -3.0 : 3.0, ez = kz ? -3.0 : 3.0;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        s[t].y[0] = fma(ey, s[t].y[2], fma(2.0, s[t].y[1], s[t].y[0]));
+        s[t].z[0] = fma(ez, s[t].z[2], fma(2.0, s[t].z[1], s[t].z[0]));
+    }
+}
+
+// Leaf targets at theta = 0.5 (Tables::p2p_cube): one 4-wave workgroup per
+// leaf, wave = child bits (ky, kz), lane = coarse cell, two targets (kx = 0,
+// 1) per lane.  FP64 VALU issue and LDS reads bound the p2p loop: per target
+// it takes ~460 FP64 operations and 108 LDS reads, where one target per lane
+// with a multiply-add per constant took 864 and 216.
+//
+// In a whole-tree solve the final rows (L 20, L_c 3, g 4 doubles a cell) go
+// through LDS and leave as the sub-grid's contiguous blocks, consecutive lanes
+// in consecutive 16-byte chunks: the L rows of kx = 0 (the even x planes, 40
+// KiB), then those of kx = 1, then L_c and g together.  Written straight from
+// the lanes each store would touch 64 rows.  Each staged row, L_c triple and
+// g quadruple is shifted by one more element every 16 cells: without that the
+// lanes' rows (2 cells apart in z, 16 in y) fall on a quarter of the banks.
+template <bool RHO>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void leaf_cube_kernel(LevelArgs a) {
+    extern __shared__ double s_win[];
+    __shared__ int s_nbr[27];
+    __shared__ int s_kind[27];
+    const int ordinal = xcd_item(blockIdx.x, gridDim.x);
+    const int2 it = a.items[a.item0 + ordinal];
+    const int slot = it.x;
+    const int th = threadIdx.x;
+    if (th < 27) {
+        const int n = a.nbr[(size_t)slot * 27 + th];
+        s_nbr[th] = n;
+        s_kind[th] = n >= 0 ? a.kind[n] : -1;
+    }
+    __syncthreads();
+    // the monopole window, one thread per row of 14 cells along z (3 of the
+    // slot below, 8, 3 of the slot above): all of a row's loads are in flight
+    // at once and its index arithmetic is done once (a thread per cell spent
+    // as many VALU instructions on it as half the p2p loop).  Zeros for refined
+    // or missing neighbours.
+    if (th < 14 * 14) {
+        const int wx = th / 14, wy = th % 14;
+        const int x = wx - 3, y = wy - 3;
+        const int rxy = (x < 0 ? 0 : x < kInx ? 1 : 2) + 3 * (y < 0 ? 0 : y < kInx ? 1 : 2);
+        const size_t at = (size_t)((x & 7) * 64 + (y & 7) * 8);
+        const double* src[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const int ns = s_nbr[rxy + 9 * q];
+            src[q] = ns >= 0 && s_kind[rxy + 9 * q] == OCTOFMM_SLOT_LEAF ? a.mon + (size_t)ns * kCells + at : nullptr;
+        }
+        double m[14];
+#pragma unroll
+        for (int i = 0; i < 14; ++i) m[i] = 0.0;
+        // (the caller's monopoles are 8-byte aligned only)
+        if (src[0]) {
+            m[0] = src[0][5];
+            load2(src[0] + 6, m + 1);
+        }
+        if (src[1]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) load2(src[1] + 2 * i, m + 3 + 2 * i);
+        }
+        if (src[2]) {
+            load2(src[2], m + 11);
+            m[13] = src[2][2];
+        }
+        double* row = s_win + cube_win(wx, wy, 0);
+#pragma unroll
+        for (int i = 0; i < 14; ++i) row[(i & 1) * kWinPlane + (i >> 1)] = m[i];
+    }
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane(th >> 6);
+    const int ky = wave >> 1, kz = wave & 1;
+    const int l = th & 63;
+    const int Cx = l >> 4, Cy = (l >> 2) & 3, Cz = l & 3;
+    P2pSums s[2];
+    p2p_cube(s_win, Cx, Cy, Cz, ky, kz, a.tab, s);
+    const int cell0 = Cx * 128 + (2 * Cy + ky) * 8 + 2 * Cz + kz;   // kx = 0; kx = 1 is 64 further
+    const double s1 = a.inv_dx * a.neg_inv_dx;
+    const bool p2m = (it.y & kItemP2M) != 0;
+    double L[2][4], C[2][3];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        L[t][0] = s[t].p * a.inv_dx;
+        L[t][1] = s[t].x * s1;
+        L[t][2] = s[t].y[0] * s1;
+        L[t][3] = s[t].z[0] * s1;
+        C[t][0] = C[t][1] = C[t][2] = 0.0;
+        if (p2m) add_p2m(a, ordinal, cell0 + 64 * t, L[t], C[t]);
+    }
+    if (!a.l2l) {   // uniform
+#pragma unroll
+        for (int t = 0; t < 2; ++t) finish_cell<RHO>(a, slot, cell0 + 64 * t, L[t], 4, C[t], p2m, true);
+        return;
+    }
+    // both targets lie in one parent cell
+    double A[20], Y[3] = {0.0, 0.0, 0.0}, lc[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < 20; ++j) A[j] = 0.0;
+    const int pn = a.parent[slot];
+    if (pn >= 0) {   // uniform
+        const size_t pr = (size_t)pn * kCells + parent_cell(a.octant[slot], Cx, Cy, Cz);
+        const double2* src = reinterpret_cast<const double2*>(a.pL + pr * 20);
+#pragma unroll
+        for (int j = 0; j < 10; ++j) {
+            const double2 v = src[j];
+            A[2 * j] = v.x;
+            A[2 * j + 1] = v.y;
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            Y[d] = a.pcom[pr * 3 + d];
+            if (RHO) lc[d] = a.pLc[pr * 3 + d];
         }
     }
-    finish_cell<RHO>(a, slot, cell, L, 4, C, p2m, true);
+    double2* b2 = reinterpret_cast<double2*>(s_win);
+    double Cf[2][3], g4[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const double* X = a.com + ((size_t)slot * kCells + cell0 + 64 * t) * 3;
+        const double dX[3] = {X[0] - Y[0], X[1] - Y[1], X[2] - Y[2]};
+        double Lf[20];
+        local_shift(A, dX, Lf);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) Lf[j] += L[t][j];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) Cf[t][d] = RHO ? C[t][d] + lc[d] : 0.0;
+        leaf_force<RHO>(a, Lf, Cf[t], g4[t]);
+        if (a.leaf_rows) {   // uniform
+            __syncthreads();   // the window (then the rows before) read
+            const int r = Cx * 64 + (cell0 & 63);
+            double2* row = b2 + r * 10 + (r >> 4);
+#pragma unroll
+            for (int j = 0; j < 10; ++j) row[j] = make_double2(Lf[2 * j], Lf[2 * j + 1]);
+            __syncthreads();
+            double2* dst = reinterpret_cast<double2*>(a.L + (size_t)slot * kCells * 20) + 640 * t;
+#pragma unroll
+            for (int i = 0; i < 10; ++i) {   // 256 rows x 10 chunks; row r is cell r + 64 (r / 64 + kx)
+                const int ch = th + 256 * i;
+                store_stream(dst + ch + ch / 640 * 640, b2[ch + (ch / 160)]);
+            }
+        }
+    }
+    if constexpr (RHO) {
+        __syncthreads();
+        double* buf = s_win;
+        double2* bg = b2 + 784;   // after the 1536 + 32 doubles of L_c
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int cell = cell0 + 64 * t;
+            buf[cell * 3 + (cell >> 4) + 0] = Cf[t][0];
+            buf[cell * 3 + (cell >> 4) + 1] = Cf[t][1];
+            buf[cell * 3 + (cell >> 4) + 2] = Cf[t][2];
+            bg[cell * 2 + (cell >> 4)] = make_double2(g4[t][0], g4[t][1]);
+            bg[cell * 2 + (cell >> 4) + 1] = make_double2(g4[t][2], g4[t][3]);
+        }
+        __syncthreads();
+        double2* lcd = reinterpret_cast<double2*>(a.Lc + (size_t)slot * kCells * 3);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {   // 768 chunks: doubles 2 ch and 2 ch + 1 of the L_c block
+            const int ch = th + 256 * i, d0 = 2 * ch, d1 = d0 + 1;
+            store_stream(lcd + ch, make_double2(buf[d0 + d0 / 48], buf[d1 + d1 / 48]));
+        }
+        if (a.g) {   // uniform
+            double2* gg = reinterpret_cast<double2*>(a.g + (size_t)slot * kCells * 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {   // 1024 chunks (cell = chunk / 2)
+                const int ch = th + 256 * i;
+                store_stream(gg + ch, bg[ch + (ch >> 5)]);
+            }
+        }
+    } else if (a.g) {   // phi slot only
+#pragma unroll
+        for (int t = 0; t < 2; ++t) a.g[((size_t)slot * kCells + cell0 + 64 * t) * 4] = g4[t][0];
+    }
 }
 
 // p2m on the staging of lane mapping 7: for leaf targets with refined
@@ -1223,16 +1429,15 @@ void launch_p2m(int nitems, hipStream_t st, const LevelArgs& la) {
 
 template <bool RHO>
 void launch_leaf(int nitems, hipStream_t st, const LevelArgs& la, const Tables& tab) {
-    const int W = kInx + 2 * tab.p2p_halo;
-    const bool cube = tab.p2p_cube != 0;
-    // window (parity planes on the cube path), and the staged L rows of half
-    // a sub-grid (256 x 20, shifted by one chunk every 16 rows)
-    const size_t win = cube ? (size_t)8 * kWinPlane : (size_t)W * W * W;
-    const size_t lds = sizeof(double) * std::max<size_t>(win, (size_t)256 * 20 + 32);
-    if (cube)
-        hipLaunchKernelGGL((leaf_kernel<RHO, true>), dim3(nitems), dim3(512), lds, st, la);
-    else
-        hipLaunchKernelGGL((leaf_kernel<RHO, false>), dim3(nitems), dim3(512), lds, st, la);
+    if (tab.p2p_cube) {
+        // the window's parity planes, or the staged L rows of 256 cells (20
+        // doubles each, shifted by one chunk every 16 rows)
+        const size_t lds = sizeof(double) * std::max<size_t>(8 * kWinPlane, 256 * 20 + 32);
+        hipLaunchKernelGGL(leaf_cube_kernel<RHO>, dim3(nitems), dim3(256), lds, st, la);
+    } else {
+        const int W = kInx + 2 * tab.p2p_halo;
+        hipLaunchKernelGGL(leaf_kernel<RHO>, dim3(nitems), dim3(512), sizeof(double) * W * W * W, st, la);
+    }
 }
 
 // One target sub-grid is split over 8 / WAVES workgroups of WAVES waves.  The

@@ -89,9 +89,12 @@ struct Tables {
     int32_t p2p_halo;
     // 1 when every class list is the whole 6^3 fine block around the target's
     // coarse cell minus the target (max |delta| = 1, i.e. theta = 0.5): the
-    // leaf kernel then walks that block with compile-time offsets and takes
-    // the constants straight from `four`
+    // leaf kernel then walks that block with compile-time offsets and folds
+    // opposite offsets before it multiplies (leaf_cube_kernel)
     int32_t p2p_cube;
+    // p2p constants of that block by |dx|, |dy|: -1/r for |dz| = 0..3, then
+    // 1/r^3 for |dz| = 0..3 (zeros at the target itself)
+    double p2pfold[4][4][8];
     int32_t np2p_k[8];
     int32_t p2plist[8][kMaxDelta * 8];
     // the distinct four-constant rows the eight lists use (342 at theta 0.5),

@@ -185,6 +185,14 @@ bool build_tables(double theta, Tables& t, char* err, size_t errlen) {
                 }
                 t.root_excluded[bi] = (!t.phase[bi] || (x == 0 && y == 0 && z == 0)) ? 1 : 0;
             }
+    for (int x = 0; x < 4; ++x)
+        for (int y = 0; y < 4; ++y)
+            for (int z = 0; z < 4; ++z) {
+                if (!(x || y || z)) continue;
+                const double r = std::sqrt(static_cast<double>(x * x + y * y + z * z));
+                t.p2pfold[x][y][z] = -1.0 / r;
+                t.p2pfold[x][y][4 + z] = 1.0 / (r * r * r);
+            }
     // coarse offsets passing the kernels' double-precision coarse test
     const double th2 = (1.0 / theta) * (1.0 / theta);
     int n = 0, maxd = 0;

@@ -663,6 +663,11 @@ struct LevelArgs {
     // persistent form of lane mapping 7: 8 work counters, one per XCD
     // (cleared by queue_reset before each launch)
     uint32_t* queue;
+    // variant 704 on small levels: workgroups per coarse block (0 or 1: the
+    // plain form), and their folded sums
+    // [item * 8 + block][part][kFolded][64]
+    double* wide_sums;
+    int32_t parts;
     int32_t nitems;
     int32_t item0;          // first item of this launch
     double inv_dx;

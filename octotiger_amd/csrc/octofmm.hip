@@ -383,6 +383,18 @@ __device__ __forceinline__ void finish_correction(const Acc<RHO>& s, const doubl
     }
 }
 
+// A target's neighbour slots and their kinds in LDS, for near_pairs (the far
+// pairs read the neighbour row through scalar loads).  Every thread of the
+// workgroup calls it.
+__device__ __forceinline__ void near_tables(const LevelArgs& a, int slot, int* s_nbr, int* s_kind) {
+    if (threadIdx.x < 27) {
+        const int n = a.nbr[(size_t)slot * 27 + threadIdx.x];
+        s_nbr[threadIdx.x] = n;
+        s_kind[threadIdx.x] = n >= 0 ? a.kind[n] : -1;
+    }
+    __syncthreads();
+}
+
 // Near pairs of a target cell over the coarse offsets di = first, first + step,
 // ...: partners in leaf slots, which carry only their monopole.
 template <bool RHO>
@@ -627,9 +639,14 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T* as_const(c
 // FP64 expansion after its 8 children; the other far offsets run in FP64.
 // The precision is uniform over the wave for each offset, so no lane waits
 // for the other precision's arithmetic.
-template <bool RHO, int SPLIT = 1, bool MIXED = false>
+//
+// WIDE (mapping 7 on small levels): the entries are split further over `parts` workgroups
+// (this one is `part`), and wave 0 leaves the folded sums of its 64 cells in
+// `sums` ([kFolded][64]) for level_reduce.
+template <bool RHO, int SPLIT = 1, bool MIXED = false, bool WIDE = false>
 __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const int* s_nbr, const int* s_kind,
-    int w, double2* __restrict__ s_stage, int sl = 0) {
+    int w, double2* __restrict__ s_stage, int sl = 0, int part = 0, double* __restrict__ sums = nullptr) {
+    static_assert(!(MIXED && WIDE), "the wide form is FP64");
     // this wave's image (wave-uniform address)
     double2* stage = s_stage + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kDirWave;
     // an opaque copy of the lane index: lane values formed from it are formed
@@ -664,8 +681,9 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
     // only the offsets with a far pair are staged (delta 0 is all near / self),
     // in the order of the far schedule
     const int nfd = tab->nsched;
-    const int q0 = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(sl);
-    // The wave's entries are those at positions q0, q0 + SPLIT, ... of the
+    const int step = WIDE ? SPLIT * a.parts : SPLIT;
+    const int q0 = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(WIDE ? part * SPLIT + sl : sl);
+    // The wave's entries are those at positions q0, q0 + step, ... of the
     // schedule; a mixed-precision plan orders it (a.mixorder) with its n64 FP64
     // entries first, so that the FP64 sums are done before the FP32 expansion
     // takes their registers.
@@ -760,11 +778,11 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
             }
         }
     };
-    if (flags & kItemNear) near_pairs<RHO>(a, lane_geom(wu), s_nbr, s_kind, q0, SPLIT, X0, X1, X2, s);
+    if (flags & kItemNear) near_pairs<RHO>(a, lane_geom(wu), s_nbr, s_kind, q0, step, X0, X1, X2, s);
     // the lane's group of 8 records in the image
     const double2* group = stage + (lane() >> 3) * kDirGroup;
     // One image: image(lanes of step j, records) between the arrival of
-    // position i's records and the refill with those of position i + SPLIT.
+    // position i's records and the refill with those of position i + step.
     auto walk = [&](int i, auto&& image) {
         // the lanes that read record j of the image: those of the classes in
         // byte j of the entry's step masks, unless their group's partner slot
@@ -779,19 +797,19 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
         const uint64_t eb = spread_groups(__builtin_amdgcn_readfirstlane(emptyb_next));
         const double2* recs =
             __builtin_amdgcn_inverse_ballot_w64(repeat_bytes(tab->sched_half[q] & 0xffu)) ? group + 48 : group;
-        if (i + SPLIT < nfd) bases(i + SPLIT);
+        if (i + step < nfd) bases(i + step);
         __builtin_amdgcn_s_waitcnt(0x3F70);   // vmcnt(0): this wave's image is in LDS
         __builtin_amdgcn_wave_barrier();
         image([&](int j) -> uint64_t { return step_lanes(ra, rb, ea, eb, j); }, recs);
         lds_wave_sync();   // every read of the image done before it is refilled
-        if (i + SPLIT < nfd) issue();
+        if (i + step < nfd) issue();
     };
     int i = q0;
     if (i < nfd) {
         bases(i);
         issue();
     }
-    for (; i < n64; i += SPLIT)
+    for (; i < n64; i += step)
         walk(i, [&](auto&& step_mask, const double2* recs) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -809,7 +827,7 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
         acc_fold<RHO>(s, trec, f);
     } else {
         finish_fp64_part<RHO>(s, f);
-        for (; i < nfd; i += SPLIT)
+        for (; i < nfd; i += step)
             walk(i, [&](auto&& step_mask, const double2* recs) {
                 float Lf[20];
 #pragma unroll
@@ -827,18 +845,23 @@ __device__ void m2l_item_direct(const LevelArgs& a, int slot, int flags, const i
     if constexpr (SPLIT > 1) {
         // no refill is in flight and every read of the image is done, so the
         // image can hold this wave's 64 x kParts partial sums (at most 11.5 KiB)
-        double* part = reinterpret_cast<double*>(stage) + (threadIdx.x & 63) * kParts;
-        if (q0 != 0) {
+        double* mine = reinterpret_cast<double*>(stage) + (threadIdx.x & 63) * kParts;
+        if (sl != 0) {
 #pragma unroll
-            for (int i = 0; i < kParts; ++i) part[i] = f[i];
+            for (int i = 0; i < kParts; ++i) mine[i] = f[i];
         }
         __syncthreads();
-        if (q0 != 0) return;
+        if (sl != 0) return;
         for (int o = 1; o < SPLIT; ++o) {
             const double* po = reinterpret_cast<const double*>(s_stage + o * kDirWave) + (threadIdx.x & 63) * kParts;
 #pragma unroll
             for (int i = 0; i < kParts; ++i) f[i] += po[i];
         }
+    }
+    if constexpr (WIDE) {
+#pragma unroll
+        for (int c = 0; c < kFolded; ++c) sums[c * 64 + (threadIdx.x & 63)] = f[c];
+        return;
     }
     // The lane's geometry again, from an opaque copy of the thread index: the
     // far loop needs none of it, and formed here it is not held in registers
@@ -1474,12 +1497,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3)))
     const int item = v / kParts;
     const int w = (v % kParts) * WAVES + (threadIdx.x >> 6);
     const int2 it = a.items[a.item0 + item];
-    if (threadIdx.x < 27) {
-        const int n = a.nbr[(size_t)it.x * 27 + threadIdx.x];
-        s_nbr[threadIdx.x] = n;
-        s_kind[threadIdx.x] = n >= 0 ? a.kind[n] : -1;
-    }
-    __syncthreads();
+    if (it.y & kItemNear) near_tables(a, it.x, s_nbr, s_kind);   // uniform per workgroup
     if (it.y & kItemLeaf) return;
     m2l_item_direct<RHO>(a, it.x, it.y, s_nbr, s_kind, w, s_stage);
 }
@@ -1494,14 +1512,66 @@ __global__ __launch_bounds__(64 * SPLIT) __attribute__((amdgpu_waves_per_eu(3)))
     const int v = xcd_item(blockIdx.x, gridDim.x);
     const int item = v >> 3, w = v & 7;
     const int2 it = a.items[a.item0 + item];
-    if (threadIdx.x < 27) {
-        const int n = a.nbr[(size_t)it.x * 27 + threadIdx.x];
-        s_nbr[threadIdx.x] = n;
-        s_kind[threadIdx.x] = n >= 0 ? a.kind[n] : -1;
-    }
-    __syncthreads();
+    if (it.y & kItemNear) near_tables(a, it.x, s_nbr, s_kind);   // uniform per workgroup
     if (it.y & kItemLeaf) return;   // uniform per workgroup
     m2l_item_direct<RHO, SPLIT, MIXED>(a, it.x, it.y, s_nbr, s_kind, w, s_stage, (int)(threadIdx.x >> 6));
+}
+
+// Variant 704 on levels with few sub-grids: each 2x2x2 coarse block's entries
+// over a.parts workgroups of 4 waves, whose folded sums meet in level_reduce.
+// In the plain form a level of n targets has 8 n workgroups, whose waves each
+// walk 6 or 7 images one after another (~3 us an image alone on a SIMD): below
+// one workgroup per CU the rest of the chip stands idle meanwhile.  Measured
+// (theta 0.5 / 0.34): 1 target 25.3 / 74.6 -> 10.7 / 15.1 us, 8 targets 26.0 /
+// 75.2 -> 16.5 / 29.3 us, 18 targets 26.4 / 76.2 -> 21.5 / 47.3 us.
+template <bool RHO>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void level_kernel_wide(LevelArgs a) {
+    __shared__ int s_nbr[27];
+    __shared__ int s_kind[27];
+    __shared__ double2 s_stage[4 * kDirWave];
+    const int v = xcd_item(blockIdx.x, gridDim.x);
+    const int block = v / a.parts, part = v - block * a.parts;
+    const int2 it = a.items[a.item0 + (block >> 3)];
+    if (it.y & kItemNear) near_tables(a, it.x, s_nbr, s_kind);   // uniform per workgroup
+    m2l_item_direct<RHO, 4, false, true>(a, it.x, it.y, s_nbr, s_kind, block & 7, s_stage, (int)(threadIdx.x >> 6), part,
+        a.wide_sums + (size_t)v * (kFolded * 64));
+}
+
+// Sums the parts of one coarse block of a target (one wave, lane = cell) in
+// part order and writes the cells' results.
+template <bool RHO>
+__global__ __launch_bounds__(64) void level_reduce(LevelArgs a) {
+    const int block = blockIdx.x;
+    const int slot = a.items[a.item0 + (block >> 3)].x;
+    const double* src = a.wide_sums + (size_t)block * a.parts * (kFolded * 64) + threadIdx.x;
+    double f[kFolded], L[20], C[3];
+#pragma unroll
+    for (int c = 0; c < kFolded; ++c) f[c] = src[c * 64];
+    for (int p = 1; p < a.parts; ++p) {
+        src += kFolded * 64;
+#pragma unroll
+        for (int c = 0; c < kFolded; ++c) f[c] += src[c * 64];
+    }
+    acc_finish<RHO>(f, L, C);
+    finish_cell<RHO>(a, slot, lane_geom(block & 7).cell, L, 20, C, true, false);
+}
+
+// Workgroups per coarse block of variant 704 on a level of n targets (0: the
+// plain form).  The sums' way through memory and the second kernel cost ~5 us,
+// about what two images take: with the 26 images of theta 0.5 the split pays
+// up to 1.75 workgroups per CU (27 targets: 26.3 us plain, 27.3 in two parts),
+// with the 92 of theta 0.34 up to three (36 targets: 109 -> 89 us, 45: 111 ->
+// 94 us, 64 in two parts: 122 -> 125 us).  At most one image per wave.
+int wide_parts(int n, const Tables& tab) {
+    if (n <= 0) return 0;
+    const int parts = std::min((tab.nsched + 3) / 4, (tab.nsched < 48 ? 448 : 768) / (8 * n));
+    return parts >= 2 ? parts : 0;
+}
+
+template <bool RHO>
+void launch_wide(int nitems, hipStream_t st, const LevelArgs& la) {
+    hipLaunchKernelGGL(level_kernel_wide<RHO>, dim3(nitems * 8 * la.parts), dim3(256), 0, st, la);
+    hipLaunchKernelGGL(level_reduce<RHO>, dim3(nitems * 8), dim3(64), 0, st, la);
 }
 
 // Persistent form of the mapping-7 kernel (variants 804, 802): a grid of
@@ -1597,7 +1667,10 @@ void launch_level(int variant, int nitems, hipStream_t st, const LevelArgs& la, 
         hipLaunchKernelGGL((level_kernel_split<RHO, 4>), dim3(nitems * 8), dim3(256), 0, st, la);
         break;
     case 704:
-        hipLaunchKernelGGL((level_kernel_dsplit<RHO, 4>), dim3(nitems * 8), dim3(256), 0, st, la);
+        if (la.parts > 1)
+            launch_wide<RHO>(nitems, st, la);
+        else
+            hipLaunchKernelGGL((level_kernel_dsplit<RHO, 4>), dim3(nitems * 8), dim3(256), 0, st, la);
         break;
     case 702:
         hipLaunchKernelGGL((level_kernel_dsplit<RHO, 2>), dim3(nitems * 8), dim3(128), 0, st, la);
@@ -2052,6 +2125,8 @@ struct octofmm_plan {
     int32_t* d_mixorder = nullptr;
     int32_t mix_n64 = 0;
     uint32_t* d_queue = nullptr;   // per-XCD work counters of the persistent variants
+    int32_t wide_parts = 0;        // variant 704 split further: workgroups per coarse block (0: not for this level)
+    double* d_wide = nullptr;      // and their folded sums [n_m2l * 8 * wide_parts][kFolded][64]
     int32_t n_p2m = 0;             // leaf items with p2m: items [n_m2l, n_m2l + n_p2m)
     double* d_p2m_out = nullptr;   // their p2m sums [n_p2m][512][8]
     int64_t mixed_far_pairs_by_offset = 0;   // FP32 far pairs under that rule
@@ -2318,6 +2393,8 @@ static octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace&
         la.mixorder = nullptr;
         la.mix_n64 = 0;
         la.queue = nullptr;
+        la.parts = 0;
+        la.wide_sums = nullptr;
         la.mon = w.mon;
         la.p2m_out = w.p2m;
         la.parent = nullptr;
@@ -2537,6 +2614,7 @@ static void plan_free(octofmm_plan* p) {
     (void)hipFree(p->d_recm);
     (void)hipFree(p->d_mixorder);
     (void)hipFree(p->d_queue);
+    (void)hipFree(p->d_wide);
     (void)hipFree(p->d_p2m_out);
     (void)hipFree(p->d_partial);
     (void)hipFree(p->d_pslots);
@@ -2613,6 +2691,8 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         la.mixorder = p->d_mixorder;
         la.mix_n64 = p->mix_n64;
         la.queue = p->d_queue;
+        la.parts = p->wide_parts;
+        la.wide_sums = p->d_wide;
         la.mon = p->d_mon;
         la.p2m_out = p->d_p2m_out;
         la.parent = p->t_parent;
@@ -3083,6 +3163,10 @@ static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* 
         return cleanup(OCTOFMM_ERR_ALLOCATION, "root partial buffer allocation failed");
     if (!root && hipMalloc((void**)&p->d_queue, sizeof(uint32_t) * 8) != hipSuccess)
         return cleanup(OCTOFMM_ERR_ALLOCATION, "work counter allocation failed");
+    if (!root && p->precision == OCTOFMM_PRECISION_FP64) p->wide_parts = wide_parts(n_m2l, T);
+    if (p->wide_parts > 0 &&
+        hipMalloc((void**)&p->d_wide, sizeof(double) * (size_t)n_m2l * 8 * p->wide_parts * kFolded * 64) != hipSuccess)
+        return cleanup(OCTOFMM_ERR_ALLOCATION, "partial sum buffer allocation failed");
     p->n_p2m = (int32_t)buckets[2].size();
     if (p->n_p2m > 0 &&
         hipMalloc((void**)&p->d_p2m_out, sizeof(double) * (size_t)p->n_p2m * kCells * 8) != hipSuccess)

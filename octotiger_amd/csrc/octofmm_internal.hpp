@@ -118,7 +118,8 @@ struct Tables {
 //              waves (variant 504), for levels with few sub-grids.
 //   mapping 7: mapping 3's staging with the coarse offsets of a block split
 //              over 4, 2 or 8 waves (variants 704, 702, 708); the partial sums
-//              meet in the waves' images.  The 8-wave split (one workgroup per
+//              meet in the waves' images.  On small FP64 levels 704
+//              splits each block further over several workgroups (wide_parts).  The 8-wave split (one workgroup per
 //              CU by its LDS) is for levels with very few sub-grids.
 //   mapping 8: mapping 7 as one persistent grid over per-XCD work counters
 //              (variants 804, 802).

@@ -155,7 +155,7 @@ octofmm_status octofmm_compute_monopole_interactions(octofmm_context* ctx,
  * counterpart in the reference: it is for callers that cannot allocate device
  * memory (tight per-node loops, code that must not call hipMalloc).  Same
  * arguments, kernels, results (bit for bit) and synchronous behaviour; its
- * device workspace is a static array in the library's code object, 16 MiB per
+ * device workspace is a static array in the library's code object, 12 MiB per
  * GPU, held from the first octofmm_create on that GPU until the process
  * ends.  The maximum is one call's inputs: a sub-grid and its 26 neighbours,
  * each of at most 512 cells (larger counts are rejected with

@@ -659,6 +659,7 @@ struct LevelArgs {
     double G;
     int32_t l2l;
     int32_t correct_am;
+    int32_t overwrite;      // outside whole-tree solves: L is written, not accumulated
     int32_t leaf_rows;      // whole-tree solves: 0 = leaf cells get g (and L_c) only, no L rows
     // persistent form of lane mapping 7: 8 work counters, one per XCD
     // (cleared by queue_reset before each launch)

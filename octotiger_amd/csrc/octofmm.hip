@@ -70,6 +70,92 @@ __device__ __forceinline__ void store_stream(double2* p, double2 v) {
 // where a lane per record spread every instruction over 64 rows.
 constexpr int kStageRow = 25;
 
+// Every branch that fills a half record sets all 12 fields in this order: with
+// fields set one by one the compiler merges the branches' last stores into one
+// of a varying index, which puts the array into scratch memory.
+__device__ __forceinline__ void set12(double* v, double a, double b, double c, double d, double e, double f, double g,
+    double h, double i, double j, double k, double l) {
+    v[0] = a;
+    v[1] = b;
+    v[2] = c;
+    v[3] = d;
+    v[4] = e;
+    v[5] = f;
+    v[6] = g;
+    v[7] = h;
+    v[8] = i;
+    v[9] = j;
+    v[10] = k;
+    v[11] = l;
+}
+
+// One half of a cell's record fields from its row (M 20, com 3): the mass,
+// dipole, quadrupole and centre (fields 0..8 and 21..23) or the octupole
+// (fields 9..20).
+__device__ __forceinline__ void record_half(const double* row, bool octupole, bool rho, double* v) {
+    if (!octupole) {
+        const double m4 = row[4], m7 = row[7], tr = (m4 + m7 + row[9]) * (1.0 / 3.0);
+        set12(v, row[0], 1.25 * row[1], 1.25 * row[2], 1.25 * row[3], (15.0 / 32.0) * (m4 - tr), (15.0 / 32.0) * row[5],
+            (15.0 / 32.0) * row[6], (15.0 / 32.0) * (m7 - tr), (15.0 / 32.0) * row[8], row[20], row[21], row[22]);
+    } else {
+        double m[10];
+#pragma unroll
+        for (int i = 0; i < 10; ++i) m[i] = (5.0 / 64.0) * row[10 + i];
+        const double tx = m[0] + m[3] + m[5], ty = m[1] + m[6] + m[8], tz = m[2] + m[7] + m[9];
+        const double xxx = m[0] - 0.6 * tx, xyy = m[3] - 0.2 * tx, xzz = m[5] - 0.2 * tx;
+        const double xxy = m[1] - 0.2 * ty, yyy = m[6] - 0.6 * ty, yzz = m[8] - 0.2 * ty;
+        const double xxz = m[2] - 0.2 * tz, yyz = m[7] - 0.2 * tz, xyz = m[4];
+        // DRHODT: coefficients of the cubic monomials
+        if (rho)
+            set12(v, xxx, xyy, xzz, xxy, yyy, yzz, xxz, yyz, xyz, 0.7 * tx, 0.7 * ty, 0.7 * tz);
+        else
+            set12(v, 0.5 * xxx, 1.5 * xyy, 1.5 * xxy, 0.5 * yyy, 1.5 * xxz, 1.5 * yyz, xxz + yyz, 3.0 * xyz, 0.0, 0.0, 0.0, 0.0);
+    }
+}
+
+// The first half's fields of a leaf cell: a monopole at the geometric cell
+// centre in the target's frame (multipole_interaction_interface.hpp:216-235),
+// rounded operation by operation as the reference does.
+__device__ __forceinline__ void record_leaf(double m, int x, int y, int z, const int* off, const double* base, double dx,
+    double* v) {
+#pragma clang fp contract(off)
+    set12(v, m, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, (double)(x + off[0]) * dx + base[0] - kInx * dx,
+        (double)(y + off[1]) * dx + base[1] - kInx * dx, (double)(z + off[2]) * dx + base[2] - kInx * dx);
+}
+
+__device__ __forceinline__ void write_half(double* row, bool octupole, const double* v) {
+    if (!octupole) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) row[i] = v[i];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) row[kRecY + i] = v[9 + i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 12; ++i) row[9 + i] = v[i];
+    }
+}
+
+// Loads n cells' M and centre rows (contiguous, M 16-byte aligned) into LDS rows.
+__device__ __forceinline__ void load_rows(const double* M, const double* com, int n, double* s_row) {
+    const int t = threadIdx.x;
+    const double2* srcM = reinterpret_cast<const double2*>(M);
+#pragma unroll
+    for (int r = 0; r < 5; ++r) {
+        const int i = t + 256 * r;
+        if (i < n * 10) {
+            const double2 m = srcM[i];
+            double* d = s_row + (i / 10) * kStageRow + 2 * (i % 10);
+            d[0] = m.x;
+            d[1] = m.y;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int i = t + 256 * r;
+        if (i < n * 3) s_row[(i / 3) * kStageRow + 20 + i % 3] = com[i];
+    }
+}
+
 __global__ __launch_bounds__(256) void stage_records(StageArgs a) {
     __shared__ double s_row[128 * kStageRow];
     const int si = blockIdx.x >> 2, q = blockIdx.x & 3;
@@ -84,90 +170,26 @@ __global__ __launch_bounds__(256) void stage_records(StageArgs a) {
     double* row = s_row + cl * kStageRow;
     double v[12];                              // this half's record fields
     float f32[10];                             // and its FP32 moments (mixed precision)
-#pragma unroll
-    for (int i = 0; i < 12; ++i) v[i] = 0.0;
     if (k == OCTOFMM_SLOT_NONLEAF) {
-        const double2* srcM = reinterpret_cast<const double2*>(a.M + row0 * 20);
-#pragma unroll
-        for (int r = 0; r < 5; ++r) {
-            const int i = t + 256 * r;
-            const double2 m = srcM[i];
-            double* d = s_row + (i / 10) * kStageRow + 2 * (i % 10);
-            d[0] = m.x;
-            d[1] = m.y;
-        }
-        const double* srcC = a.com + row0 * 3;
-        for (int i = t; i < 128 * 3; i += 256) s_row[(i / 3) * kStageRow + 20 + i % 3] = srcC[i];
+        load_rows(a.M + row0 * 20, a.com + row0 * 3, 128, s_row);
         __syncthreads();
-        if (!octupole) {
-            // fields 0..8 and the centre (v[9..11])
-            const double m4 = row[4], m7 = row[7], tr = (m4 + m7 + row[9]) * (1.0 / 3.0);
-            v[0] = row[0];
-#pragma unroll
-            for (int i = 1; i < 4; ++i) v[i] = 1.25 * row[i];
-            v[4] = (15.0 / 32.0) * (m4 - tr);
-            v[5] = (15.0 / 32.0) * row[5];
-            v[6] = (15.0 / 32.0) * row[6];
-            v[7] = (15.0 / 32.0) * (m7 - tr);
-            v[8] = (15.0 / 32.0) * row[8];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) v[9 + i] = row[20 + i];
-        } else {
-            // fields 9..20
-            double m[10];
-#pragma unroll
-            for (int i = 0; i < 10; ++i) m[i] = (5.0 / 64.0) * row[10 + i];
-            const double tx = m[0] + m[3] + m[5], ty = m[1] + m[6] + m[8], tz = m[2] + m[7] + m[9];
-            const double xxx = m[0] - 0.6 * tx, xyy = m[3] - 0.2 * tx, xzz = m[5] - 0.2 * tx;
-            const double xxy = m[1] - 0.2 * ty, yyy = m[6] - 0.6 * ty, yzz = m[8] - 0.2 * ty;
-            const double xxz = m[2] - 0.2 * tz, yyz = m[7] - 0.2 * tz, xyz = m[4];
-            if (a.rho) {
-                v[0] = xxx;
-                v[1] = xyy;
-                v[2] = xzz;
-                v[3] = xxy;
-                v[4] = yyy;
-                v[5] = yzz;
-                v[6] = xxz;
-                v[7] = yyz;
-                v[8] = xyz;
-                v[9] = 0.7 * tx;
-                v[10] = 0.7 * ty;
-                v[11] = 0.7 * tz;
-            } else {
-                // coefficients of the cubic monomials
-                v[0] = 0.5 * xxx;
-                v[1] = 1.5 * xyy;
-                v[2] = 1.5 * xxy;
-                v[3] = 0.5 * yyy;
-                v[4] = 1.5 * xxz;
-                v[5] = 1.5 * yyz;
-                v[6] = xxz + yyz;
-                v[7] = 3.0 * xyz;
-            }
-        }
+        record_half(row, octupole, a.rho != 0, v);
         if (a.recm) {
 #pragma unroll
             for (int i = 0; i < 10; ++i)
                 f32[i] = (float)(row[10 * octupole + i] * (octupole ? record_scale(10 + i) : record_scale(i)));
         }
     } else {
+        const bool leaf = k == OCTOFMM_SLOT_LEAF && !octupole;
+        const int cell = c0 + cl;
+        if (leaf)
+            record_leaf(a.mon[row0 + cl], cell >> 6, (cell >> 3) & 7, cell & 7, a.foff + 3 * slot, a.fxbase + 3 * slot,
+                a.dx, v);
+        else
+            set12(v, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0);
 #pragma unroll
-        for (int i = 0; i < 10; ++i) f32[i] = 0.0f;
-        if (k == OCTOFMM_SLOT_LEAF && !octupole) {
-            // a monopole at the geometric cell centre in the target's frame
-            // (multipole_interaction_interface.hpp:216-235), rounded operation
-            // by operation as the reference does
-#pragma clang fp contract(off)
-            const int cell = c0 + cl;
-            const int* fo = a.foff + 3 * slot;
-            const double* fb = a.fxbase + 3 * slot;
-            v[0] = a.mon[row0 + cl];
-            f32[0] = (float)v[0];
-            v[9] = (double)((cell >> 6) + fo[0]) * a.dx + fb[0] - kInx * a.dx;
-            v[10] = (double)(((cell >> 3) & 7) + fo[1]) * a.dx + fb[1] - kInx * a.dx;
-            v[11] = (double)((cell & 7) + fo[2]) * a.dx + fb[2] - kInx * a.dx;
-        }
+        for (int i = 1; i < 10; ++i) f32[i] = 0.0f;
+        f32[0] = leaf ? (float)v[0] : 0.0f;
     }
     // the row of the block's r-th record: coarse cell r >> 3 of the layer,
     // child r & 7
@@ -184,15 +206,7 @@ __global__ __launch_bounds__(256) void stage_records(StageArgs a) {
         }
     };
     __syncthreads();   // every row read before its record overwrites it
-    if (!octupole) {
-#pragma unroll
-        for (int i = 0; i < 9; ++i) row[i] = v[i];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) row[kRecY + i] = v[9 + i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < 12; ++i) row[9 + i] = v[i];
-    }
+    write_half(row, octupole, v);
     __syncthreads();
     out(a.rec);
     if (a.recm) {   // uniform: the mixed-precision records of the same cells
@@ -219,6 +233,97 @@ __global__ __launch_bounds__(256) void stage_records(StageArgs a) {
         }
         __syncthreads();
         out(a.recm);
+    }
+}
+
+// Staging of the per-sub-grid entry points.  The host packs the sub-grid and
+// the cells of its neighbours within the stencil's reach (12^3 cells at theta
+// 0.5, a ninth of the 27 sub-grids) into pinned memory, which this kernel reads
+// where it lies: one pass over PCIe in coalesced rows, with no device copy in
+// between.  It writes the records the interaction kernels read, the monopoles
+// and (leaf targets) the centres, and the one-target level's tables.  Slot 0 is
+// the target, the neighbour in raw direction d is slot packed_slot(d); packed
+// cells run over the neighbour's box, x slowest.
+__host__ __device__ __forceinline__ int packed_slot(int raw) { return raw == 13 ? 0 : raw < 13 ? raw + 1 : raw; }
+__host__ __device__ __forceinline__ int packed_raw(int slot) { return slot == 0 ? 13 : slot <= 13 ? slot - 1 : slot; }
+
+// First cell and extent along one axis of the cells a neighbour hands over,
+// d = -1, 0, 1 its direction.
+__host__ __device__ __forceinline__ void packed_box(int d, int reach, int& lo, int& n) {
+    lo = d < 0 ? kInx - reach : 0;
+    n = d == 0 ? kInx : reach;
+}
+
+struct PackedArgs {
+    const double* src;      // pinned host memory: per slot M [n][20], com [n][3] (refined), mon [n] (leaf);
+                            // a leaf target's com [512][3] after its mon
+    int32_t off[27];        // first double of each slot
+    int32_t kind[27];       // octofmm_slot_kind, or -1: absent
+    int32_t reach;
+    int32_t rho;
+    int32_t leaf_target;
+    int32_t item_flags;
+    double xbase[3];
+    double dx;
+    double* rec;            // [27][512][24]
+    double* mon;            // [27][512]
+    double* com;            // [512][3] a leaf target's centres
+    int32_t* meta;          // items[2] nbr[27] kind[27]
+};
+
+__global__ __launch_bounds__(256) void stage_packed(PackedArgs a) {
+    __shared__ double s_row[128 * kStageRow];
+    const int slot = blockIdx.x >> 2, c0 = (blockIdx.x & 3) * 128;
+    const int t = threadIdx.x;
+    if (blockIdx.x == 0 && t < 27) {
+        if (t < 2) a.meta[t] = t == 0 ? 0 : a.item_flags;
+        a.meta[2 + t] = a.kind[packed_slot(t)] >= 0 ? packed_slot(t) : -1;
+        a.meta[29 + t] = a.kind[t];
+    }
+    const int k = a.kind[slot], raw = packed_raw(slot);
+    int lo[3], n[3];
+    packed_box(raw % 3 - 1, a.reach, lo[0], n[0]);
+    packed_box(raw / 3 % 3 - 1, a.reach, lo[1], n[1]);
+    packed_box(raw / 9 - 1, a.reach, lo[2], n[2]);
+    const int ncell = n[0] * n[1] * n[2], cnt = ncell - c0 < 128 ? ncell - c0 : 128;
+    if (k < 0 || cnt <= 0) return;             // uniform per block
+    const double* src = a.src + a.off[slot];
+    auto cell_of = [&](int i, int& x, int& y, int& z) {
+        x = lo[0] + i / (n[1] * n[2]);
+        y = lo[1] + i / n[2] % n[1];
+        z = lo[2] + i % n[2];
+    };
+    const int cl = t & 127, octupole = t >> 7;
+    double* row = s_row + cl * kStageRow;
+    double v[12];
+    if (k == OCTOFMM_SLOT_NONLEAF) {
+        load_rows(src + (size_t)c0 * 20, src + (size_t)ncell * 20 + (size_t)c0 * 3, cnt, s_row);
+        __syncthreads();
+        record_half(row, octupole, a.rho != 0, v);   // (rows past cnt: unused)
+    } else if (cl < cnt && !octupole) {
+        int x, y, z;
+        cell_of(c0 + cl, x, y, z);
+        const int off[3] = {kInx + kInx * (raw % 3 - 1), kInx + kInx * (raw / 3 % 3 - 1), kInx + kInx * (raw / 9 - 1)};
+        record_leaf(src[c0 + cl], x, y, z, off, a.xbase, a.dx, v);
+        const int cell = x * 64 + y * 8 + z;
+        a.mon[(size_t)slot * kCells + cell] = v[0];
+        if (a.leaf_target && slot == 0) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) a.com[cell * 3 + d] = src[kCells + cell * 3 + d];
+        }
+    } else {
+        set12(v, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0);
+    }
+    __syncthreads();
+    if (cl < cnt) write_half(row, octupole, v);
+    __syncthreads();
+    for (int ch = t; ch < cnt * 12; ch += 256) {
+        const int r = ch / 12, part = ch % 12;
+        int x, y, z;
+        cell_of(c0 + r, x, y, z);
+        const double* from = s_row + r * kStageRow + 2 * part;
+        reinterpret_cast<double2*>(a.rec + ((size_t)slot * kCells + record_of_cell(x, y, z)) * kRecDoubles)[part] =
+            make_double2(from[0], from[1]);
     }
 }
 
@@ -326,7 +431,7 @@ __device__ __forceinline__ void finish_cell(const LevelArgs& a, int slot, int ce
     double* Co = a.Lc + ((size_t)slot * kCells + cell) * 3;
     if (!a.l2l) {
         for (int i = 0; i < ncomp / 2; ++i) {
-            double2 v = Lo[i];
+            double2 v = a.overwrite ? make_double2(0.0, 0.0) : Lo[i];
             v.x += L[2 * i];
             v.y += L[2 * i + 1];
             Lo[i] = v;
@@ -1764,60 +1869,14 @@ __global__ void zero_fill(double* p, size_t n) {
     if (i < n) p[i] = 0.0;
 }
 
-// Partial halos of the per-sub-grid entry points: a neighbour that hands over
-// only some of its cells (grid::get_ilist_n_bnd order,
+// Partial halo slots of a level plan (octofmm_partial_slot): a neighbour that
+// hands over only some of its cells (grid::get_ilist_n_bnd order,
 // multipole_interaction_interface.hpp:177,257, p2m_interaction_interface.hpp:142,239)
 // becomes a full slot with zeros in every cell it did not hand over, which is
-// what update_input's zero padding gives.  One block per such neighbour: it
-// zeroes the slot, then writes each listed cell from its position in the
-// handed-over arrays.  The host lists each cell once (its last occurrence),
-// so no two threads write one cell.
-struct ScatterArgs {
-    const double* cM;       // [26][512][20] handed-over multipoles, by partial direction q
-    const double* ccom;     // [26][512][3]
-    const double* cmon;     // [26][512]
-    const int2* cidx;       // [26][512] (cell, position)
-    double* M;              // [27][512][20] slots
-    double* com;            // [27][512][3]
-    double* mon;            // [27][512]
-    int32_t slot[26];       // slot of partial direction q
-    int32_t count[26];      // listed cells of q
-    int32_t multipole[26];  // 1: multipoles and centres of mass, 0: monopoles
-};
-
-__global__ __launch_bounds__(256) void scatter_partial(ScatterArgs a) {
-    const int q = blockIdx.x, t = threadIdx.x;
-    const int s = a.slot[q], n = a.count[q];
-    const bool mp = a.multipole[q] != 0;
-    double* M = a.M + (size_t)s * kCells * 20;
-    double* C = a.com + (size_t)s * kCells * 3;
-    double* m = a.mon + (size_t)s * kCells;
-    if (mp) {
-        for (int i = t; i < kCells * 20; i += 256) M[i] = 0.0;
-        for (int i = t; i < kCells * 3; i += 256) C[i] = 0.0;
-    } else {
-        for (int i = t; i < kCells; i += 256) m[i] = 0.0;
-    }
-    __syncthreads();
-    const int2* idx = a.cidx + (size_t)q * kCells;
-    for (int i = t; i < n; i += 256) {
-        const int2 e = idx[i];
-        if (mp) {
-            const double* src = a.cM + ((size_t)q * kCells + e.y) * 20;
-#pragma unroll
-            for (int c = 0; c < 20; ++c) M[e.x * 20 + c] = src[c];
-            const double* sc = a.ccom + ((size_t)q * kCells + e.y) * 3;
-            C[e.x * 3] = sc[0];
-            C[e.x * 3 + 1] = sc[1];
-            C[e.x * 3 + 2] = sc[2];
-        } else {
-            m[e.x] = a.cmon[(size_t)q * kCells + e.y];
-        }
-    }
-}
-
-// Partial halo slots of a level plan (octofmm_partial_slot): the same scatter
-// as scatter_partial, one block per slot, from descriptors in device memory.
+// what update_input's zero padding gives.  One block per such slot, from
+// descriptors in device memory: it zeroes the slot, then writes each listed
+// cell from its position in the handed-over arrays.  The host lists each cell
+// once (its last occurrence), so no two threads write one cell.
 struct PartialSlot {
     const double* M;        // [count][20] handed-over multipoles (non-leaf slot)
     const double* com;      // [count][3]
@@ -1984,71 +2043,52 @@ constexpr size_t kRecTailBytes = 4096;
 // item comes first so it stays 8-byte aligned
 constexpr int kMetaItems = 0;
 constexpr int kMetaNbr = 2;
-constexpr int kMetaKind = kMetaNbr + 27 * 27;
-constexpr int kMetaFoff = kMetaKind + 27;
-constexpr int kMetaSize = kMetaFoff + 81;
+constexpr int kMetaKind = kMetaNbr + 27;
+constexpr int kMetaSize = kMetaKind + 27;
 
-// Device workspace of the per-sub-grid entry points: a 27-slot level (slot =
-// raw direction index, 13 = the target sub-grid), the neighbour data as the
-// caller hands it over, and the root kernel's chunk sums.  Every region starts
-// on a 256-byte boundary of one block.
+// Most workgroups per coarse block of a one-target level (wide_parts)
+constexpr int kWideMax = (kMaxDelta + 3) / 4;
+
+// Device workspace of the per-sub-grid entry points: a 27-slot level (slot 0 the
+// target sub-grid, packed_slot(d) its neighbour in direction d), the partial
+// sums of the interaction kernels and the root kernel's chunk sums.  Every
+// region starts on a 256-byte boundary of one block.
 struct SubgridWorkspace {
-    double* M = nullptr;        // [27][512][20]
-    double* com = nullptr;      // [27][512][3]
-    double* mon = nullptr;      // [27][512]
     double* rec = nullptr;      // [27][512][24] + tail
-    double* L = nullptr;        // [27][512][20]: slot 13 holds the target's L
-    double* Lc = nullptr;       // [27][512][3]
+    double* mon = nullptr;      // [27][512]
+    double* com = nullptr;      // [512][3] a leaf target's centres
+    double* wide = nullptr;     // [8][kWideMax][kFolded][64]
     double* partial = nullptr;  // [kRootChunks][512][24]
-    double* cM = nullptr;       // [26][512][20] partial halos as handed over, by partial direction
-    double* ccom = nullptr;     // [26][512][3]
-    double* cmon = nullptr;     // [26][512]
-    int2* cidx = nullptr;       // [26][512] (cell, position in the handed-over arrays)
-    int32_t* meta = nullptr;    // kMetaSize
-    double* fx = nullptr;       // [27][3]
     double* p2m = nullptr;      // [512][8] p2m sums of a leaf target
+    int32_t* meta = nullptr;    // kMetaSize
 };
 
 constexpr size_t ws_align(size_t n) { return (n + 255) & ~size_t(255); }
-constexpr size_t kWsM = 0;
-constexpr size_t kWsCom = kWsM + ws_align(sizeof(double) * 27 * kCells * 20);
-constexpr size_t kWsMon = kWsCom + ws_align(sizeof(double) * 27 * kCells * 3);
-constexpr size_t kWsRec = kWsMon + ws_align(sizeof(double) * 27 * kCells);
-constexpr size_t kWsL = kWsRec + ws_align(sizeof(double) * 27 * kCells * kRecDoubles + kRecTailBytes);
-constexpr size_t kWsLc = kWsL + ws_align(sizeof(double) * 27 * kCells * 20);
-constexpr size_t kWsPartial = kWsLc + ws_align(sizeof(double) * 27 * kCells * 3);
-constexpr size_t kWsCM = kWsPartial + ws_align(sizeof(double) * kRootChunks * kCells * kRecDoubles);
-constexpr size_t kWsCCom = kWsCM + ws_align(sizeof(double) * 26 * kCells * 20);
-constexpr size_t kWsCMon = kWsCCom + ws_align(sizeof(double) * 26 * kCells * 3);
-constexpr size_t kWsCIdx = kWsCMon + ws_align(sizeof(double) * 26 * kCells);
-constexpr size_t kWsMeta = kWsCIdx + ws_align(sizeof(int2) * 26 * kCells);
-constexpr size_t kWsFx = kWsMeta + ws_align(sizeof(int32_t) * kMetaSize);
-constexpr size_t kWsP2m = kWsFx + ws_align(sizeof(double) * 81);
-constexpr size_t kWsBytes = kWsP2m + ws_align(sizeof(double) * kCells * 8);
+constexpr size_t kWsRec = 0;
+constexpr size_t kWsMon = kWsRec + ws_align(sizeof(double) * 27 * kCells * kRecDoubles + kRecTailBytes);
+constexpr size_t kWsCom = kWsMon + ws_align(sizeof(double) * 27 * kCells);
+constexpr size_t kWsWide = kWsCom + ws_align(sizeof(double) * kCells * 3);
+constexpr size_t kWsPartial = kWsWide + ws_align(sizeof(double) * 8 * kWideMax * kFolded * 64);
+constexpr size_t kWsP2m = kWsPartial + ws_align(sizeof(double) * kRootChunks * kCells * kRecDoubles);
+constexpr size_t kWsMeta = kWsP2m + ws_align(sizeof(double) * kCells * 8);
+constexpr size_t kWsBytes = kWsMeta + ws_align(sizeof(int32_t) * kMetaSize);
 
 SubgridWorkspace carve_workspace(char* base) {
     SubgridWorkspace w;
-    w.M = reinterpret_cast<double*>(base + kWsM);
-    w.com = reinterpret_cast<double*>(base + kWsCom);
-    w.mon = reinterpret_cast<double*>(base + kWsMon);
     w.rec = reinterpret_cast<double*>(base + kWsRec);
-    w.L = reinterpret_cast<double*>(base + kWsL);
-    w.Lc = reinterpret_cast<double*>(base + kWsLc);
+    w.mon = reinterpret_cast<double*>(base + kWsMon);
+    w.com = reinterpret_cast<double*>(base + kWsCom);
+    w.wide = reinterpret_cast<double*>(base + kWsWide);
     w.partial = reinterpret_cast<double*>(base + kWsPartial);
-    w.cM = reinterpret_cast<double*>(base + kWsCM);
-    w.ccom = reinterpret_cast<double*>(base + kWsCCom);
-    w.cmon = reinterpret_cast<double*>(base + kWsCMon);
-    w.cidx = reinterpret_cast<int2*>(base + kWsCIdx);
-    w.meta = reinterpret_cast<int32_t*>(base + kWsMeta);
-    w.fx = reinterpret_cast<double*>(base + kWsFx);
     w.p2m = reinterpret_cast<double*>(base + kWsP2m);
+    w.meta = reinterpret_cast<int32_t*>(base + kWsMeta);
     return w;
 }
 
 }   // namespace
 
 // Workspace of octofmm_compute_multipole_interactions_noalloc: one per-sub-grid
-// workspace (kWsBytes, 16.0 MiB) in the code object's device memory, so that
+// workspace (kWsBytes, 12 MiB) in the code object's device memory, so that
 // entry point never allocates.  Each GPU the library runs on holds its own
 // copy until the process ends.  In host code `scratch` names a host-side
 // stand-in, not a device address: host code uses only the address
@@ -2086,14 +2126,23 @@ struct octofmm_context {
     hipStream_t stream = nullptr;
     std::string err;
     // per-sub-grid entry points: the device workspace (one allocation on the
-    // first call) and the host-side metadata they upload, built at creation
+    // first call) and the pinned memory, made at creation, that a call packs
+    // its inputs into and gets its results from (the kernels read and write it
+    // where it lies)
     SubgridWorkspace ws;
     char* d_ws = nullptr;
     char* d_scratch = nullptr;     // this device's `scratch` (set at creation)
-    int32_t* h_meta = nullptr;     // items[2] nbr[27*27] kind[27] foff[27*3]
-    double* h_fx = nullptr;        // [27][3]
-    int2* h_idx = nullptr;         // [26][512] (cell, position) of partial halos
+    double* h_pin = nullptr;       // results [512][20], [512][3], then the packed inputs
+    int reach = 0;                 // cells of a neighbour within the stencil's reach, per axis
 };
+
+// doubles of the results at the front of the pinned memory, and the cells its
+// packed inputs hold at most: the sub-grid and the halo within reach
+constexpr size_t kPinOut = (size_t)kCells * 23;
+static size_t pin_cells(const Tables& tab) {
+    const size_t w = kInx + 4 * (size_t)tab.max_delta;
+    return w * w * w;
+}
 
 struct octofmm_plan {
     octofmm_context* ctx = nullptr;
@@ -2227,139 +2276,104 @@ octofmm_status check_finite_inputs(octofmm_context* c, const octofmm_subgrid* in
     return OCTOFMM_OK;
 }
 
-// Loads one sub-grid descriptor into a workspace, on the context's stream:
-// the target's own arrays and every full neighbour are copied from the
-// caller's memory straight into their slots; a partial halo is copied as
-// handed over into its compact region and scatter_partial writes it into its
-// zeroed slot; then the 27-slot metadata.  Slots the metadata does not list
-// are never read, and staging reads only M and com of non-leaf slots and mon
-// of leaf slots, so nothing else needs clearing between calls.  The host
-// buffers read by the copies (c->h_meta, h_fx, h_idx) stay untouched until
-// the caller synchronises the stream.
-octofmm_status load_subgrid(octofmm_context* c, const SubgridWorkspace& w, const octofmm_subgrid* in,
-    bool leaf_target, bool root, int item_flags) {
-    hipStream_t st = c->stream;
-    int32_t* meta = c->h_meta;
-    int32_t* items = meta + kMetaItems;
-    int32_t* nbr = meta + kMetaNbr;  // only row 13 is used
-    int32_t* kind = meta + kMetaKind;
-    int32_t* foff = meta + kMetaFoff;
-    items[0] = 13;
-    items[1] = item_flags;
-    for (int i = 0; i < 27 * 27; ++i) nbr[i] = -1;
+// Packs one sub-grid descriptor into the context's pinned memory for
+// stage_packed: the target's own arrays whole, of each neighbour the cells
+// within the stencil's reach.  A partial halo contributes its listed cells
+// (later entries win, as in update_input's loop over the list) and zeros
+// elsewhere, which is what update_input's zero padding gives.
+void pack_subgrid(octofmm_context* c, const octofmm_subgrid* in, bool leaf_target, bool root, int item_flags,
+    PackedArgs& pa) {
+    double* dst = c->h_pin + kPinOut;
+    pa.src = dst;
+    pa.reach = c->reach;
+    pa.leaf_target = leaf_target ? 1 : 0;
+    pa.item_flags = item_flags;
+    pa.rho = in->type == OCTOFMM_RHO;
+    pa.dx = in->dx;
+    for (int k = 0; k < 3; ++k) pa.xbase[k] = in->xbase[k];
+    size_t at = 0;
     for (int sl = 0; sl < 27; ++sl) {
-        kind[sl] = -1;
-        const int d[3] = {sl % 3 - 1, (sl / 3) % 3 - 1, sl / 9 - 1};
-        for (int k = 0; k < 3; ++k) {
-            foff[3 * sl + k] = kInx + kInx * d[k];
-            c->h_fx[3 * sl + k] = in->xbase[k];
-        }
+        pa.off[sl] = 0;
+        pa.kind[sl] = -1;
     }
-    const size_t nM = (size_t)kCells * 20, nC = (size_t)kCells * 3;
     if (leaf_target) {
-        HIPC(c, hipMemcpyAsync(w.mon + 13 * kCells, in->mon, sizeof(double) * kCells, hipMemcpyHostToDevice, st));
-        HIPC(c, hipMemcpyAsync(w.com + 13 * nC, in->com, sizeof(double) * nC, hipMemcpyHostToDevice, st));
-        kind[13] = OCTOFMM_SLOT_LEAF;
+        pa.kind[0] = OCTOFMM_SLOT_LEAF;
+        std::memcpy(dst, in->mon, sizeof(double) * kCells);
+        std::memcpy(dst + kCells, in->com, sizeof(double) * kCells * 3);
+        at = (size_t)kCells * 4;
     } else {
-        HIPC(c, hipMemcpyAsync(w.M + 13 * nM, in->M, sizeof(double) * nM, hipMemcpyHostToDevice, st));
-        HIPC(c, hipMemcpyAsync(w.com + 13 * nC, in->com, sizeof(double) * nC, hipMemcpyHostToDevice, st));
-        kind[13] = OCTOFMM_SLOT_NONLEAF;
+        pa.kind[0] = OCTOFMM_SLOT_NONLEAF;
+        std::memcpy(dst, in->M, sizeof(double) * kCells * 20);
+        std::memcpy(dst + (size_t)kCells * 20, in->com, sizeof(double) * kCells * 3);
+        at = (size_t)kCells * 23;
     }
-    nbr[13 * 27 + 13] = 13;
-    ScatterArgs sa;
-    std::memset(&sa, 0, sizeof(sa));
-    int np = 0;
     for (int f = 0; f < (root ? 0 : 26); ++f) {
         const octofmm_neighbor& nb = in->neighbors[f];
-        const int sl = raw_of_flat(f);
+        const int raw = raw_of_flat(f), sl = packed_slot(raw);
         const bool multipole = nb.kind == OCTOFMM_NEIGHBOR_MULTIPOLE && nb.M && nb.com;
         const bool monopole = nb.kind == OCTOFMM_NEIGHBOR_MONOPOLE && nb.mon;
         if (!multipole && !monopole) continue;   // empty, or refined without data: the reference skips it
+        pa.kind[sl] = multipole ? OCTOFMM_SLOT_NONLEAF : OCTOFMM_SLOT_LEAF;
+        pa.off[sl] = (int32_t)at;
+        int lo[3], n[3];
+        packed_box(raw % 3 - 1, c->reach, lo[0], n[0]);
+        packed_box(raw / 3 % 3 - 1, c->reach, lo[1], n[1]);
+        packed_box(raw / 9 - 1, c->reach, lo[2], n[2]);
+        const size_t ncell = (size_t)n[0] * n[1] * n[2];
+        double* d0 = dst + at;
+        double* d1 = d0 + ncell * 20;
+        at += ncell * (multipole ? 23 : 1);
         if (nb.count == kCells && !nb.cells) {
-            if (multipole) {
-                HIPC(c, hipMemcpyAsync(w.M + sl * nM, nb.M, sizeof(double) * nM, hipMemcpyHostToDevice, st));
-                HIPC(c, hipMemcpyAsync(w.com + sl * nC, nb.com, sizeof(double) * nC, hipMemcpyHostToDevice, st));
-            } else {
-                HIPC(c, hipMemcpyAsync(w.mon + sl * kCells, nb.mon, sizeof(double) * kCells, hipMemcpyHostToDevice, st));
-            }
-        } else {
-            // each listed cell once, from its last occurrence (later entries win,
-            // as in update_input's loop over the list)
-            int16_t last[kCells];
-            for (int i = 0; i < kCells; ++i) last[i] = -1;
-            for (int i = 0; i < nb.count; ++i) last[nb.cells[i]] = (int16_t)i;
-            int2* idx = c->h_idx + (size_t)np * kCells;
-            int n = 0;
-            for (int cell = 0; cell < kCells; ++cell)
-                if (last[cell] >= 0) idx[n++] = make_int2(cell, last[cell]);
-            if (nb.count > 0) {
-                if (multipole) {
-                    HIPC(c, hipMemcpyAsync(w.cM + np * nM, nb.M, sizeof(double) * 20 * nb.count,
-                        hipMemcpyHostToDevice, st));
-                    HIPC(c, hipMemcpyAsync(w.ccom + np * nC, nb.com, sizeof(double) * 3 * nb.count,
-                        hipMemcpyHostToDevice, st));
-                } else {
-                    HIPC(c, hipMemcpyAsync(w.cmon + (size_t)np * kCells, nb.mon, sizeof(double) * nb.count,
-                        hipMemcpyHostToDevice, st));
+            for (int x = lo[0]; x < lo[0] + n[0]; ++x)
+                for (int y = lo[1]; y < lo[1] + n[1]; ++y) {
+                    const size_t cell = (size_t)x * 64 + y * 8 + lo[2], nz = (size_t)n[2];
+                    if (multipole) {
+                        std::memcpy(d0, nb.M + cell * 20, sizeof(double) * 20 * nz);
+                        std::memcpy(d1, nb.com + cell * 3, sizeof(double) * 3 * nz);
+                        d0 += 20 * nz;
+                        d1 += 3 * nz;
+                    } else {
+                        std::memcpy(d0, nb.mon + cell, sizeof(double) * nz);
+                        d0 += nz;
+                    }
                 }
-            }
-            sa.slot[np] = sl;
-            sa.count[np] = n;
-            sa.multipole[np] = multipole ? 1 : 0;
-            ++np;
+            continue;
         }
-        kind[sl] = multipole ? OCTOFMM_SLOT_NONLEAF : OCTOFMM_SLOT_LEAF;
-        nbr[13 * 27 + sl] = sl;
+        int16_t last[kCells];
+        for (int i = 0; i < kCells; ++i) last[i] = -1;
+        for (int i = 0; i < nb.count; ++i) last[nb.cells[i]] = (int16_t)i;
+        for (int x = lo[0]; x < lo[0] + n[0]; ++x)
+            for (int y = lo[1]; y < lo[1] + n[1]; ++y)
+                for (int z = lo[2]; z < lo[2] + n[2]; ++z) {
+                    const int i = last[x * 64 + y * 8 + z];
+                    if (!multipole) {
+                        *d0++ = i >= 0 ? nb.mon[i] : 0.0;
+                        continue;
+                    }
+                    for (int k = 0; k < 20; ++k) d0[k] = i >= 0 ? nb.M[(size_t)i * 20 + k] : 0.0;
+                    for (int k = 0; k < 3; ++k) d1[k] = i >= 0 ? nb.com[(size_t)i * 3 + k] : 0.0;
+                    d0 += 20;
+                    d1 += 3;
+                }
     }
-    HIPC(c, hipMemcpyAsync(w.meta, meta, sizeof(int32_t) * kMetaSize, hipMemcpyHostToDevice, st));
-    HIPC(c, hipMemcpyAsync(w.fx, c->h_fx, sizeof(double) * 81, hipMemcpyHostToDevice, st));
-    if (np > 0) {
-        HIPC(c, hipMemcpyAsync(w.cidx, c->h_idx, sizeof(int2) * kCells * np, hipMemcpyHostToDevice, st));
-        sa.cM = w.cM;
-        sa.ccom = w.ccom;
-        sa.cmon = w.cmon;
-        sa.cidx = w.cidx;
-        sa.M = w.M;
-        sa.com = w.com;
-        sa.mon = w.mon;
-        hipLaunchKernelGGL(scatter_partial, dim3(np), dim3(256), 0, st, sa);
-        HIPC(c, hipGetLastError());
-    }
-    return OCTOFMM_OK;
 }
 
-}   // namespace
-
-// Runs one loaded sub-grid through a workspace: the caller's L is copied in
-// and the kernels add the sub-grid's interactions to it (the same single
-// addition per component a host-side L += result makes), then L comes back,
-// and L_c (when the call writes it) is copied out; synchronous.
-static octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace& w, double dx, int type,
-    int item_flags, bool root, double* L, double* L_c) {
+// The kernels of one packed sub-grid on the context's stream: its interactions
+// alone go to the results in the pinned memory.
+octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace& w, PackedArgs& pa, bool root) {
     hipStream_t st = c->stream;
-    const int rho = type == OCTOFMM_RHO;
-    StageArgs sa;
-    sa.M = w.M;
-    sa.com = w.com;
-    sa.mon = w.mon;
-    sa.kind = w.meta + kMetaKind;
-    sa.fxbase = w.fx;
-    sa.foff = w.meta + kMetaFoff;
-    sa.rec = w.rec;
-    sa.recm = nullptr;
-    sa.rho = rho;
-    sa.list = nullptr;
-    sa.dx = dx;
-    sa.nslots = 27;
-    hipLaunchKernelGGL(stage_records, dim3(27 * 4), dim3(256), 0, st, sa);
+    const bool rho = pa.rho != 0;
+    pa.rec = w.rec;
+    pa.mon = w.mon;
+    pa.com = w.com;
+    pa.meta = w.meta;
+    hipLaunchKernelGGL(stage_packed, dim3(root ? 4 : 27 * 4), dim3(256), 0, st, pa);
     HIPC(c, hipGetLastError());
-    const size_t nL = (size_t)kCells * 20, nC = (size_t)kCells * 3;
-    double* L13 = w.L + 13 * nL;
-    double* C13 = w.Lc + 13 * nC;
-    HIPC(c, hipMemcpyAsync(L13, L, sizeof(double) * nL, hipMemcpyHostToDevice, st));
+    double* L = c->h_pin;
+    double* Lc = c->h_pin + (size_t)kCells * 20;
     if (root) {
         RootArgs ra;
-        ra.rec = w.rec + (size_t)13 * kCells * kRecDoubles;
+        ra.rec = w.rec;
         ra.tab = c->d_tab;
         ra.partial = w.partial;
         ra.per_chunk = kCells / kRootChunks;
@@ -2371,68 +2385,80 @@ static octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace&
         HIPC(c, hipGetLastError());
         RootReduceArgs rr;
         rr.partial = w.partial;
-        rr.L = L13;
-        rr.Lc = C13;
+        rr.L = L;
+        rr.Lc = Lc;
         rr.nchunks = kRootChunks;
         rr.rho = rho;
-        rr.overwrite = 0;
+        rr.overwrite = 1;
         hipLaunchKernelGGL(root_reduce, dim3((kCells * 23 + 255) / 256), dim3(256), 0, st, rr);
         HIPC(c, hipGetLastError());
-    } else {
-        LevelArgs la;
-        la.rec = w.rec;
-        la.com = w.com;
-        la.L = w.L;
-        la.Lc = w.Lc;
-        la.nbr = w.meta + kMetaNbr;
-        la.kind = w.meta + kMetaKind;
-        la.items = reinterpret_cast<const int2*>(w.meta + kMetaItems);
-        la.tab = c->d_tab;
-        la.mixbits = nullptr;
-        la.recm = nullptr;
-        la.mixorder = nullptr;
-        la.mix_n64 = 0;
-        la.queue = nullptr;
-        la.parts = 0;
-        la.wide_sums = nullptr;
-        la.mon = w.mon;
-        la.p2m_out = w.p2m;
-        la.parent = nullptr;
-        la.octant = nullptr;
-        la.pL = la.pLc = la.pcom = nullptr;
-        la.g = nullptr;
-        la.G = 1.0;
-        la.l2l = 0;
-        la.correct_am = 0;
-        la.leaf_rows = 1;
-        la.nitems = 1;
-        la.item0 = 0;
-        la.inv_dx = 1.0 / dx;
-        la.neg_inv_dx = -1.0 / dx;
-        if (item_flags & kItemLeaf) {
-            if (item_flags & kItemP2M) {
-                if (rho)
-                    launch_p2m<true>(1, st, la);
-                else
-                    launch_p2m<false>(1, st, la);
-                HIPC(c, hipGetLastError());
-            }
-            if (rho)
-                launch_leaf<true>(1, st, la, c->tab);
-            else
-                launch_leaf<false>(1, st, la, c->tab);
-        } else if (rho) {
-            launch_level<true>(8, 1, st, la);
-        } else {
-            launch_level<false>(8, 1, st, la);
-        }
-        HIPC(c, hipGetLastError());
+        return OCTOFMM_OK;
     }
-    HIPC(c, hipMemcpyAsync(L, L13, sizeof(double) * nL, hipMemcpyDeviceToHost, st));
-    if (L_c) HIPC(c, hipMemcpyAsync(L_c, C13, sizeof(double) * nC, hipMemcpyDeviceToHost, st));
-    HIPC(c, hipStreamSynchronize(st));
+    LevelArgs la;
+    std::memset(&la, 0, sizeof(la));
+    la.rec = w.rec;
+    la.com = w.com;
+    la.L = L;
+    la.Lc = Lc;
+    la.nbr = w.meta + kMetaNbr;
+    la.kind = w.meta + kMetaKind;
+    la.items = reinterpret_cast<const int2*>(w.meta + kMetaItems);
+    la.tab = c->d_tab;
+    la.parts = wide_parts(1, c->tab);
+    la.wide_sums = w.wide;
+    la.mon = w.mon;
+    la.p2m_out = w.p2m;
+    la.G = 1.0;
+    la.leaf_rows = 1;
+    la.overwrite = 1;
+    la.nitems = 1;
+    la.inv_dx = 1.0 / pa.dx;
+    la.neg_inv_dx = -1.0 / pa.dx;
+    if (pa.item_flags & kItemLeaf) {
+        if (pa.item_flags & kItemP2M) {
+            if (rho)
+                launch_p2m<true>(1, st, la);
+            else
+                launch_p2m<false>(1, st, la);
+            HIPC(c, hipGetLastError());
+        }
+        if (rho)
+            launch_leaf<true>(1, st, la, c->tab);
+        else
+            launch_leaf<false>(1, st, la, c->tab);
+    } else if (rho) {
+        launch_level<true>(704, 1, st, la);
+    } else {
+        launch_level<false>(704, 1, st, la);
+    }
+    HIPC(c, hipGetLastError());
     return OCTOFMM_OK;
 }
+
+// One per-sub-grid call through a workspace, synchronous: packs the inputs,
+// runs the kernels and adds their results to the caller's L (the same single
+// addition per component a device-side L += result makes); L_c is copied out
+// when the call writes it.
+octofmm_status run_subgrid(octofmm_context* c, const SubgridWorkspace& w, const octofmm_subgrid* in, bool leaf_target,
+    bool root, int item_flags, double* L, double* L_c) {
+    PackedArgs pa;
+    pack_subgrid(c, in, leaf_target, root, item_flags, pa);
+    const octofmm_status s = launch_subgrid(c, w, pa, root);
+    const hipError_t e = hipStreamSynchronize(c->stream);   // also before an error leaves the pinned memory to the next call
+    if (s != OCTOFMM_OK) return s;
+    HIPC(c, e);
+    const double* out = c->h_pin;
+    if (leaf_target) {
+        for (int i = 0; i < kCells; ++i)
+            for (int k = 0; k < 4; ++k) L[i * 20 + k] += out[i * 20 + k];
+    } else {
+        for (int i = 0; i < kCells * 20; ++i) L[i] += out[i];
+    }
+    if (L_c) std::memcpy(L_c, out + (size_t)kCells * 20, sizeof(double) * kCells * 3);
+    return OCTOFMM_OK;
+}
+
+}   // namespace
 
 // ===========================================================================
 // C-ABI
@@ -2468,20 +2494,20 @@ octofmm_status octofmm_create(const octofmm_config* cfg, octofmm_context** out) 
     c->theta = cfg->theta;
     c->flags = cfg->flags;
     c->err.reserve(600);   // error texts (at most 511 characters) are stored without allocating
-    c->h_meta = new int32_t[kMetaSize];
-    c->h_fx = new double[81];
-    c->h_idx = new int2[26 * kCells];
     char err[256];
     if (!build_tables(cfg->theta, c->tab, err, sizeof(err))) {
         delete c;
         return OCTOFMM_ERR_THETA;
     }
     if (hipSetDevice(c->device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_pin, sizeof(double) * (kPinOut + pin_cells(c->tab) * 23), hipHostMallocDefault) !=
+            hipSuccess ||
         hipMalloc((void**)&c->d_tab, sizeof(Tables)) != hipSuccess ||
         hipMemcpy(c->d_tab, &c->tab, sizeof(Tables), hipMemcpyHostToDevice) != hipSuccess) {
         octofmm_destroy(c);
         return OCTOFMM_ERR_HIP;
     }
+    c->reach = 2 * c->tab.max_delta;
     c->d_scratch = scratch_address(c->device);
     if (!c->d_scratch) {
         octofmm_destroy(c);
@@ -2495,9 +2521,7 @@ octofmm_status octofmm_destroy(octofmm_context* c) {
     if (!c) return OCTOFMM_OK;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    delete[] c->h_meta;
-    delete[] c->h_fx;
-    delete[] c->h_idx;
+    (void)hipHostFree(c->h_pin);
     (void)hipFree(c->d_ws);
     (void)hipFree(c->d_tab);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -2540,9 +2564,7 @@ octofmm_status octofmm_compute_multipole_interactions(octofmm_context* c, const 
     (void)hipGetLastError();   // launch checks below report this call's launches only
     s = ensure_workspace(c);
     if (s != OCTOFMM_OK) return s;
-    s = load_subgrid(c, c->ws, in, false, root, flags);
-    if (s != OCTOFMM_OK) return s;
-    return launch_subgrid(c, c->ws, in->dx, in->type, flags, root, L, in->type == OCTOFMM_RHO ? L_c : nullptr);
+    return run_subgrid(c, c->ws, in, false, root, flags, L, in->type == OCTOFMM_RHO ? L_c : nullptr);
 }
 
 // The same call with the workspace in `scratch` instead of the context's
@@ -2563,9 +2585,7 @@ octofmm_status octofmm_compute_multipole_interactions_noalloc(octofmm_context* c
     (void)hipGetLastError();   // launch checks below report this call's launches only
     std::lock_guard<std::mutex> lock(g_scratch_call_mu[c->device]);
     const SubgridWorkspace w = carve_workspace(c->d_scratch);
-    s = load_subgrid(c, w, in, false, root, flags);
-    if (s != OCTOFMM_OK) return s;
-    return launch_subgrid(c, w, in->dx, in->type, flags, root, L, in->type == OCTOFMM_RHO ? L_c : nullptr);
+    return run_subgrid(c, w, in, false, root, flags, L, in->type == OCTOFMM_RHO ? L_c : nullptr);
 }
 
 octofmm_status octofmm_compute_monopole_interactions(octofmm_context* c, const octofmm_subgrid* in,
@@ -2588,10 +2608,7 @@ octofmm_status octofmm_compute_monopole_interactions(octofmm_context* c, const o
     s = ensure_workspace(c);
     if (s != OCTOFMM_OK) return s;
     const int flags = kItemLeaf | (p2m ? kItemP2M : 0);
-    s = load_subgrid(c, c->ws, in, true, false, flags);
-    if (s != OCTOFMM_OK) return s;
-    return launch_subgrid(c, c->ws, in->dx, in->type, flags, false, L,
-        in->type == OCTOFMM_RHO && p2m ? L_c : nullptr);
+    return run_subgrid(c, c->ws, in, true, false, flags, L, in->type == OCTOFMM_RHO && p2m ? L_c : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -2705,6 +2722,7 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         la.l2l = p->l2l ? 1 : 0;
         la.correct_am = p->t_correct_am;
         la.leaf_rows = p->leaf_rows;
+        la.overwrite = 0;
         la.inv_dx = 1.0 / p->dx;
         la.neg_inv_dx = -1.0 / p->dx;
         const bool rho = p->type == OCTOFMM_RHO;

@@ -645,6 +645,11 @@ struct LevelArgs {
     // leaf targets with refined neighbours: the p2m sums (L0..3, L_c, 0) of
     // each cell, [p2m item][512][8], written by p2m_kernel for leaf_kernel
     double* p2m_out;
+    // its work lists (P2mPacks)
+    const int32_t* p2m_hdr;
+    const int32_t* p2m_units;
+    const int32_t* p2m_idx;
+    const int32_t* p2m_di;
     // Whole-tree solves (l2l != 0): the level's expansions are written, not
     // accumulated, as interactions + the parent cell's final expansion
     // re-expanded about the cell's centre of mass (and L_c + the parent's

@@ -269,6 +269,10 @@ struct PackedArgs {
     double* mon;            // [27][512]
     double* com;            // [512][3] a leaf target's centres
     int32_t* meta;          // items[2] nbr[27] kind[27]
+    const int32_t* packs_src;   // p2m work lists in pinned memory, packs_n words, copied to packs
+    int32_t* packs;
+    int32_t packs_n;
+    double* p2m;            // [512][8] p2m sums, cleared for leaf targets
 };
 
 __global__ __launch_bounds__(256) void stage_packed(PackedArgs a) {
@@ -280,6 +284,9 @@ __global__ __launch_bounds__(256) void stage_packed(PackedArgs a) {
         a.meta[2 + t] = a.kind[packed_slot(t)] >= 0 ? packed_slot(t) : -1;
         a.meta[29 + t] = a.kind[t];
     }
+    for (int i = blockIdx.x * 256 + t; i < a.packs_n; i += gridDim.x * 256) a.packs[i] = a.packs_src[i];
+    if (a.leaf_target)
+        for (int i = blockIdx.x * 256 + t; i < kCells * 8; i += gridDim.x * 256) a.p2m[i] = 0.0;
     const int k = a.kind[slot], raw = packed_raw(slot);
     int lo[3], n[3];
     packed_box(raw % 3 - 1, a.reach, lo[0], n[0]);
@@ -1386,173 +1393,136 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void l
     }
 }
 
-// p2m on the staging of lane mapping 7: for leaf targets with refined
-// neighbours, the pairs whose partner cell lies in a refined neighbour slot
-// (far and near alike, monopole_kernel_templates.hpp:69-239) are the M2L pair
-// set of the target's cells restricted to those slots.  So a workgroup of
-// SPLIT waves takes one coarse block of one such leaf (lane = coarse cell x
-// child, as in the M2L kernels) and walks only the coarse offsets that reach
-// a refined neighbour from that block; each offset's 64 partner records are
-// staged into the wave's LDS image by direct loads and read as 8-lane
-// broadcasts.  The waves split the offsets and hand their sums to wave 0,
-// which adds them in wave order and writes each cell's (L0..3, L_c, 0) to
-// p2m_out[p2m item][cell].
-template <bool RHO, int SPLIT>
-__device__ void p2m_item(const LevelArgs& a, int slot, int ordinal, int w, const int* s_nbr, const int* s_kind,
-    const int* s_live, int nlive, double2* __restrict__ s_stage, int sl) {
-    double2* stage = s_stage + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kDirWave;
-    const int l = threadIdx.x & 63, c = l >> 3;
-    const auto* tab = as_const(a.tab);
-    const int wu = __builtin_amdgcn_readfirstlane(w);
-    const LaneGeom g = lane_geom(wu);
-    const double* xc = a.com + ((size_t)slot * kCells + g.cell) * 3;
+// p2m: for leaf targets with refined neighbours, the pairs whose partner cell
+// lies in a refined neighbour slot (far and near alike,
+// monopole_kernel_templates.hpp:69-239), which are the M2L pair set of the
+// target's cells restricted to those slots.  Only coarse cells at the faces,
+// edges and corners towards refined neighbours have any, and between 1 and 26
+// partner coarse cells each at theta 0.5, so the host lists them when the plan
+// is made (build_p2m_packs): a unit is one coarse cell of one leaf, a pack is 8
+// units of like length, from any leaves.  One workgroup of 4 waves takes a
+// pack: lane = (unit, child), wave sl takes the units' entries sl, sl + 4, ...,
+// staging each entry's 8 x 8 partner records into its LDS image by direct loads
+// and reading them as 8-lane broadcasts; the waves hand their sums to wave 0,
+// which adds them in wave order.  Walked by 2x2x2 coarse blocks of a leaf
+// instead, half the lanes of a face's blocks and 7 of 8 of a corner's idled and
+// half the workgroups found nothing to do.
+// Bound by the FP64 VALU like the M2L kernel, and by its share of the chip
+// while it runs beside that one: a 2048-slot level of mixed kinds takes 741 us
+// in place of 803, the solve of a 10,697-sub-grid tree 1338 in place of 1416.
+//
+// FULL: every pair of an entry's 8 x 8 cells is in the stencil (theta 0.5).
+template <bool RHO, bool FULL>
+__global__ __launch_bounds__(256) void p2m_kernel(LevelArgs a) {
+    __shared__ double2 s_stage[4 * kDirWave];
+    const int pack = xcd_item(blockIdx.x, gridDim.x);
+    const int sl = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    double2* stage = s_stage + sl * kDirWave;
+    const int l = threadIdx.x & 63, k = l & 7;
+    const auto* hdr = as_const(a.p2m_hdr) + 2 * __builtin_amdgcn_readfirstlane(pack);
+    const int first = hdr[0], n = hdr[1];
+    const int unit = a.p2m_units[(size_t)pack * 8 + (l >> 3)];   // -1: none
+    const int C = unit & 63, ordinal = unit < 0 ? 0 : unit >> 6;
+    const int cell = (2 * (C >> 4) + (k >> 2)) * 64 + (2 * ((C >> 2) & 3) + ((k >> 1) & 1)) * 8 + 2 * (C & 3) + (k & 1);
+    const double* xc = a.com + ((size_t)a.items[a.item0 + ordinal].x * kCells + cell) * 3;
     const double X0 = xc[0], X1 = xc[1], X2 = xc[2];
     Acc<RHO> s;
     acc_clear(s);
-    const int bx = ((wu >> 2) & 1) * 2, by = ((wu >> 1) & 1) * 2, bz = (wu & 1) * 2;
-    // partner coarse cell of group gi at offset (ax, ay, az): its records, and
-    // bit gi of `absent` where it is not in a refined neighbour slot
-    auto group_base = [&](int gi, int ax, int ay, int az, unsigned& absent) -> const char* {
-        const int px = bx + ((gi >> 2) & 1) + ax, py = by + ((gi >> 1) & 1) + ay, pz = bz + (gi & 1) + az;
-        const int raw = (px < 0 ? 0 : (px < 4 ? 1 : 2)) + 3 * (py < 0 ? 0 : (py < 4 ? 1 : 2)) +
-            9 * (pz < 0 ? 0 : (pz < 4 ? 1 : 2));
-        const int ns = s_nbr[raw];
-        const bool refined = raw != 13 && ns >= 0 && s_kind[raw] == OCTOFMM_SLOT_NONLEAF;
-        if (!refined) absent |= 1u << gi;
-        const int cb = ((px & 3) * 16 + (py & 3) * 4 + (pz & 3)) * 8;
-        return reinterpret_cast<const char*>(a.rec + ((size_t)(refined ? ns : 0) * kCells + cb) * kRecDoubles);
-    };
-    const unsigned loff = (unsigned)l * 16u;
-    const char* nbase[8];
+    // the records of entry e's 8 partner coarse cells; bit g of `absent` where
+    // unit g has fewer entries
+    unsigned nrec[8];
     unsigned absent_next = 0;
-    auto bases = [&](int di) {
-        const int ax = tab->delta[di][0], ay = tab->delta[di][1], az = tab->delta[di][2];
+    auto bases = [&](int e) {
+        const auto* row = as_const(a.p2m_idx) + (size_t)(first + e) * 8;
         unsigned absent = 0;
 #pragma unroll
-        for (int gi = 0; gi < 8; ++gi) nbase[gi] = group_base(gi, ax, ay, az, absent);
-        asm volatile("" ::"s"(nbase[0]), "s"(nbase[1]), "s"(nbase[2]), "s"(nbase[3]), "s"(nbase[4]),
-                     "s"(nbase[5]), "s"(nbase[6]), "s"(nbase[7]));
+        for (int g = 0; g < 8; ++g) {
+            const int r = row[g];
+            if (r < 0) absent |= 1u << g;
+            nrec[g] = (unsigned)(r < 0 ? 0 : r);
+        }
+        form_sgprs(nrec);
         absent_next = absent;
     };
     // the full-wave loads of every group first, the half-wave loads after
     // them in a branch of their own (as in m2l_item_direct)
+    const char* rb = reinterpret_cast<const char*>(a.rec);
+    const unsigned loff = (unsigned)l * 16u;
     auto issue = [&]() {
 #pragma unroll
-        for (int gi = 0; gi < 8; ++gi)
-            __builtin_amdgcn_global_load_lds(nbase[gi] + loff, (lds_ptr)(stage + gi * kDirGroup), 16, 0, 0);
+        for (int g = 0; g < 8; ++g)
+            __builtin_amdgcn_global_load_lds(uniform_ptr(rb + (size_t)nrec[g] * kRecBytes) + loff,
+                                             (lds_ptr)(stage + g * kDirGroup), 16, 0, 0);
         if (l < 32) {
 #pragma unroll
-            for (int gi = 0; gi < 8; ++gi)
-                __builtin_amdgcn_global_load_lds(nbase[gi] + 1024 + loff, (lds_ptr)(stage + gi * kDirGroup + 64), 16, 0, 0);
+            for (int g = 0; g < 8; ++g)
+                __builtin_amdgcn_global_load_lds(uniform_ptr(rb + (size_t)nrec[g] * kRecBytes + 1024) + loff,
+                                                 (lds_ptr)(stage + g * kDirGroup + 64), 16, 0, 0);
         }
     };
-    const double2* group = stage + c * kDirGroup;
-    const int q0 = __builtin_amdgcn_readfirstlane(sl);
-    if (q0 < nlive) {
-        bases(s_live[q0]);
+    const double2* group = stage + (l >> 3) * kDirGroup;
+    if (sl < n) {
+        bases(sl);
         issue();
     }
-    for (int q = q0; q < nlive; q += SPLIT) {
-        // lanes of step j: the classes in byte j of the offset's pair rows,
-        // in the groups whose partner is in a refined slot (lane mask formed
-        // in scalar registers, lane = group * 8 + class)
-        const int di = s_live[q];
-        const uint64_t rows = tab->allrows[di];
-        const uint64_t gone = spread_groups(absent_next);
-        if (q + SPLIT < nlive) bases(s_live[q + SPLIT]);
+    for (int e = sl; e < n; e += 4) {
+        const uint64_t here = ~spread_groups(absent_next);
+        // the lane's pairs of this entry (byte k of the offset's pair bits)
+        unsigned mine = 0xffu;
+        if constexpr (!FULL) {
+            const int di = a.p2m_di[(size_t)(first + e) * 8 + (l >> 3)];
+            mine = (unsigned)((a.tab->farbits[di] | a.tab->nearbits[di]) >> (8 * k)) & 0xffu;
+        }
+        if (e + 4 < n) bases(e + 4);
         __builtin_amdgcn_s_waitcnt(0x3F70);   // vmcnt(0): this wave's image is in LDS
         __builtin_amdgcn_wave_barrier();
+        if (__builtin_amdgcn_inverse_ballot_w64(here)) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            if (__builtin_amdgcn_inverse_ballot_w64(step_lanes(rows, 0, gone, 0, j))) {
-                Rec cur;
+            for (int j = 0; j < 8; ++j) {
+                if (FULL || (mine & (1u << j))) {
+                    Rec cur;
 #pragma unroll
-                for (int i = 0; i < 12; ++i) cur.v[i] = group[j * 12 + i];
-                p2m_pair_rec<RHO>(cur, X0, X1, X2, s);
+                    for (int i = 0; i < 12; ++i) cur.v[i] = group[j * 12 + i];
+                    p2m_pair_rec<RHO>(cur, X0, X1, X2, s);
+                }
             }
         }
         lds_wave_sync();   // every read of the image done before it is refilled
-        if (q + SPLIT < nlive) issue();
+        if (e + 4 < n) issue();
     }
-    // waves 1..SPLIT-1 hand their sums to wave 0 through their own images
-    double L[4], C[3];
-    p2m_finish<RHO>(s, L, C);
+    // waves 1..3 hand their sums to wave 0 through their own images
+    double L[4], C3[3];
+    p2m_finish<RHO>(s, L, C3);
     double* part = reinterpret_cast<double*>(stage) + l * 7;
-    if (q0 != 0) {
+    if (sl != 0) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) part[i] = L[i];
-        part[4] = C[0];
-        part[5] = C[1];
-        part[6] = C[2];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) part[4 + i] = C3[i];
     }
     __syncthreads();
-    if (q0 != 0) return;
-    for (int o = 1; o < SPLIT; ++o) {
+    if (sl != 0 || unit < 0) return;
+    for (int o = 1; o < 4; ++o) {
         const double* po = reinterpret_cast<const double*>(s_stage + o * kDirWave) + l * 7;
 #pragma unroll
         for (int i = 0; i < 4; ++i) L[i] += po[i];
-        C[0] += po[4];
-        C[1] += po[5];
-        C[2] += po[6];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) C3[i] += po[4 + i];
     }
-    double2* out = reinterpret_cast<double2*>(a.p2m_out + ((size_t)ordinal * kCells + g.cell) * 8);
+    double2* out = reinterpret_cast<double2*>(a.p2m_out + ((size_t)ordinal * kCells + cell) * 8);
     out[0] = make_double2(L[0], L[1]);
     out[1] = make_double2(L[2], L[3]);
-    out[2] = make_double2(C[0], C[1]);
-    out[3] = make_double2(C[2], 0.0);
-}
-
-// One workgroup of SPLIT waves per (leaf item with p2m, coarse block); the
-// items are a.items[a.item0 ...], in the order their sums are stored.
-template <bool RHO, int SPLIT>
-__global__ __launch_bounds__(64 * SPLIT) void p2m_kernel(LevelArgs a) {
-    __shared__ int s_nbr[27];
-    __shared__ int s_kind[27];
-    __shared__ int s_live[kMaxDelta];
-    __shared__ int s_nlive;
-    __shared__ double2 s_stage[SPLIT * kDirWave];
-    const int v = xcd_item(blockIdx.x, gridDim.x);
-    const int ordinal = v >> 3, w = v & 7;
-    const int2 it = a.items[a.item0 + ordinal];
-    if (threadIdx.x < 27) {
-        const int n = a.nbr[(size_t)it.x * 27 + threadIdx.x];
-        s_nbr[threadIdx.x] = n;
-        s_kind[threadIdx.x] = n >= 0 ? a.kind[n] : -1;
-    }
-    __syncthreads();
-    // the coarse offsets with a pair whose partner coarse cell, seen from this
-    // block, lies in a refined neighbour slot (wave 0, one offset per lane,
-    // compacted in offset order by a ballot)
-    if (threadIdx.x < 64) {
-        const Tables* tab = a.tab;
-        const int lane = threadIdx.x;
-        const int bx = ((w >> 2) & 1) * 2, by = ((w >> 1) & 1) * 2, bz = (w & 1) * 2;
-        int n = 0;
-        for (int base = 0; base < tab->ndelta; base += 64) {
-            const int di = base + lane;
-            bool live = false;
-            if (di < tab->ndelta && (tab->farbits[di] | tab->nearbits[di])) {
-                const int ax = tab->delta[di][0], ay = tab->delta[di][1], az = tab->delta[di][2];
-                for (int gi = 0; gi < 8; ++gi) {
-                    const int px = bx + ((gi >> 2) & 1) + ax, py = by + ((gi >> 1) & 1) + ay, pz = bz + (gi & 1) + az;
-                    const int raw = (px < 0 ? 0 : (px < 4 ? 1 : 2)) + 3 * (py < 0 ? 0 : (py < 4 ? 1 : 2)) +
-                        9 * (pz < 0 ? 0 : (pz < 4 ? 1 : 2));
-                    live = live || (raw != 13 && s_nbr[raw] >= 0 && s_kind[raw] == OCTOFMM_SLOT_NONLEAF);
-                }
-            }
-            const uint64_t m = __ballot(live);
-            if (live) s_live[n + __popcll(m & ((uint64_t(1) << lane) - 1))] = di;
-            n += __popcll(m);
-        }
-        if (lane == 0) s_nlive = n;
-    }
-    __syncthreads();
-    p2m_item<RHO, SPLIT>(a, it.x, ordinal, w, s_nbr, s_kind, s_live, s_nlive, s_stage, (int)(threadIdx.x >> 6));
+    out[2] = make_double2(C3[0], C3[1]);
+    out[3] = make_double2(C3[2], 0.0);
 }
 
 template <bool RHO>
-void launch_p2m(int nitems, hipStream_t st, const LevelArgs& la) {
-    hipLaunchKernelGGL((p2m_kernel<RHO, 4>), dim3(nitems * 8), dim3(256), 0, st, la);
+void launch_p2m(int npacks, hipStream_t st, const LevelArgs& la, const Tables& tab) {
+    if (npacks <= 0) return;
+    if (tab.p2p_cube)
+        hipLaunchKernelGGL((p2m_kernel<RHO, true>), dim3(npacks), dim3(256), 0, st, la);
+    else
+        hipLaunchKernelGGL((p2m_kernel<RHO, false>), dim3(npacks), dim3(256), 0, st, la);
 }
 
 template <bool RHO>
@@ -2036,6 +2006,93 @@ __global__ __launch_bounds__(256) void m2m_kernel(M2MArgs a) {
 namespace {
 
 constexpr int kRootChunks = 64;
+
+// Work lists of p2m_kernel.  hdr: first row and number of rows of each pack;
+// units: 8 per pack, ordinal * 64 + coarse cell, or -1; idx: per row (entry)
+// and unit the partner coarse cell's first record, or -1; di: its offset.
+struct P2mPacks {
+    std::vector<int32_t> hdr, units, idx, di;
+    int npacks() const { return (int)hdr.size() / 2; }
+};
+
+// The coarse cells of a sub-grid that reach into its neighbour in direction
+// raw: (own coarse cell, offset, first record in the neighbour).
+struct P2mReach {
+    struct Hit {
+        int16_t C, di, rec;
+    };
+    std::vector<Hit> by_raw[27];
+};
+
+void build_p2m_reach(const Tables& T, P2mReach& r) {
+    for (int di = 0; di < T.ndelta; ++di) {
+        if (!(T.farbits[di] | T.nearbits[di])) continue;
+        for (int C = 0; C < 64; ++C) {
+            const int px = (C >> 4) + T.delta[di][0], py = ((C >> 2) & 3) + T.delta[di][1], pz = (C & 3) + T.delta[di][2];
+            const int raw = (px < 0 ? 0 : px < 4 ? 1 : 2) + 3 * (py < 0 ? 0 : py < 4 ? 1 : 2) +
+                9 * (pz < 0 ? 0 : pz < 4 ? 1 : 2);
+            if (raw != 13)
+                r.by_raw[raw].push_back(
+                    {(int16_t)C, (int16_t)di, (int16_t)(((px & 3) * 16 + (py & 3) * 4 + (pz & 3)) * 8)});
+        }
+    }
+}
+
+// refined(ordinal, raw): the slot of that item's neighbour where it is
+// refined, else -1.  Units go to packs by falling length, in item order where
+// equal, so a pack's 8 units are of like length and near each other.
+template <typename F>
+void build_p2m_packs(const P2mReach& reach, int nitems, F&& refined, P2mPacks& out) {
+    struct Unit {
+        int32_t id, first, n;
+    };
+    std::vector<Unit> units;
+    std::vector<int32_t> rec, di;
+    int longest = 0;
+    std::vector<int32_t> crec[64], cdi[64];
+    for (int o = 0; o < nitems; ++o) {
+        for (int C = 0; C < 64; ++C) {
+            crec[C].clear();
+            cdi[C].clear();
+        }
+        for (int raw = 0; raw < 27; ++raw) {
+            const int slot = raw == 13 ? -1 : refined(o, raw);
+            if (slot < 0) continue;
+            for (const P2mReach::Hit& h : reach.by_raw[raw]) {
+                crec[h.C].push_back(slot * kCells + h.rec);
+                cdi[h.C].push_back(h.di);
+            }
+        }
+        for (int C = 0; C < 64; ++C) {
+            if (crec[C].empty()) continue;
+            units.push_back({o * 64 + C, (int32_t)rec.size(), (int32_t)crec[C].size()});
+            longest = std::max(longest, (int)crec[C].size());
+            rec.insert(rec.end(), crec[C].begin(), crec[C].end());
+            di.insert(di.end(), cdi[C].begin(), cdi[C].end());
+        }
+    }
+    std::vector<std::vector<int32_t>> by_n(longest + 1);
+    for (size_t u = 0; u < units.size(); ++u) by_n[units[u].n].push_back((int32_t)u);
+    std::vector<int32_t> order;
+    for (int n = longest; n > 0; --n) order.insert(order.end(), by_n[n].begin(), by_n[n].end());
+    for (size_t p = 0; p < order.size(); p += 8) {
+        const int rows = units[order[p]].n, first = (int)out.idx.size() / 8;
+        out.hdr.push_back(first);
+        out.hdr.push_back(rows);
+        out.idx.resize((size_t)(first + rows) * 8, -1);
+        out.di.resize((size_t)(first + rows) * 8, 0);
+        for (int g = 0; g < 8; ++g) {
+            const bool have = p + g < order.size();
+            out.units.push_back(have ? units[order[p + g]].id : -1);
+            if (!have) continue;
+            const Unit& u = units[order[p + g]];
+            for (int e = 0; e < u.n; ++e) {
+                out.idx[(size_t)(first + e) * 8 + g] = rec[u.first + e];
+                out.di[(size_t)(first + e) * 8 + g] = di[u.first + e];
+            }
+        }
+    }
+}
 // record buffers end with a tail the direct-to-LDS staging may read into
 // (one 16-byte pad chunk past the last record)
 constexpr size_t kRecTailBytes = 4096;
@@ -2061,7 +2118,13 @@ struct SubgridWorkspace {
     double* partial = nullptr;  // [kRootChunks][512][24]
     double* p2m = nullptr;      // [512][8] p2m sums of a leaf target
     int32_t* meta = nullptr;    // kMetaSize
+    int32_t* packs = nullptr;   // p2m work lists (kPackWords)
 };
+
+// p2m work lists of one leaf target, in words: hdr 2 x 8, units 64, then idx
+// and di of at most 8 packs of kMaxDelta rows
+constexpr int kPackHead = 16 + 64;
+constexpr int kPackWords = kPackHead + 2 * 8 * 8 * kMaxDelta;
 
 constexpr size_t ws_align(size_t n) { return (n + 255) & ~size_t(255); }
 constexpr size_t kWsRec = 0;
@@ -2071,7 +2134,8 @@ constexpr size_t kWsWide = kWsCom + ws_align(sizeof(double) * kCells * 3);
 constexpr size_t kWsPartial = kWsWide + ws_align(sizeof(double) * 8 * kWideMax * kFolded * 64);
 constexpr size_t kWsP2m = kWsPartial + ws_align(sizeof(double) * kRootChunks * kCells * kRecDoubles);
 constexpr size_t kWsMeta = kWsP2m + ws_align(sizeof(double) * kCells * 8);
-constexpr size_t kWsBytes = kWsMeta + ws_align(sizeof(int32_t) * kMetaSize);
+constexpr size_t kWsPacks = kWsMeta + ws_align(sizeof(int32_t) * kMetaSize);
+constexpr size_t kWsBytes = kWsPacks + ws_align(sizeof(int32_t) * kPackWords);
 
 SubgridWorkspace carve_workspace(char* base) {
     SubgridWorkspace w;
@@ -2082,6 +2146,7 @@ SubgridWorkspace carve_workspace(char* base) {
     w.partial = reinterpret_cast<double*>(base + kWsPartial);
     w.p2m = reinterpret_cast<double*>(base + kWsP2m);
     w.meta = reinterpret_cast<int32_t*>(base + kWsMeta);
+    w.packs = reinterpret_cast<int32_t*>(base + kWsPacks);
     return w;
 }
 
@@ -2132,8 +2197,9 @@ struct octofmm_context {
     SubgridWorkspace ws;
     char* d_ws = nullptr;
     char* d_scratch = nullptr;     // this device's `scratch` (set at creation)
-    double* h_pin = nullptr;       // results [512][20], [512][3], then the packed inputs
+    double* h_pin = nullptr;       // results [512][20], [512][3], the packed inputs, p2m work lists
     int reach = 0;                 // cells of a neighbour within the stencil's reach, per axis
+    P2mReach p2m_reach;
 };
 
 // doubles of the results at the front of the pinned memory, and the cells its
@@ -2177,7 +2243,10 @@ struct octofmm_plan {
     int32_t wide_parts = 0;        // variant 704 split further: workgroups per coarse block (0: not for this level)
     double* d_wide = nullptr;      // and their folded sums [n_m2l * 8 * wide_parts][kFolded][64]
     int32_t n_p2m = 0;             // leaf items with p2m: items [n_m2l, n_m2l + n_p2m)
-    double* d_p2m_out = nullptr;   // their p2m sums [n_p2m][512][8]
+    double* d_p2m_out = nullptr;   // their p2m sums [n_p2m][512][8], zeros where a cell has no p2m pair
+    int32_t n_packs = 0;           // p2m work lists (P2mPacks): hdr, units, idx, di
+    int32_t* d_packs = nullptr;
+    size_t packs_units = 0, packs_idx = 0, packs_di = 0;   // first words of the lists behind hdr
     int64_t mixed_far_pairs_by_offset = 0;   // FP32 far pairs under that rule
     int64_t mixed_far_pairs_by_pair = 0;     // and under the per-pair rule of mapping 0
     bool root = false;             // root sub-grid: root stencil over slot 0
@@ -2291,6 +2360,7 @@ void pack_subgrid(octofmm_context* c, const octofmm_subgrid* in, bool leaf_targe
     pa.rho = in->type == OCTOFMM_RHO;
     pa.dx = in->dx;
     for (int k = 0; k < 3; ++k) pa.xbase[k] = in->xbase[k];
+    pa.packs_n = 0;
     size_t at = 0;
     for (int sl = 0; sl < 27; ++sl) {
         pa.off[sl] = 0;
@@ -2358,15 +2428,34 @@ void pack_subgrid(octofmm_context* c, const octofmm_subgrid* in, bool leaf_targe
     }
 }
 
+// The p2m work lists of a packed leaf target, into the pinned memory behind
+// the inputs: hdr, units, idx, di.  Returns the number of packs.
+int pack_p2m(octofmm_context* c, PackedArgs& pa) {
+    P2mPacks pk;
+    build_p2m_packs(c->p2m_reach, 1,
+        [&](int, int raw) { return pa.kind[packed_slot(raw)] == OCTOFMM_SLOT_NONLEAF ? packed_slot(raw) : -1; }, pk);
+    int32_t* dst = reinterpret_cast<int32_t*>(c->h_pin + kPinOut + pin_cells(c->tab) * 23);
+    std::copy(pk.hdr.begin(), pk.hdr.end(), dst);
+    std::copy(pk.units.begin(), pk.units.end(), dst + 16);
+    std::copy(pk.idx.begin(), pk.idx.end(), dst + kPackHead);
+    std::copy(pk.di.begin(), pk.di.end(), dst + kPackHead + pk.idx.size());
+    pa.packs_src = dst;
+    pa.packs_n = kPackHead + 2 * (int)pk.idx.size();
+    return pk.npacks();
+}
+
 // The kernels of one packed sub-grid on the context's stream: its interactions
 // alone go to the results in the pinned memory.
 octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace& w, PackedArgs& pa, bool root) {
     hipStream_t st = c->stream;
+    const int npacks = (pa.item_flags & kItemP2M) ? pack_p2m(c, pa) : 0;
     const bool rho = pa.rho != 0;
     pa.rec = w.rec;
     pa.mon = w.mon;
     pa.com = w.com;
     pa.meta = w.meta;
+    pa.packs = w.packs;
+    pa.p2m = w.p2m;
     hipLaunchKernelGGL(stage_packed, dim3(root ? 4 : 27 * 4), dim3(256), 0, st, pa);
     HIPC(c, hipGetLastError());
     double* L = c->h_pin;
@@ -2408,6 +2497,10 @@ octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace& w, Pac
     la.wide_sums = w.wide;
     la.mon = w.mon;
     la.p2m_out = w.p2m;
+    la.p2m_hdr = w.packs;
+    la.p2m_units = w.packs + 16;
+    la.p2m_idx = w.packs + kPackHead;
+    la.p2m_di = w.packs + kPackHead + (pa.packs_n - kPackHead) / 2;
     la.G = 1.0;
     la.leaf_rows = 1;
     la.overwrite = 1;
@@ -2415,13 +2508,11 @@ octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace& w, Pac
     la.inv_dx = 1.0 / pa.dx;
     la.neg_inv_dx = -1.0 / pa.dx;
     if (pa.item_flags & kItemLeaf) {
-        if (pa.item_flags & kItemP2M) {
-            if (rho)
-                launch_p2m<true>(1, st, la);
-            else
-                launch_p2m<false>(1, st, la);
-            HIPC(c, hipGetLastError());
-        }
+        if (rho)
+            launch_p2m<true>(npacks, st, la, c->tab);
+        else
+            launch_p2m<false>(npacks, st, la, c->tab);
+        HIPC(c, hipGetLastError());
         if (rho)
             launch_leaf<true>(1, st, la, c->tab);
         else
@@ -2500,7 +2591,8 @@ octofmm_status octofmm_create(const octofmm_config* cfg, octofmm_context** out) 
         return OCTOFMM_ERR_THETA;
     }
     if (hipSetDevice(c->device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_pin, sizeof(double) * (kPinOut + pin_cells(c->tab) * 23), hipHostMallocDefault) !=
+        hipHostMalloc((void**)&c->h_pin, sizeof(double) * (kPinOut + pin_cells(c->tab) * 23) + sizeof(int32_t) * kPackWords,
+            hipHostMallocDefault) !=
             hipSuccess ||
         hipMalloc((void**)&c->d_tab, sizeof(Tables)) != hipSuccess ||
         hipMemcpy(c->d_tab, &c->tab, sizeof(Tables), hipMemcpyHostToDevice) != hipSuccess) {
@@ -2508,6 +2600,7 @@ octofmm_status octofmm_create(const octofmm_config* cfg, octofmm_context** out) 
         return OCTOFMM_ERR_HIP;
     }
     c->reach = 2 * c->tab.max_delta;
+    build_p2m_reach(c->tab, c->p2m_reach);
     c->d_scratch = scratch_address(c->device);
     if (!c->d_scratch) {
         octofmm_destroy(c);
@@ -2633,6 +2726,7 @@ static void plan_free(octofmm_plan* p) {
     (void)hipFree(p->d_queue);
     (void)hipFree(p->d_wide);
     (void)hipFree(p->d_p2m_out);
+    (void)hipFree(p->d_packs);
     (void)hipFree(p->d_partial);
     (void)hipFree(p->d_pslots);
     (void)hipFree(p->d_pidx);
@@ -2739,10 +2833,14 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
             // the leaf items with p2m lead the leaf items
             la.nitems = p->n_p2m;
             la.item0 = p->n_m2l;
+            la.p2m_hdr = p->d_packs;
+            la.p2m_units = p->d_packs + p->packs_units;
+            la.p2m_idx = p->d_packs + p->packs_idx;
+            la.p2m_di = p->d_packs + p->packs_di;
             if (rho)
-                launch_p2m<true>(p->n_p2m, st, la);
+                launch_p2m<true>(p->n_packs, st, la, c->tab);
             else
-                launch_p2m<false>(p->n_p2m, st, la);
+                launch_p2m<false>(p->n_packs, st, la, c->tab);
             HIPC(c, hipGetLastError());
         }
         if ((stage_mask & 4) && p->nitems > p->n_m2l) {
@@ -3186,9 +3284,30 @@ static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* 
         hipMalloc((void**)&p->d_wide, sizeof(double) * (size_t)n_m2l * 8 * p->wide_parts * kFolded * 64) != hipSuccess)
         return cleanup(OCTOFMM_ERR_ALLOCATION, "partial sum buffer allocation failed");
     p->n_p2m = (int32_t)buckets[2].size();
-    if (p->n_p2m > 0 &&
-        hipMalloc((void**)&p->d_p2m_out, sizeof(double) * (size_t)p->n_p2m * kCells * 8) != hipSuccess)
-        return cleanup(OCTOFMM_ERR_ALLOCATION, "p2m sum buffer allocation failed");
+    if (p->n_p2m > 0) {
+        const size_t bytes = sizeof(double) * (size_t)p->n_p2m * kCells * 8;
+        P2mPacks pk;
+        build_p2m_packs(c->p2m_reach, p->n_p2m,
+            [&](int o, int raw) {
+                const int n = lv->neighbors[(size_t)buckets[2][o].x * 27 + raw];
+                return n >= 0 && lv->kind[n] == OCTOFMM_SLOT_NONLEAF ? n : -1;
+            },
+            pk);
+        p->n_packs = pk.npacks();
+        std::vector<int32_t> all(pk.hdr);
+        p->packs_units = all.size();
+        all.insert(all.end(), pk.units.begin(), pk.units.end());
+        p->packs_idx = all.size();
+        all.insert(all.end(), pk.idx.begin(), pk.idx.end());
+        p->packs_di = all.size();
+        if (!T.p2p_cube) all.insert(all.end(), pk.di.begin(), pk.di.end());
+        if (hipMalloc((void**)&p->d_p2m_out, bytes) != hipSuccess ||
+            hipMalloc((void**)&p->d_packs, sizeof(int32_t) * std::max<size_t>(1, all.size())) != hipSuccess)
+            return cleanup(OCTOFMM_ERR_ALLOCATION, "p2m buffer allocation failed");
+        if (hipMemset(p->d_p2m_out, 0, bytes) != hipSuccess ||
+            hipMemcpy(p->d_packs, all.data(), sizeof(int32_t) * all.size(), hipMemcpyHostToDevice) != hipSuccess)
+            return cleanup(OCTOFMM_ERR_HIP, "p2m work list upload failed");
+    }
     if (!pslots.empty()) {
         if (hipMalloc((void**)&p->d_pidx, sizeof(int2) * std::max<size_t>(1, pidx.size())) != hipSuccess ||
             hipMalloc((void**)&p->d_pslots, sizeof(PartialSlot) * pslots.size()) != hipSuccess)

@@ -624,6 +624,14 @@ struct StageArgs {
     int32_t rho;            // record form: RHO or DRHODT octupole fields
 };
 
+// Levels of one stage_records launch, and the most slots (of 4 workgroups each)
+// of levels that share one: four workgroups a CU, one round of the chip.
+constexpr int kStageLevels = 4;
+constexpr int kStageTogether = 256;
+struct StageGroup {
+    StageArgs a[kStageLevels];
+};
+
 struct LevelArgs {
     const double* rec;      // partner records
     const double* com;      // input centres of mass (leaf targets)

@@ -156,9 +156,14 @@ __device__ __forceinline__ void load_rows(const double* M, const double* com, in
     }
 }
 
-__global__ __launch_bounds__(256) void stage_records(StageArgs a) {
+// One launch stages up to kStageLevels levels, one after another: the levels
+// of a tree that are too small to fill the chip share one (tree_launch).
+__global__ __launch_bounds__(256) void stage_records(StageGroup g) {
     __shared__ double s_row[128 * kStageRow];
-    const int si = blockIdx.x >> 2, q = blockIdx.x & 3;
+    int si = blockIdx.x >> 2, lvl = 0;
+    const int q = blockIdx.x & 3;
+    while (lvl < kStageLevels - 1 && si >= g.a[lvl].nslots) si -= g.a[lvl++].nslots;   // uniform
+    const StageArgs& a = g.a[lvl];
     if (si >= a.nslots) return;                // uniform per block
     const int slot = a.list ? a.list[si] : si;
     const int k = a.kind[slot];
@@ -1643,10 +1648,37 @@ int wide_parts(int n, const Tables& tab) {
     return parts >= 2 ? parts : 0;
 }
 
-template <bool RHO>
-void launch_wide(int nitems, hipStream_t st, const LevelArgs& la) {
-    hipLaunchKernelGGL(level_kernel_wide<RHO>, dim3(nitems * 8 * la.parts), dim3(256), 0, st, la);
-    hipLaunchKernelGGL(level_reduce<RHO>, dim3(nitems * 8), dim3(64), 0, st, la);
+// Bytes of level_kernel_wide's sums.
+size_t wide_bytes(int n, int parts) { return sizeof(double) * (size_t)n * 8 * parts * kFolded * 64; }
+
+void launch_wide_sums(int nitems, hipStream_t st, const LevelArgs& la, bool rho) {
+    const dim3 grid(nitems * 8 * la.parts);
+    if (rho)
+        hipLaunchKernelGGL(level_kernel_wide<true>, grid, dim3(256), 0, st, la);
+    else
+        hipLaunchKernelGGL(level_kernel_wide<false>, grid, dim3(256), 0, st, la);
+}
+
+void launch_wide_reduce(int nitems, hipStream_t st, const LevelArgs& la, bool rho) {
+    if (rho)
+        hipLaunchKernelGGL(level_reduce<true>, dim3(nitems * 8), dim3(64), 0, st, la);
+    else
+        hipLaunchKernelGGL(level_reduce<false>, dim3(nitems * 8), dim3(64), 0, st, la);
+}
+
+// In a whole-tree solve the levels of up to 96 targets (three workgroups a CU)
+// run sums first: level_kernel_wide needs only the level's records, so the
+// sums of the coarse levels, the root's among them, run side by side, and of
+// the chain from level to level only level_reduce with its downward pass is
+// left (329-sub-grid tree: 160 -> 125 us a solve, 10,697: 1338 -> 1307; the sums
+// of a level of 8 targets take 11 us beside those of 32 and the reduction 6,
+// where the level kernels took 22 and 30 one after the other).  Larger levels
+// fill the chip by themselves, and their sums would cost as much traffic as
+// their results.  Workgroups per coarse block of such a level, 0 for a larger
+// one.
+int sums_first_parts(int n, const Tables& tab) {
+    if (n <= 0 || n > 96) return 0;
+    return std::max(1, std::min((tab.nsched + 3) / 4, 96 / n));
 }
 
 // Persistent form of the mapping-7 kernel (variants 804, 802): a grid of
@@ -1742,8 +1774,10 @@ void launch_level(int variant, int nitems, hipStream_t st, const LevelArgs& la, 
         hipLaunchKernelGGL((level_kernel_split<RHO, 4>), dim3(nitems * 8), dim3(256), 0, st, la);
         break;
     case 704:
-        if (la.parts > 1)
-            launch_wide<RHO>(nitems, st, la);
+        if (la.parts > 1) {
+            launch_wide_sums(nitems, st, la, RHO);
+            launch_wide_reduce(nitems, st, la, RHO);
+        }
         else
             hipLaunchKernelGGL((level_kernel_dsplit<RHO, 4>), dim3(nitems * 8), dim3(256), 0, st, la);
         break;
@@ -2215,6 +2249,8 @@ struct octofmm_plan {
     int32_t nslots = 0, nitems = 0, type = 0, precision = 0, flags = 0;
     int32_t n_m2l = 0;             // items [0, n_m2l) are non-leaf, the rest leaf targets
     int32_t n_stage = 0;           // slots whose partner records some item reads
+    int32_t stage_slots() const { return d_stage_list ? n_stage : nslots; }
+    bool sums_first = false;       // whole-tree solve: level_kernel_wide and level_reduce launched apart
     int32_t* d_stage_list = nullptr;   // those slots, or null when all are read
     double dx = 0.0;
     const double* d_M = nullptr;
@@ -2734,8 +2770,38 @@ static void plan_free(octofmm_plan* p) {
     delete p;
 }
 
+// Stages the records of n <= kStageLevels plans in one launch.
+static octofmm_status launch_stage(octofmm_context* c, hipStream_t st, octofmm_plan* const* plans, int n) {
+    StageGroup g;
+    int slots = 0;
+    for (int i = 0; i < kStageLevels; ++i) {
+        StageArgs& sa = g.a[i];
+        const octofmm_plan* p = plans[i < n ? i : 0];
+        sa.M = p->d_M;
+        sa.com = p->d_com;
+        sa.mon = p->d_mon;
+        sa.kind = p->d_kind;
+        sa.fxbase = p->d_fxbase;
+        sa.foff = p->d_foff;
+        sa.rec = p->d_rec;
+        sa.recm = p->d_recm;
+        sa.rho = p->type == OCTOFMM_RHO;
+        sa.list = p->d_stage_list;
+        sa.dx = p->dx;
+        sa.nslots = i >= n ? 0 : p->stage_slots();
+        slots += sa.nslots;
+    }
+    if (slots > 0) {
+        hipLaunchKernelGGL(stage_records, dim3(slots * 4), dim3(256), 0, st, g);
+        HIPC(c, hipGetLastError());
+    }
+    return OCTOFMM_OK;
+}
+
 // stage_mask bit 0: stage the partner records; bit 1: the root kernel, or the
-// level kernel over the multipole-target items; bit 2: the leaf kernel over
+// level kernel over the multipole-target items (a sums-first level: what
+// level_reduce does of it); bit 4: a sums-first level's level_kernel_wide,
+// which goes before bit 1; bit 2: the leaf kernel over
 // the monopole-target items; bit 3: the p2m kernel of the leaf items with
 // refined neighbours, whose sums the leaf kernel reads (so bit 3 goes before
 // bit 2, on the same stream or ordered before it).  Bits 1 and 2 write
@@ -2748,23 +2814,8 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         HIPC(c, hipGetLastError());
     }
     if (stage_mask & 1) {
-        StageArgs sa;
-        sa.M = p->d_M;
-        sa.com = p->d_com;
-        sa.mon = p->d_mon;
-        sa.kind = p->d_kind;
-        sa.fxbase = p->d_fxbase;
-        sa.foff = p->d_foff;
-        sa.rec = p->d_rec;
-        sa.recm = p->d_recm;
-        sa.rho = p->type == OCTOFMM_RHO;
-        sa.list = p->d_stage_list;
-        sa.dx = p->dx;
-        sa.nslots = p->d_stage_list ? p->n_stage : p->nslots;
-        if (sa.nslots > 0) {
-            hipLaunchKernelGGL(stage_records, dim3(sa.nslots * 4), dim3(256), 0, st, sa);
-            HIPC(c, hipGetLastError());
-        }
+        const octofmm_status s = launch_stage(c, st, &p, 1);
+        if (s != OCTOFMM_OK) return s;
     }
     if ((stage_mask & 2) && p->root) {
         RootArgs ra;
@@ -2787,7 +2838,7 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         rr.overwrite = p->l2l ? 1 : 0;
         hipLaunchKernelGGL(root_reduce, dim3((kCells * 23 + 255) / 256), dim3(256), 0, st, rr);
         HIPC(c, hipGetLastError());
-    } else if (!p->root && (stage_mask & 14) && p->nitems > 0) {
+    } else if (!p->root && (stage_mask & 30) && p->nitems > 0) {
         LevelArgs la;
         la.rec = p->d_rec;
         la.com = p->d_com;
@@ -2820,10 +2871,13 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         la.inv_dx = 1.0 / p->dx;
         la.neg_inv_dx = -1.0 / p->dx;
         const bool rho = p->type == OCTOFMM_RHO;
-        if ((stage_mask & 2) && p->n_m2l > 0) {
+        if ((stage_mask & 18) && p->n_m2l > 0) {
             la.nitems = p->n_m2l;
             la.item0 = 0;
-            if (rho)
+            if (p->sums_first) {
+                if (stage_mask & 16) launch_wide_sums(p->n_m2l, st, la, rho);
+                if (stage_mask & 2) launch_wide_reduce(p->n_m2l, st, la, rho);
+            } else if (rho)
                 launch_level<true>(p->variant, p->n_m2l, st, la, p->precision == OCTOFMM_PRECISION_MIXED);
             else
                 launch_level<false>(p->variant, p->n_m2l, st, la, p->precision == OCTOFMM_PRECISION_MIXED);
@@ -3073,7 +3127,7 @@ static octofmm_status plan_autotune_run(octofmm_plan* p) {
 
 // First half of level plan creation: checks, work items, pair counts, device
 // tables.  The kernel variant and the graph come in level_plan_finish.
-static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* lv, octofmm_plan** out) {
+static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* lv, bool in_tree, octofmm_plan** out) {
     if (lv->nslots <= 0 || !lv->neighbors || !lv->kind || !lv->xbase || lv->ntargets < 0 ||
         (lv->ntargets > 0 && !lv->targets))
         return fail(c, OCTOFMM_ERR_INVALID_ARGUMENT, "bad level description");
@@ -3279,9 +3333,17 @@ static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* 
         return cleanup(OCTOFMM_ERR_ALLOCATION, "root partial buffer allocation failed");
     if (!root && hipMalloc((void**)&p->d_queue, sizeof(uint32_t) * 8) != hipSuccess)
         return cleanup(OCTOFMM_ERR_ALLOCATION, "work counter allocation failed");
-    if (!root && p->precision == OCTOFMM_PRECISION_FP64) p->wide_parts = wide_parts(n_m2l, T);
+    if (!root && p->precision == OCTOFMM_PRECISION_FP64) {
+        // (a forced variant runs its plain form in a tree, too)
+        if (in_tree && !std::getenv("OCTOFMM_VARIANT")) {
+            p->wide_parts = sums_first_parts(n_m2l, T);
+            p->sums_first = p->wide_parts > 0;
+            if (p->sums_first) p->variant = 704;
+        }
+        if (!p->sums_first) p->wide_parts = wide_parts(n_m2l, T);
+    }
     if (p->wide_parts > 0 &&
-        hipMalloc((void**)&p->d_wide, sizeof(double) * (size_t)n_m2l * 8 * p->wide_parts * kFolded * 64) != hipSuccess)
+        hipMalloc((void**)&p->d_wide, wide_bytes(n_m2l, p->wide_parts)) != hipSuccess)
         return cleanup(OCTOFMM_ERR_ALLOCATION, "partial sum buffer allocation failed");
     p->n_p2m = (int32_t)buckets[2].size();
     if (p->n_p2m > 0) {
@@ -3452,7 +3514,7 @@ octofmm_status octofmm_level_plan_create(octofmm_context* c, const octofmm_level
     if (!lv || !out) return fail(c, OCTOFMM_ERR_INVALID_ARGUMENT, "null level or plan");
     *out = nullptr;
     octofmm_plan* p = nullptr;
-    octofmm_status s = level_plan_build(c, lv, &p);
+    octofmm_status s = level_plan_build(c, lv, false, &p);
     if (s != OCTOFMM_OK) return s;
     s = level_plan_finish(p, lv->flags);
     if (s != OCTOFMM_OK) return s;
@@ -3533,10 +3595,10 @@ struct octofmm_tree_plan {
         double* L = nullptr;
         double* Lc = nullptr;
         double* g = nullptr;
+        double* d_xbase = nullptr;    // the node tables: one block
         int32_t* d_kind = nullptr;
         int32_t* d_parent = nullptr;
         int32_t* d_octant = nullptr;
-        double* d_xbase = nullptr;
         octofmm_plan* plan = nullptr;
     };
     octofmm_context* ctx = nullptr;
@@ -3547,12 +3609,12 @@ struct octofmm_tree_plan {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     // the interactions phase forks onto three more streams: one stages the
-    // partner records of every level, coarsest first, the other two run the
-    // leaf kernels of alternate levels (the leaf kernel of level l + 1 need not
-    // wait for that of level l); the level kernels stay on the caller's stream
+    // partner records of every level, coarsest first; of the other two [0] runs
+    // the leaf kernels and [1] p2m, and both the sums of sums-first levels; the
+    // level kernels stay on the caller's stream
     hipStream_t side_stage = nullptr, side_leaf[2] = {nullptr, nullptr};
     hipEvent_t ev_up = nullptr, ev_join_stage = nullptr, ev_join_leaf[2] = {nullptr, nullptr};
-    std::vector<hipEvent_t> ev_stage, ev_level;
+    std::vector<hipEvent_t> ev_stage, ev_level, ev_sums, ev_p2m;
 };
 
 namespace {
@@ -3567,15 +3629,14 @@ void tree_free(octofmm_tree_plan* t) {
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : t->ev_level)
         if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : t->ev_sums)
+        if (e) (void)hipEventDestroy(e);
     if (t->side_stage) (void)hipStreamDestroy(t->side_stage);
     for (hipStream_t s : t->side_leaf)
         if (s) (void)hipStreamDestroy(s);
     for (auto& l : t->lv) {
         plan_free(l.plan);
-        (void)hipFree(l.d_kind);
-        (void)hipFree(l.d_parent);
-        (void)hipFree(l.d_octant);
-        (void)hipFree(l.d_xbase);
+        (void)hipFree(l.d_xbase);   // and the tables behind it
     }
     delete t;
 }
@@ -3588,6 +3649,7 @@ octofmm_status tree_launch(octofmm_tree_plan* t, hipStream_t st, int phases) {
     if (phases & 1)
         for (int l = nl - 1; l >= 0; --l) {
             const auto& L = t->lv[l];
+            if (l == 0 && t->lv[0].plan && t->lv[0].plan->root) continue;   // a refined root has no parent to sum into
             M2MArgs a;
             a.M = L.M;
             a.com = L.com;
@@ -3608,32 +3670,54 @@ octofmm_status tree_launch(octofmm_tree_plan* t, hipStream_t st, int phases) {
     // write the final expansions (the downward pass is fused into them), so
     // both kernels of level l read the finished non-leaf sub-grids of level
     // l - 1, which only the level kernel of l - 1 writes: the leaf kernel of
-    // level l waits for that kernel and for its own level's records, and
-    // overlaps the level kernels that follow.  Staging depends only on the
-    // upward pass.
+    // level l waits for that kernel and for its own p2m, and overlaps the level
+    // kernels that follow.  Staging depends only on the upward pass, p2m and
+    // the small levels' sums (sums_first_parts) only on staging: they fill the
+    // chip while the coarse levels, too small for that, pass one after another.
     if (phases & 2) {
         hipStream_t ss = t->side_stage;
         HIPC(c, hipEventRecord(t->ev_up, st));
         HIPC(c, hipStreamWaitEvent(ss, t->ev_up, 0));
         for (hipStream_t sl : t->side_leaf) HIPC(c, hipStreamWaitEvent(sl, t->ev_up, 0));
-        for (int l = 0; l < nl; ++l) {
-            const octofmm_status s = plan_launch(t->lv[l].plan, ss, 1);
+        for (int l = 0; l < nl;) {
+            // levels that one round of workgroups stages go in one launch
+            octofmm_plan* group[kStageLevels];
+            int n = 0, slots = 0;
+            while (n < kStageLevels && l + n < nl &&
+                (n == 0 || slots + t->lv[l + n].plan->stage_slots() <= kStageTogether)) {
+                group[n] = t->lv[l + n].plan;
+                slots += group[n++]->stage_slots();
+            }
+            const octofmm_status s = launch_stage(c, ss, group, n);
             if (s != OCTOFMM_OK) return s;
-            HIPC(c, hipEventRecord(t->ev_stage[l], ss));
+            for (; n > 0; --n, ++l) HIPC(c, hipEventRecord(t->ev_stage[l], ss));
+        }
+        // what needs only a level's records: the sums of the small levels and
+        // every level's p2m, ahead of all that waits for a level above
+        for (int l = 0; l < nl; ++l) {
+            octofmm_plan* p = t->lv[l].plan;
+            if (p->sums_first) {
+                hipStream_t sl = t->side_leaf[l & 1];
+                HIPC(c, hipStreamWaitEvent(sl, t->ev_stage[l], 0));
+                const octofmm_status s = plan_launch(p, sl, 16);
+                if (s != OCTOFMM_OK) return s;
+                HIPC(c, hipEventRecord(t->ev_sums[l], sl));
+            }
+            if (p->n_p2m == 0) continue;
+            HIPC(c, hipStreamWaitEvent(t->side_leaf[1], t->ev_stage[l], 0));
+            const octofmm_status s = plan_launch(p, t->side_leaf[1], 8);
+            if (s != OCTOFMM_OK) return s;
+            HIPC(c, hipEventRecord(t->ev_p2m[l], t->side_leaf[1]));
         }
         for (int l = 0; l < nl; ++l) {
             octofmm_plan* p = t->lv[l].plan;
-            HIPC(c, hipStreamWaitEvent(st, t->ev_stage[l], 0));
+            HIPC(c, hipStreamWaitEvent(st, p->sums_first ? t->ev_sums[l] : t->ev_stage[l], 0));
             octofmm_status s = plan_launch(p, st, 2);
             if (s != OCTOFMM_OK) return s;
             HIPC(c, hipEventRecord(t->ev_level[l], st));
             if (!p->root && p->nitems > p->n_m2l) {
-                // the p2m sums need only this level's records; the leaf
-                // kernel also needs the finished level above
-                hipStream_t sl = t->side_leaf[l & 1];
-                HIPC(c, hipStreamWaitEvent(sl, t->ev_stage[l], 0));
-                s = plan_launch(p, sl, 8);
-                if (s != OCTOFMM_OK) return s;
+                hipStream_t sl = t->side_leaf[0];
+                if (p->n_p2m > 0) HIPC(c, hipStreamWaitEvent(sl, t->ev_p2m[l], 0));
                 if (l > 0) HIPC(c, hipStreamWaitEvent(sl, t->ev_level[l - 1], 0));
                 s = plan_launch(p, sl, 4);
                 if (s != OCTOFMM_OK) return s;
@@ -3717,6 +3801,8 @@ octofmm_status octofmm_tree_plan_create(octofmm_context* c, const octofmm_tree* 
     t->lv.resize(nl);
     t->ev_stage.assign(nl, nullptr);
     t->ev_level.assign(nl, nullptr);
+    t->ev_sums.assign(nl, nullptr);
+    t->ev_p2m.assign(nl, nullptr);
     auto cleanup = [&](octofmm_status s, const char* what) {
         tree_free(t);
         return fail(c, s, "%s", what);
@@ -3729,7 +3815,9 @@ octofmm_status octofmm_tree_plan_create(octofmm_context* c, const octofmm_tree* 
             ok = ok && hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess;
         for (int l = 0; l < nl; ++l)
             ok = ok && hipEventCreateWithFlags(&t->ev_stage[l], hipEventDisableTiming) == hipSuccess &&
-                 hipEventCreateWithFlags(&t->ev_level[l], hipEventDisableTiming) == hipSuccess;
+                 hipEventCreateWithFlags(&t->ev_level[l], hipEventDisableTiming) == hipSuccess &&
+                 hipEventCreateWithFlags(&t->ev_sums[l], hipEventDisableTiming) == hipSuccess &&
+                 hipEventCreateWithFlags(&t->ev_p2m[l], hipEventDisableTiming) == hipSuccess;
         if (!ok) return cleanup(OCTOFMM_ERR_HIP, "tree stream or event creation failed");
     }
     for (int l = 0; l < nl; ++l) {
@@ -3744,15 +3832,20 @@ octofmm_status octofmm_tree_plan_create(octofmm_context* c, const octofmm_tree* 
         D.Lc = L.d_L_c;
         D.g = L.d_g;
         const size_t n = (size_t)L.nnodes;
-        if (hipMalloc((void**)&D.d_kind, sizeof(int32_t) * n) != hipSuccess ||
-            hipMalloc((void**)&D.d_parent, sizeof(int32_t) * n) != hipSuccess ||
-            hipMalloc((void**)&D.d_octant, sizeof(int32_t) * n) != hipSuccess ||
-            hipMalloc((void**)&D.d_xbase, sizeof(double) * 3 * n) != hipSuccess)
+        // one block: xbase, kind, parent, octant
+        std::vector<double> tables((3 * n * sizeof(double) + 3 * n * sizeof(int32_t) + 7) / 8);
+        std::copy(L.xbase, L.xbase + 3 * n, tables.begin());
+        int32_t* ti = reinterpret_cast<int32_t*>(tables.data() + 3 * n);
+        std::copy(L.kind, L.kind + n, ti);
+        std::copy(L.parent, L.parent + n, ti + n);
+        std::copy(L.octant, L.octant + n, ti + 2 * n);
+        const size_t bytes = tables.size() * sizeof(double);
+        if (hipMalloc((void**)&D.d_xbase, bytes) != hipSuccess)
             return cleanup(OCTOFMM_ERR_ALLOCATION, "tree table allocation failed");
-        if (hipMemcpy(D.d_kind, L.kind, sizeof(int32_t) * n, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(D.d_parent, L.parent, sizeof(int32_t) * n, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(D.d_octant, L.octant, sizeof(int32_t) * n, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(D.d_xbase, L.xbase, sizeof(double) * 3 * n, hipMemcpyHostToDevice) != hipSuccess)
+        D.d_kind = reinterpret_cast<int32_t*>(D.d_xbase + 3 * n);
+        D.d_parent = D.d_kind + n;
+        D.d_octant = D.d_parent + n;
+        if (hipMemcpy(D.d_xbase, tables.data(), bytes, hipMemcpyHostToDevice) != hipSuccess)
             return cleanup(OCTOFMM_ERR_HIP, "tree table upload failed");
         t->stats.nodes += L.nnodes;
         for (int i = 0; i < L.nnodes; ++i) t->stats.leaves += L.kind[i] == OCTOFMM_SLOT_LEAF;
@@ -3795,7 +3888,7 @@ octofmm_status octofmm_tree_plan_create(octofmm_context* c, const octofmm_tree* 
         // the level's plan is tuned only once its epilogue is the fused
         // downward pass it runs with in the solve
         octofmm_plan* lp = nullptr;
-        octofmm_status s = level_plan_build(c, &lv, &lp);
+        octofmm_status s = level_plan_build(c, &lv, true, &lp);
         if (s == OCTOFMM_OK) {
             lp->l2l = true;
             lp->t_parent = t->lv[l].d_parent;
@@ -3807,7 +3900,7 @@ octofmm_status octofmm_tree_plan_create(octofmm_context* c, const octofmm_tree* 
             lp->t_G = t->G;
             lp->t_correct_am = t->correct_am;
             lp->leaf_rows = (tr->flags & OCTOFMM_TREE_LEAF_G_ONLY) ? 0 : 1;
-            s = level_plan_finish(lp, lv.flags);
+            s = level_plan_finish(lp, lp->sums_first ? 0 : lv.flags);
         }
         if (s != OCTOFMM_OK) {
             const std::string msg = c->err;

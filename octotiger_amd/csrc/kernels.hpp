@@ -635,6 +635,8 @@ struct StageGroup {
 struct LevelArgs {
     const double* rec;      // partner records
     const double* com;      // input centres of mass (leaf targets)
+    const double* xbase;    // [nslots][3] and cell size, whole-tree solves
+    double dx;
     double* L;
     double* Lc;
     const int32_t* nbr;     // [nslots][27]

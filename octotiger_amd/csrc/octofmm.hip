@@ -375,6 +375,12 @@ __device__ __forceinline__ int partner_base(const LaneGeom& g, int ax, int ay, i
     return ((px & 3) * 16 + (py & 3) * 4 + (pz & 3)) * 8;
 }
 
+// geometric centre xbase + i*dx, rounded as written (grid_fmm.cpp:1669-1671)
+__device__ __forceinline__ double cell_centre(double xb, int i, double dx) {
+#pragma clang fp contract(off)
+    return xb + (double)i * dx;
+}
+
 // Result of one target cell.  Level plans accumulate L (ncomp components:
 // 20 for M2L targets, 4 for leaves) and overwrite L_c when the kernel forms
 // it (write_c).  In a whole-tree solve the cell's final expansion is written
@@ -1235,19 +1241,26 @@ __device__ __forceinline__ void p2p_cube(const double* s_win, int Cx, int Cy, in
 //
 // In a whole-tree solve the final rows (L 20, L_c 3, g 4 doubles a cell) go
 // through LDS and leave as the sub-grid's contiguous blocks, consecutive lanes
-// in consecutive 16-byte chunks: the L rows of kx = 0 (the even x planes, 40
-// KiB), then those of kx = 1, then L_c and g together.  Written straight from
-// the lanes each store would touch 64 rows.  Each staged row, L_c triple and
-// g quadruple is shifted by one more element every 16 cells: without that the
+// in consecutive 16-byte chunks: the L rows of two x planes at a time (20 KiB),
+// with the first of them L_c and g of 256 cells.  Written straight from the
+// lanes each store would touch 64 rows.  Each staged row, L_c triple and g
+// quadruple is shifted by one more element every 16 cells: without that the
 // lanes' rows (2 cells apart in z, 16 in y) fall on a quarter of the banks.
+//
+// A leaf alternates between waiting for its window, FP64 work and 110 KiB of
+// stores; alone on the chip 5568 leaves take 200 us, 3.4 TB/s with the VALU a
+// third busy, so what counts is how many leaves share a CU.  The staging fits in
+// the window's 35 KiB and the kernel in 128 registers, so 4 do (a staging of
+// all even or odd planes at once, 40 KiB, left room for 3): a solve of 9361
+// leaves takes 1290 us in place of 1313.
 template <bool RHO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void leaf_cube_kernel(LevelArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void leaf_cube_kernel(LevelArgs a) {
     extern __shared__ double s_win[];
     __shared__ int s_nbr[27];
     __shared__ int s_kind[27];
     const int ordinal = xcd_item(blockIdx.x, gridDim.x);
     const int2 it = a.items[a.item0 + ordinal];
-    const int slot = it.x;
+    const int slot = __builtin_amdgcn_readfirstlane(it.x);
     const int th = threadIdx.x;
     if (th < 27) {
         const int n = a.nbr[(size_t)slot * 27 + th];
@@ -1301,19 +1314,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void l
     const int cell0 = Cx * 128 + (2 * Cy + ky) * 8 + 2 * Cz + kz;   // kx = 0; kx = 1 is 64 further
     const double s1 = a.inv_dx * a.neg_inv_dx;
     const bool p2m = (it.y & kItemP2M) != 0;
-    double L[2][4], C[2][3];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        L[t][0] = s[t].p * a.inv_dx;
-        L[t][1] = s[t].x * s1;
-        L[t][2] = s[t].y[0] * s1;
-        L[t][3] = s[t].z[0] * s1;
-        C[t][0] = C[t][1] = C[t][2] = 0.0;
-        if (p2m) add_p2m(a, ordinal, cell0 + 64 * t, L[t], C[t]);
-    }
+    auto sums = [&](int t, double* L, double* C) {
+        L[0] = s[t].p * a.inv_dx;
+        L[1] = s[t].x * s1;
+        L[2] = s[t].y[0] * s1;
+        L[3] = s[t].z[0] * s1;
+        C[0] = C[1] = C[2] = 0.0;
+        if (p2m) add_p2m(a, ordinal, cell0 + 64 * t, L, C);
+    };
     if (!a.l2l) {   // uniform
 #pragma unroll
-        for (int t = 0; t < 2; ++t) finish_cell<RHO>(a, slot, cell0 + 64 * t, L[t], 4, C[t], p2m, true);
+        for (int t = 0; t < 2; ++t) {
+            double L[4], C[3];
+            sums(t, L, C);
+            finish_cell<RHO>(a, slot, cell0 + 64 * t, L, 4, C, p2m, true);
+        }
         return;
     }
     // both targets lie in one parent cell
@@ -1336,65 +1351,83 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void l
             if (RHO) lc[d] = a.pLc[pr * 3 + d];
         }
     }
+    // staged: L rows of 128 cells, L_c and g of 256, each shifted by one more
+    // element every 16 cells
     double2* b2 = reinterpret_cast<double2*>(s_win);
-    double Cf[2][3], g4[2][4];
+    double* bc = s_win + 128 * 20 + 16;
+    double2* bg = reinterpret_cast<double2*>(bc + 256 * 3 + 16);
+    const int r = Cx * 64 + (cell0 & 63);   // cell r + 64 (r / 64 + kx)
+    double2* row = b2 + (r & 127) * 10 + ((r & 127) >> 4);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const double* X = a.com + ((size_t)slot * kCells + cell0 + 64 * t) * 3;
-        const double dX[3] = {X[0] - Y[0], X[1] - Y[1], X[2] - Y[2]};
-        double Lf[20];
+        double dX[3];
+        if constexpr (RHO) {
+            // the centres the upward pass of this solve stored (12 KiB a leaf), formed again
+            const auto* xb = as_const(a.xbase) + 3 * slot;
+            dX[0] = cell_centre(xb[0], 2 * Cx + t, a.dx) - Y[0];
+            dX[1] = cell_centre(xb[1], 2 * Cy + ky, a.dx) - Y[1];
+            dX[2] = cell_centre(xb[2], 2 * Cz + kz, a.dx) - Y[2];
+        } else {
+            const double* X = a.com + ((size_t)slot * kCells + cell0 + 64 * t) * 3;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) dX[d] = X[d] - Y[d];
+        }
+        double L[4], C[3], Lf[20], Cf[3], g4[4];
+        sums(t, L, C);
         local_shift(A, dX, Lf);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) Lf[j] += L[t][j];
+        for (int j = 0; j < 4; ++j) Lf[j] += L[j];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) Cf[t][d] = RHO ? C[t][d] + lc[d] : 0.0;
-        leaf_force<RHO>(a, Lf, Cf[t], g4[t]);
-        if (a.leaf_rows) {   // uniform
-            __syncthreads();   // the window (then the rows before) read
-            const int r = Cx * 64 + (cell0 & 63);
-            double2* row = b2 + r * 10 + (r >> 4);
+        for (int d = 0; d < 3; ++d) Cf[d] = RHO ? C[d] + lc[d] : 0.0;
+        leaf_force<RHO>(a, Lf, Cf, g4);
+        if constexpr (!RHO) {   // phi slot only
+            if (a.g) a.g[((size_t)slot * kCells + cell0 + 64 * t) * 4] = g4[0];
+        }
+        __syncthreads();   // the window (then the rows before) read
+        if constexpr (RHO) {
+            double* c = bc + r * 3 + (r >> 4);
+            c[0] = Cf[0];
+            c[1] = Cf[1];
+            c[2] = Cf[2];
+            double2* g = bg + r * 2 + (r >> 4);
+            g[0] = make_double2(g4[0], g4[1]);
+            g[1] = make_double2(g4[2], g4[3]);
+        }
+        double2* dst = reinterpret_cast<double2*>(a.L + (size_t)slot * kCells * 20) + 640 * t;
 #pragma unroll
-            for (int j = 0; j < 10; ++j) row[j] = make_double2(Lf[2 * j], Lf[2 * j + 1]);
-            __syncthreads();
-            double2* dst = reinterpret_cast<double2*>(a.L + (size_t)slot * kCells * 20) + 640 * t;
+        for (int h = 0; h < 2; ++h) {
+            if (a.leaf_rows) {   // uniform
+                if (h == 1) __syncthreads();
+                if ((Cx >> 1) == h) {
 #pragma unroll
-            for (int i = 0; i < 10; ++i) {   // 256 rows x 10 chunks; row r is cell r + 64 (r / 64 + kx)
-                const int ch = th + 256 * i;
-                store_stream(dst + ch + ch / 640 * 640, b2[ch + (ch / 160)]);
+                    for (int j = 0; j < 10; ++j) row[j] = make_double2(Lf[2 * j], Lf[2 * j + 1]);
+                }
+            }
+            if (a.leaf_rows || h == 0) __syncthreads();
+            if (a.leaf_rows) {
+#pragma unroll
+                for (int i = 0; i < 5; ++i) {   // 128 rows x 10 chunks
+                    const int ch = th + 256 * i;
+                    store_stream(dst + h * 2560 + ch + ch / 640 * 640, b2[ch + ch / 160]);
+                }
+            }
+            if (RHO && h == 0) {
+                double2* lcd = reinterpret_cast<double2*>(a.Lc + (size_t)slot * kCells * 3) + 96 * t;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {   // 384 chunks: doubles 2 ch and 2 ch + 1
+                    const int ch = th + 256 * i, d0 = 2 * ch + ch / 24;
+                    if (ch < 384) store_stream(lcd + ch + ch / 96 * 96, make_double2(bc[d0], bc[d0 + 1]));
+                }
+                if (a.g) {   // uniform
+                    double2* gg = reinterpret_cast<double2*>(a.g + (size_t)slot * kCells * 4) + 128 * t;
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {   // 512 chunks
+                        const int ch = th + 256 * i;
+                        store_stream(gg + ch + ch / 128 * 128, bg[ch + (ch >> 5)]);
+                    }
+                }
             }
         }
-    }
-    if constexpr (RHO) {
-        __syncthreads();
-        double* buf = s_win;
-        double2* bg = b2 + 784;   // after the 1536 + 32 doubles of L_c
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int cell = cell0 + 64 * t;
-            buf[cell * 3 + (cell >> 4) + 0] = Cf[t][0];
-            buf[cell * 3 + (cell >> 4) + 1] = Cf[t][1];
-            buf[cell * 3 + (cell >> 4) + 2] = Cf[t][2];
-            bg[cell * 2 + (cell >> 4)] = make_double2(g4[t][0], g4[t][1]);
-            bg[cell * 2 + (cell >> 4) + 1] = make_double2(g4[t][2], g4[t][3]);
-        }
-        __syncthreads();
-        double2* lcd = reinterpret_cast<double2*>(a.Lc + (size_t)slot * kCells * 3);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {   // 768 chunks: doubles 2 ch and 2 ch + 1 of the L_c block
-            const int ch = th + 256 * i, d0 = 2 * ch, d1 = d0 + 1;
-            store_stream(lcd + ch, make_double2(buf[d0 + d0 / 48], buf[d1 + d1 / 48]));
-        }
-        if (a.g) {   // uniform
-            double2* gg = reinterpret_cast<double2*>(a.g + (size_t)slot * kCells * 4);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {   // 1024 chunks (cell = chunk / 2)
-                const int ch = th + 256 * i;
-                store_stream(gg + ch, bg[ch + (ch >> 5)]);
-            }
-        }
-    } else if (a.g) {   // phi slot only
-#pragma unroll
-        for (int t = 0; t < 2; ++t) a.g[((size_t)slot * kCells + cell0 + 64 * t) * 4] = g4[t][0];
     }
 }
 
@@ -1533,9 +1566,9 @@ void launch_p2m(int npacks, hipStream_t st, const LevelArgs& la, const Tables& t
 template <bool RHO>
 void launch_leaf(int nitems, hipStream_t st, const LevelArgs& la, const Tables& tab) {
     if (tab.p2p_cube) {
-        // the window's parity planes, or the staged L rows of 256 cells (20
-        // doubles each, shifted by one chunk every 16 rows)
-        const size_t lds = sizeof(double) * std::max<size_t>(8 * kWinPlane, 256 * 20 + 32);
+        // the window's parity planes; the staged results take less
+        constexpr size_t lds = sizeof(double) * 8 * kWinPlane;
+        static_assert(8 * kWinPlane >= (128 * 20 + 16) + (256 * 3 + 16) + 2 * (256 * 2 + 16));
         hipLaunchKernelGGL(leaf_cube_kernel<RHO>, dim3(nitems), dim3(256), lds, st, la);
     } else {
         const int W = kInx + 2 * tab.p2p_halo;
@@ -1920,12 +1953,6 @@ __global__ __launch_bounds__(256) void scatter_slots(const PartialSlot* __restri
             ms[q.x] = e.mon[q.y];
         }
     }
-}
-
-// geometric centre xbase + i*dx, rounded as written (grid_fmm.cpp:1669-1671)
-__device__ __forceinline__ double cell_centre(double xb, int i, double dx) {
-#pragma clang fp contract(off)
-    return xb + (double)i * dx;
 }
 
 // Upward pass of one level (grid::compute_multipoles, src/grid_fmm.cpp:1639-1803):
@@ -2868,6 +2895,8 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         la.correct_am = p->t_correct_am;
         la.leaf_rows = p->leaf_rows;
         la.overwrite = 0;
+        la.xbase = p->d_fxbase;
+        la.dx = p->dx;
         la.inv_dx = 1.0 / p->dx;
         la.neg_inv_dx = -1.0 / p->dx;
         const bool rho = p->type == OCTOFMM_RHO;

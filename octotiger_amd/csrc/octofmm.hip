@@ -2313,11 +2313,11 @@ struct octofmm_plan {
     int32_t mix_n64 = 0;
     uint32_t* d_queue = nullptr;   // per-XCD work counters of the persistent variants
     int32_t wide_parts = 0;        // variant 704 split further: workgroups per coarse block (0: not for this level)
-    double* d_wide = nullptr;      // and their folded sums [n_m2l * 8 * wide_parts][kFolded][64]
+    double* d_wide = nullptr;      // and their folded sums [n_m2l * 8 * wide_parts][kFolded][64] (behind d_rec)
     int32_t n_p2m = 0;             // leaf items with p2m: items [n_m2l, n_m2l + n_p2m)
     double* d_p2m_out = nullptr;   // their p2m sums [n_p2m][512][8], zeros where a cell has no p2m pair
     int32_t n_packs = 0;           // p2m work lists (P2mPacks): hdr, units, idx, di
-    int32_t* d_packs = nullptr;
+    int32_t* d_packs = nullptr;    // (behind d_p2m_out)
     size_t packs_units = 0, packs_idx = 0, packs_di = 0;   // first words of the lists behind hdr
     int64_t mixed_far_pairs_by_offset = 0;   // FP32 far pairs under that rule
     int64_t mixed_far_pairs_by_pair = 0;     // and under the per-pair rule of mapping 0
@@ -2796,9 +2796,7 @@ static void plan_free(octofmm_plan* p) {
     (void)hipFree(p->d_recm);
     (void)hipFree(p->d_mixorder);
     (void)hipFree(p->d_queue);
-    (void)hipFree(p->d_wide);
     (void)hipFree(p->d_p2m_out);
-    (void)hipFree(p->d_packs);
     (void)hipFree(p->d_partial);
     (void)hipFree(p->d_pslots);
     (void)hipFree(p->d_pidx);
@@ -3352,8 +3350,21 @@ static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* 
         plan_free(p);
         return fail(c, s, "%s", what);
     };
-    if (hipMalloc((void**)&p->d_rec, (size_t)ns * kCells * kRecDoubles * sizeof(double) + kRecTailBytes) != hipSuccess)
+    if (!root && p->precision == OCTOFMM_PRECISION_FP64) {
+        // (a forced variant runs its plain form in a tree, too)
+        if (in_tree && !std::getenv("OCTOFMM_VARIANT")) {
+            p->wide_parts = sums_first_parts(n_m2l, T);
+            p->sums_first = p->wide_parts > 0;
+            if (p->sums_first) p->variant = 704;
+        }
+        if (!p->sums_first) p->wide_parts = wide_parts(n_m2l, T);
+    }
+    // the records and, behind them, the wide form's sums in one block
+    const size_t rec_bytes = (size_t)ns * kCells * kRecDoubles * sizeof(double) + kRecTailBytes;
+    if (hipMalloc((void**)&p->d_rec, rec_bytes + wide_bytes(n_m2l, p->wide_parts)) != hipSuccess)
         return cleanup(OCTOFMM_ERR_ALLOCATION, "record buffer allocation failed");
+    static_assert(kRecTailBytes % sizeof(double) == 0);
+    p->d_wide = p->d_rec + rec_bytes / sizeof(double);
     if (hipMalloc((void**)&p->d_nbr, sizeof(int32_t) * 27 * ns) != hipSuccess ||
         hipMalloc((void**)&p->d_kind, sizeof(int32_t) * ns) != hipSuccess ||
         hipMalloc((void**)&p->d_foff, sizeof(int32_t) * 3 * ns) != hipSuccess ||
@@ -3371,18 +3382,6 @@ static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* 
         return cleanup(OCTOFMM_ERR_ALLOCATION, "root partial buffer allocation failed");
     if (!root && hipMalloc((void**)&p->d_queue, sizeof(uint32_t) * 8) != hipSuccess)
         return cleanup(OCTOFMM_ERR_ALLOCATION, "work counter allocation failed");
-    if (!root && p->precision == OCTOFMM_PRECISION_FP64) {
-        // (a forced variant runs its plain form in a tree, too)
-        if (in_tree && !std::getenv("OCTOFMM_VARIANT")) {
-            p->wide_parts = sums_first_parts(n_m2l, T);
-            p->sums_first = p->wide_parts > 0;
-            if (p->sums_first) p->variant = 704;
-        }
-        if (!p->sums_first) p->wide_parts = wide_parts(n_m2l, T);
-    }
-    if (p->wide_parts > 0 &&
-        hipMalloc((void**)&p->d_wide, wide_bytes(n_m2l, p->wide_parts)) != hipSuccess)
-        return cleanup(OCTOFMM_ERR_ALLOCATION, "partial sum buffer allocation failed");
     p->n_p2m = (int32_t)buckets[2].size();
     if (p->n_p2m > 0) {
         const size_t bytes = sizeof(double) * (size_t)p->n_p2m * kCells * 8;
@@ -3401,9 +3400,9 @@ static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* 
         all.insert(all.end(), pk.idx.begin(), pk.idx.end());
         p->packs_di = all.size();
         if (!T.p2p_cube) all.insert(all.end(), pk.di.begin(), pk.di.end());
-        if (hipMalloc((void**)&p->d_p2m_out, bytes) != hipSuccess ||
-            hipMalloc((void**)&p->d_packs, sizeof(int32_t) * std::max<size_t>(1, all.size())) != hipSuccess)
+        if (hipMalloc((void**)&p->d_p2m_out, bytes + sizeof(int32_t) * all.size()) != hipSuccess)
             return cleanup(OCTOFMM_ERR_ALLOCATION, "p2m buffer allocation failed");
+        p->d_packs = reinterpret_cast<int32_t*>(p->d_p2m_out + bytes / sizeof(double));
         if (hipMemset(p->d_p2m_out, 0, bytes) != hipSuccess ||
             hipMemcpy(p->d_packs, all.data(), sizeof(int32_t) * all.size(), hipMemcpyHostToDevice) != hipSuccess)
             return cleanup(OCTOFMM_ERR_HIP, "p2m work list upload failed");

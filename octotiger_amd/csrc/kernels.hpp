@@ -801,16 +801,14 @@ struct M2MArgs {
     const double* M;        // [n][512][20] this level
     double* com;            // [n][512][3]  this level (leaf centres written for RHO)
     const double* mon;      // [n][512]
-    const int32_t* kind;
     const int32_t* parent;
     const int32_t* octant;
+    const int32_t* order;   // [n] nodes of the level: nleaf leaves, then the refined ones
     const double* xbase;    // [n][3]
     double* pM;             // parent level [np][512][20]
     double* pcom;           // parent level [np][512][3]
     double dx;
-    int32_t nnodes;
-    int32_t rho;
+    int32_t nleaf;
 };
-
 
 }   // namespace octofmm

@@ -1964,42 +1964,178 @@ __global__ __launch_bounds__(256) void scatter_slots(const PartialSlot* __restri
     }
 }
 
-// Upward pass of one level (grid::compute_multipoles, src/grid_fmm.cpp:1639-1803):
-// one lane per child cell, 8 consecutive lanes per coarse cell (512 per
-// node).  For RHO the leaf nodes' cell centres are written first; the 8 lanes
-// form the coarse cell's mass and mass-weighted centre by a fixed butterfly,
-// shift their child's multipole to it, and sum the shifted multipoles in
-// child order through LDS, each lane summing and storing 2 or 3 components of
-// the parent's cell.
-__global__ __launch_bounds__(256) void m2m_kernel(M2MArgs a) {
-    __shared__ double s_m2m[256 * 11];
-    const int gid = blockIdx.x * 256 + threadIdx.x;
-    if (gid >= a.nnodes * kCells) return;     // whole 8-lane groups exit together
-    const int n = gid >> 9, q = (gid >> 3) & 63, ci = gid & 7;
-    const int ip = q >> 4, jp = (q >> 2) & 3, kp = q & 3;
-    const bool leaf = a.kind[n] == OCTOFMM_SLOT_LEAF;   // uniform per node, so per wave
-    const int u = (2 * ip + (ci & 1)) * 64 + (2 * jp + ((ci >> 1) & 1)) * 8 + (2 * kp + ((ci >> 2) & 1));
-    const double* xb = a.xbase + 3 * n;
-    if (leaf && a.rho) {
-        // the leaf cells' centres, consecutive lanes on consecutive cells so
-        // the stores coalesce
-        const int v = gid & (kCells - 1);
-        double* Xv = a.com + ((size_t)n * kCells + v) * 3;
-        Xv[0] = cell_centre(xb[0], v >> 6, a.dx);
-        Xv[1] = cell_centre(xb[1], (v >> 3) & 7, a.dx);
-        Xv[2] = cell_centre(xb[2], v & 7, a.dx);
+// Upward pass of one leaf: one wave, lane = coarse cell, whose 8 monopoles it
+// sums about their centre of mass (for RHO, which it forms; DRHODT takes the
+// stored ones) without meeting another lane.  The rows go through the wave's
+// LDS (32 cells at a time) and leave as the runs of 4 cells they are in the
+// parent, and for RHO the leaf cells' centres as the contiguous block they are,
+// in 16-byte pieces.  Bound by what it moves, 28 KiB a leaf: 5568 leaves take 24
+// us (6.5 TB/s, part of it from the caches), where 8 lanes per coarse cell, with
+// seven times the instructions and stores of single doubles 24 bytes apart, took
+// 43 to 54.
+template <bool RHO>
+__device__ __forceinline__ void m2m_leaf(const M2MArgs& a, int n, double* s_rows) {
+    const int l = threadIdx.x & 63;
+    const int ip = l >> 4, jp = (l >> 2) & 3, kp = l & 3;
+    const auto* xb = as_const(a.xbase) + 3 * n;
+    const int pn = as_const(a.parent)[n], oct = as_const(a.octant)[n];
+    const size_t u0 = (size_t)n * kCells + ip * 128 + jp * 16 + kp * 2;
+    double m[8];   // child (kx, ky, kz) at 4 kx + 2 ky + kz
+#pragma unroll
+    for (int q = 0; q < 4; ++q) load2(a.mon + u0 + (q >> 1) * 64 + (q & 1) * 8, m + 2 * q);
+    if constexpr (RHO) {
+        // the cells' centres: 192 pieces of two doubles for each pair of x planes
+        double* com = a.com + (size_t)n * (kCells * 3);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            int first[2], step[2];
+            double base[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int d = 2 * (l + 64 * j) + e, cell = d / 3, c = d - 3 * cell;
+                first[e] = c == 0 ? cell >> 6 : c == 1 ? (cell >> 3) & 7 : cell & 7;
+                step[e] = c == 0 ? 2 : 0;
+                base[e] = c == 0 ? xb[0] : c == 1 ? xb[1] : xb[2];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const double2_a8 v = {cell_centre(base[0], first[0] + q * step[0], a.dx),
+                    cell_centre(base[1], first[1] + q * step[1], a.dx)};
+                __builtin_nontemporal_store(v, reinterpret_cast<double2_a8*>(com + 384 * q + 2 * (l + 64 * j)));
+            }
+        }
     }
+    if (pn < 0) return;   // uniform
+    const size_t pc = (size_t)pn * kCells + parent_cell(oct, ip, jp, kp);
+    double B[20];
+    if constexpr (RHO) {
+        // the children's centres form a grid: their moments about Y by one axis
+        // after the other, T[x][y^i z^j], from 2 weights per axis and power
+        double d[3][2][4];   // axis, side, power
+        const double mx0 = (m[0] + m[1]) + (m[2] + m[3]), mx1 = (m[4] + m[5]) + (m[6] + m[7]);
+        const double my0 = (m[0] + m[1]) + (m[4] + m[5]), my1 = (m[2] + m[3]) + (m[6] + m[7]);
+        const double mz0 = (m[0] + m[2]) + (m[4] + m[6]), mz1 = (m[1] + m[3]) + (m[5] + m[7]);
+        const double mtot = mx0 + mx1;
+        const double lo[3] = {mx0, my0, mz0}, hi[3] = {mx1, my1, mz1};
+        const int at[3] = {2 * ip, 2 * jp, 2 * kp};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double c0 = cell_centre(xb[c], at[c], a.dx), c1 = cell_centre(xb[c], at[c] + 1, a.dx);
+            const double Y = (c0 * lo[c] + c1 * hi[c]) / mtot;
+            a.pcom[pc * 3 + c] = Y;
+            d[c][0][1] = c0 - Y;
+            d[c][1][1] = c1 - Y;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                d[c][k][2] = d[c][k][1] * d[c][k][1];
+                d[c][k][3] = d[c][k][2] * d[c][k][1];
+            }
+        }
+        double T[2][4][4];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            double Z[2][4];
+#pragma unroll
+            for (int y = 0; y < 2; ++y) {
+                const double m0 = m[4 * x + 2 * y], m1 = m[4 * x + 2 * y + 1];
+                Z[y][0] = m0 + m1;
+#pragma unroll
+                for (int j = 1; j < 4; ++j) Z[y][j] = fma(m1, d[2][1][j], m0 * d[2][0][j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                T[x][0][j] = Z[0][j] + Z[1][j];
+#pragma unroll
+                for (int i = 1; i + j < 4; ++i) T[x][i][j] = fma(Z[1][j], d[1][1][i], Z[0][j] * d[1][0][i]);
+            }
+        }
+        auto moment = [&](int h, int i, int j) -> double {
+            return h == 0 ? T[0][i][j] + T[1][i][j] : fma(T[1][i][j], d[0][1][h], T[0][i][j] * d[0][0][h]);
+        };
+        auto moment_of = [&](int b, int c, int e) -> double {   // axes b, c, e (3: none)
+            return moment((b == 0) + (c == 0) + (e == 0), (b == 1) + (c == 1) + (e == 1), (b == 2) + (c == 2) + (e == 2));
+        };
+        B[0] = moment(0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            B[1 + b] = moment_of(b, 3, 3);
+#pragma unroll
+            for (int c = b; c < 3; ++c) {
+                B[tmap2(b, c)] = moment_of(b, c, 3);
+#pragma unroll
+                for (int e = c; e < 3; ++e) B[tmap3(b, c, e)] = moment_of(b, c, e);
+            }
+        }
+    } else {
+        double Y[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) Y[c] = a.pcom[pc * 3 + c];
+#pragma unroll
+        for (int j = 0; j < 20; ++j) B[j] = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            double X[6];   // the centres of a pair along z
+            const double* src = a.com + (u0 + (q >> 1) * 64 + (q & 1) * 8) * 3;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) load2(src + 2 * k, X + 2 * k);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const double dX[3] = {X[3 * k] - Y[0], X[3 * k + 1] - Y[1], X[3 * k + 2] - Y[2]};
+                double S[20];
+                monopole_shift(m[2 * q + k], dX, S);
+#pragma unroll
+                for (int j = 0; j < 20; ++j) B[j] += S[j];
+            }
+        }
+    }
+    double2* row = reinterpret_cast<double2*>(s_rows) + (l & 31) * 10;
+    const double2* rows = reinterpret_cast<const double2*>(s_rows);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if (h == 1) lds_wave_sync();   // the first half's rows are read before they are overwritten
+        if ((l >> 5) == h) {
+#pragma unroll
+            for (int j = 0; j < 10; ++j) row[j] = make_double2(B[2 * j], B[2 * j + 1]);
+        }
+        lds_wave_sync();
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {   // 32 rows x 10 pieces
+            const int ch = l + 64 * i, r = 32 * h + ch / 10;
+            const double2 v = rows[ch];
+            double* dst = a.pM + ((size_t)pn * kCells + parent_cell(oct, r >> 4, (r >> 2) & 3, r & 3)) * 20 + 2 * (ch % 10);
+            *reinterpret_cast<double2_a8*>(dst) = double2_a8{v.x, v.y};
+        }
+    }
+}
+
+// Upward pass of one level (grid::compute_multipoles, src/grid_fmm.cpp:1639-1803).
+// The first workgroups take the leaves, four each (m2m_leaf).  Two workgroups
+// take a refined node, one lane per child cell, 8 consecutive lanes per coarse
+// cell: for RHO the 8 lanes form the coarse cell's mass and mass-weighted
+// centre by a fixed butterfly, shift their child's multipole to it, and sum the
+// shifted multipoles in child order through LDS, each lane summing and storing
+// 2 or 3 components of the parent's cell.
+template <bool RHO>
+__global__ __launch_bounds__(256) void m2m_kernel(M2MArgs a) {
+    __shared__ __attribute__((aligned(16))) double s_m2m[256 * 11];
+    const int nb = (a.nleaf + 3) >> 2;
+    if ((int)blockIdx.x < nb) {
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        const int i = (int)blockIdx.x * 4 + wave;
+        if (i < a.nleaf) m2m_leaf<RHO>(a, as_const(a.order)[i], s_m2m + wave * (32 * 20));
+        return;
+    }
+    const int rest = (int)blockIdx.x - nb;
+    const int n = as_const(a.order)[a.nleaf + (rest >> 1)];
+    const int q = (((rest & 1) << 8) + (int)threadIdx.x) >> 3, ci = threadIdx.x & 7;
+    const int ip = q >> 4, jp = (q >> 2) & 3, kp = q & 3;
+    const int u = (2 * ip + (ci & 1)) * 64 + (2 * jp + ((ci >> 1) & 1)) * 8 + (2 * kp + ((ci >> 2) & 1));
     const int pn = a.parent[n];
     if (pn < 0) return;                        // uniform per node
     const int pc = parent_cell(a.octant[n], ip, jp, kp);
     double* Yp = a.pcom + ((size_t)pn * kCells + pc) * 3;
     double A[20];
-    double x0, x1, x2;
-    if (leaf) {
-        A[0] = a.mon[(size_t)n * kCells + u];
-#pragma unroll
-        for (int j = 1; j < 20; ++j) A[j] = 0.0;
-    } else {
+    {
         const double2* src = reinterpret_cast<const double2*>(a.M + ((size_t)n * kCells + u) * 20);
 #pragma unroll
         for (int j = 0; j < 10; ++j) {
@@ -2008,19 +2144,10 @@ __global__ __launch_bounds__(256) void m2m_kernel(M2MArgs a) {
             A[2 * j + 1] = v.y;
         }
     }
-    if (leaf && a.rho) {
-        // the centre stored above for cell u, formed again rather than read back
-        x0 = cell_centre(xb[0], u >> 6, a.dx);
-        x1 = cell_centre(xb[1], (u >> 3) & 7, a.dx);
-        x2 = cell_centre(xb[2], u & 7, a.dx);
-    } else {
-        const double* X = a.com + ((size_t)n * kCells + u) * 3;
-        x0 = X[0];
-        x1 = X[1];
-        x2 = X[2];
-    }
+    const double* X = a.com + ((size_t)n * kCells + u) * 3;
+    const double x0 = X[0], x1 = X[1], x2 = X[2];
     double Y[3];
-    if (a.rho) {
+    if constexpr (RHO) {
         const double mtot = sum8(A[0]);
         Y[0] = sum8(x0 * A[0]) / mtot;
         Y[1] = sum8(x1 * A[0]) / mtot;
@@ -2037,10 +2164,7 @@ __global__ __launch_bounds__(256) void m2m_kernel(M2MArgs a) {
     }
     const double dX[3] = {x0 - Y[0], x1 - Y[1], x2 - Y[2]};
     double B[20];
-    if (leaf)
-        monopole_shift(A[0], dX, B);
-    else
-        multipole_shift(A, dX, B);
+    multipole_shift(A, dX, B);
     // the 8 children's shifted multipoles meet in the wave's LDS rows, 10
     // components at a time (11 doubles apart, so the 8 lanes reading one
     // component hit distinct banks; two passes of 10 halve the LDS a
@@ -3636,6 +3760,8 @@ struct octofmm_tree_plan {
         int32_t* d_kind = nullptr;
         int32_t* d_parent = nullptr;
         int32_t* d_octant = nullptr;
+        int32_t* d_order = nullptr;   // the leaves, then the refined nodes
+        int32_t nleaf = 0;
         octofmm_plan* plan = nullptr;
     };
     octofmm_context* ctx = nullptr;
@@ -3684,7 +3810,6 @@ void tree_free(octofmm_tree_plan* t) {
 octofmm_status tree_launch(octofmm_tree_plan* t, hipStream_t st, int phases) {
     octofmm_context* c = t->ctx;
     const int nl = (int)t->lv.size();
-    const int rho = t->type == OCTOFMM_RHO;
     if (phases & 1)
         for (int l = nl - 1; l >= 0; --l) {
             const auto& L = t->lv[l];
@@ -3693,16 +3818,19 @@ octofmm_status tree_launch(octofmm_tree_plan* t, hipStream_t st, int phases) {
             a.M = L.M;
             a.com = L.com;
             a.mon = L.mon;
-            a.kind = L.d_kind;
             a.parent = L.d_parent;
             a.octant = L.d_octant;
             a.xbase = L.d_xbase;
             a.pM = l > 0 ? t->lv[l - 1].M : nullptr;
             a.pcom = l > 0 ? t->lv[l - 1].com : nullptr;
             a.dx = L.dx;
-            a.nnodes = L.nnodes;
-            a.rho = rho;
-            hipLaunchKernelGGL(m2m_kernel, dim3((L.nnodes * kCells + 255) / 256), dim3(256), 0, st, a);
+            a.order = L.d_order;
+            a.nleaf = L.nleaf;
+            const dim3 grid((L.nleaf + 3) / 4 + 2 * (L.nnodes - L.nleaf));
+            if (t->type == OCTOFMM_RHO)
+                hipLaunchKernelGGL(m2m_kernel<true>, grid, dim3(256), 0, st, a);
+            else
+                hipLaunchKernelGGL(m2m_kernel<false>, grid, dim3(256), 0, st, a);
             HIPC(c, hipGetLastError());
         }
     // Interactions of every level, root first.  Each level's kernels also
@@ -3871,19 +3999,25 @@ octofmm_status octofmm_tree_plan_create(octofmm_context* c, const octofmm_tree* 
         D.Lc = L.d_L_c;
         D.g = L.d_g;
         const size_t n = (size_t)L.nnodes;
-        // one block: xbase, kind, parent, octant
-        std::vector<double> tables((3 * n * sizeof(double) + 3 * n * sizeof(int32_t) + 7) / 8);
+        // one block: xbase, kind, parent, octant, order
+        std::vector<double> tables((3 * n * sizeof(double) + 4 * n * sizeof(int32_t) + 7) / 8);
         std::copy(L.xbase, L.xbase + 3 * n, tables.begin());
         int32_t* ti = reinterpret_cast<int32_t*>(tables.data() + 3 * n);
         std::copy(L.kind, L.kind + n, ti);
         std::copy(L.parent, L.parent + n, ti + n);
         std::copy(L.octant, L.octant + n, ti + 2 * n);
+        int32_t* to = ti + 3 * n;
+        for (const int32_t k : {OCTOFMM_SLOT_LEAF, OCTOFMM_SLOT_NONLEAF})
+            for (int i = 0; i < L.nnodes; ++i)
+                if (L.kind[i] == k) *to++ = i;
+        D.nleaf = (int32_t)std::count(L.kind, L.kind + n, (int32_t)OCTOFMM_SLOT_LEAF);
         const size_t bytes = tables.size() * sizeof(double);
         if (hipMalloc((void**)&D.d_xbase, bytes) != hipSuccess)
             return cleanup(OCTOFMM_ERR_ALLOCATION, "tree table allocation failed");
         D.d_kind = reinterpret_cast<int32_t*>(D.d_xbase + 3 * n);
         D.d_parent = D.d_kind + n;
         D.d_octant = D.d_parent + n;
+        D.d_order = D.d_octant + n;
         if (hipMemcpy(D.d_xbase, tables.data(), bytes, hipMemcpyHostToDevice) != hipSuccess)
             return cleanup(OCTOFMM_ERR_HIP, "tree table upload failed");
         t->stats.nodes += L.nnodes;

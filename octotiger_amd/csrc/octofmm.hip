@@ -2241,49 +2241,52 @@ void build_p2m_packs(const P2mReach& reach, int nitems, F&& refined, P2mPacks& o
         int32_t id, first, n;
     };
     std::vector<Unit> units;
-    std::vector<int32_t> rec, di;
-    int longest = 0;
-    std::vector<int32_t> crec[64], cdi[64];
+    std::vector<int32_t> rec, di;   // the units' entries, one unit after another
     for (int o = 0; o < nitems; ++o) {
-        for (int C = 0; C < 64; ++C) {
-            crec[C].clear();
-            cdi[C].clear();
-        }
+        int slot[27], count[64] = {}, at[64];
         for (int raw = 0; raw < 27; ++raw) {
-            const int slot = raw == 13 ? -1 : refined(o, raw);
-            if (slot < 0) continue;
-            for (const P2mReach::Hit& h : reach.by_raw[raw]) {
-                crec[h.C].push_back(slot * kCells + h.rec);
-                cdi[h.C].push_back(h.di);
-            }
+            slot[raw] = raw == 13 ? -1 : refined(o, raw);
+            if (slot[raw] < 0) continue;
+            for (const P2mReach::Hit& h : reach.by_raw[raw]) ++count[h.C];
         }
+        int end = (int)rec.size();
         for (int C = 0; C < 64; ++C) {
-            if (crec[C].empty()) continue;
-            units.push_back({o * 64 + C, (int32_t)rec.size(), (int32_t)crec[C].size()});
-            longest = std::max(longest, (int)crec[C].size());
-            rec.insert(rec.end(), crec[C].begin(), crec[C].end());
-            di.insert(di.end(), cdi[C].begin(), cdi[C].end());
+            at[C] = end;
+            if (count[C] > 0) units.push_back({o * 64 + C, end, count[C]});
+            end += count[C];
+        }
+        rec.resize(end);
+        di.resize(end);
+        for (int raw = 0; raw < 27; ++raw) {
+            if (slot[raw] < 0) continue;
+            for (const P2mReach::Hit& h : reach.by_raw[raw]) {
+                rec[at[h.C]] = slot[raw] * kCells + h.rec;
+                di[at[h.C]++] = h.di;
+            }
         }
     }
-    std::vector<std::vector<int32_t>> by_n(longest + 1);
-    for (size_t u = 0; u < units.size(); ++u) by_n[units[u].n].push_back((int32_t)u);
-    std::vector<int32_t> order;
-    for (int n = longest; n > 0; --n) order.insert(order.end(), by_n[n].begin(), by_n[n].end());
-    for (size_t p = 0; p < order.size(); p += 8) {
-        const int rows = units[order[p]].n, first = (int)out.idx.size() / 8;
-        out.hdr.push_back(first);
-        out.hdr.push_back(rows);
-        out.idx.resize((size_t)(first + rows) * 8, -1);
-        out.di.resize((size_t)(first + rows) * 8, 0);
-        for (int g = 0; g < 8; ++g) {
-            const bool have = p + g < order.size();
-            out.units.push_back(have ? units[order[p + g]].id : -1);
-            if (!have) continue;
-            const Unit& u = units[order[p + g]];
-            for (int e = 0; e < u.n; ++e) {
-                out.idx[(size_t)(first + e) * 8 + g] = rec[u.first + e];
-                out.di[(size_t)(first + e) * 8 + g] = di[u.first + e];
-            }
+    int end_of[kMaxDelta + 2] = {};   // counting sort: units of n entries lie before end_of[n]
+    for (const Unit& u : units) ++end_of[u.n];
+    for (int n = kMaxDelta; n >= 0; --n) end_of[n] += end_of[n + 1];
+    std::vector<int32_t> order(units.size());
+    for (size_t u = units.size(); u-- > 0;) order[--end_of[units[u].n]] = (int32_t)u;
+    const size_t npacks = (units.size() + 7) / 8;
+    out.hdr.resize(2 * npacks);
+    int rows = 0;
+    for (size_t p = 0; p < npacks; ++p) {
+        out.hdr[2 * p] = rows;
+        rows += out.hdr[2 * p + 1] = units[order[8 * p]].n;
+    }
+    out.units.assign(8 * npacks, -1);
+    out.idx.assign((size_t)rows * 8, -1);
+    out.di.assign((size_t)rows * 8, 0);
+    for (size_t q = 0; q < order.size(); ++q) {
+        const Unit& u = units[order[q]];
+        out.units[q] = u.id;
+        const size_t first = (size_t)out.hdr[2 * (q / 8)] * 8 + q % 8;
+        for (int e = 0; e < u.n; ++e) {
+            out.idx[first + 8 * e] = rec[u.first + e];
+            out.di[first + 8 * e] = di[u.first + e];
         }
     }
 }

@@ -626,7 +626,7 @@ struct StageArgs {
 
 // Levels of one stage_records launch, and the most slots (of 4 workgroups each)
 // of levels that share one: four workgroups a CU, one round of the chip.
-constexpr int kStageLevels = 4;
+constexpr int kStageLevels = 6;
 constexpr int kStageTogether = 256;
 struct StageGroup {
     StageArgs a[kStageLevels];
@@ -686,6 +686,7 @@ struct LevelArgs {
     int32_t parts;
     int32_t nitems;
     int32_t item0;          // first item of this launch
+    int32_t leaf0;          // first leaf item
     double inv_dx;
     double neg_inv_dx;
 };
@@ -693,9 +694,23 @@ struct LevelArgs {
 struct RootArgs {
     const double* rec;      // records of the root slot (512 x 24)
     const Tables* tab;
-    double* partial;        // [nchunks][512][24]
-    int32_t per_chunk;
-    int32_t nchunks;
+    double* partial;        // [kRootChunks][512][24]
+};
+
+// tree_sums_kernel: the root's pairs, and per level the workgroups of its sums
+// (items x 8 x parts) and of its p2m (packs).
+struct TreeSums {
+    RootArgs root;
+    int32_t sums[kStageLevels];
+    int32_t packs[kStageLevels];
+    LevelArgs a[kStageLevels];
+};
+
+// Leaf targets of up to kLeafLevels levels, one after another.
+constexpr int kLeafLevels = 4;
+struct LeafGroup {
+    int32_t n[kLeafLevels];
+    LevelArgs a[kLeafLevels];
 };
 
 struct RootReduceArgs {

@@ -1263,11 +1263,14 @@ __device__ __forceinline__ void p2p_cube(const double* s_win, int Cx, int Cy, in
 // all even or odd planes at once, 40 KiB, left room for 3): a solve of 9361
 // leaves takes 1290 us in place of 1313.
 template <bool RHO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void leaf_cube_kernel(LevelArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void leaf_cube_kernel(LeafGroup g) {
     extern __shared__ double s_win[];
     __shared__ int s_nbr[27];
     __shared__ int s_kind[27];
-    const int ordinal = xcd_item(blockIdx.x, gridDim.x);
+    int at = blockIdx.x, lvl = 0;
+    while (lvl < kLeafLevels - 1 && at >= g.n[lvl]) at -= g.n[lvl++];   // uniform
+    const LevelArgs& a = g.a[lvl];
+    const int ordinal = xcd_item(at, g.n[lvl]);
     const int2 it = a.items[a.item0 + ordinal];
     const int slot = __builtin_amdgcn_readfirstlane(it.x);
     const int th = threadIdx.x;
@@ -1460,9 +1463,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
 //
 // FULL: every pair of an entry's 8 x 8 cells is in the stencil (theta 0.5).
 template <bool RHO, bool FULL>
-__global__ __launch_bounds__(256) void p2m_kernel(LevelArgs a) {
-    __shared__ double2 s_stage[4 * kDirWave];
-    const int pack = xcd_item(blockIdx.x, gridDim.x);
+__device__ __forceinline__ void p2m_pack(const LevelArgs& a, int pack, double2* s_stage) {
     const int sl = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     double2* stage = s_stage + sl * kDirWave;
     const int l = threadIdx.x & 63, k = l & 7;
@@ -1471,7 +1472,7 @@ __global__ __launch_bounds__(256) void p2m_kernel(LevelArgs a) {
     const int unit = a.p2m_units[(size_t)pack * 8 + (l >> 3)];   // -1: none
     const int C = unit & 63, ordinal = unit < 0 ? 0 : unit >> 6;
     const int cell = (2 * (C >> 4) + (k >> 2)) * 64 + (2 * ((C >> 2) & 3) + ((k >> 1) & 1)) * 8 + 2 * (C & 3) + (k & 1);
-    const double* xc = a.com + ((size_t)a.items[a.item0 + ordinal].x * kCells + cell) * 3;
+    const double* xc = a.com + ((size_t)a.items[a.leaf0 + ordinal].x * kCells + cell) * 3;
     const double X0 = xc[0], X1 = xc[1], X2 = xc[2];
     Acc<RHO> s;
     acc_clear(s);
@@ -1563,6 +1564,12 @@ __global__ __launch_bounds__(256) void p2m_kernel(LevelArgs a) {
     out[3] = make_double2(C3[2], 0.0);
 }
 
+template <bool RHO, bool FULL>
+__global__ __launch_bounds__(256) void p2m_kernel(LevelArgs a) {
+    __shared__ double2 s_stage[4 * kDirWave];
+    p2m_pack<RHO, FULL>(a, xcd_item(blockIdx.x, gridDim.x), s_stage);
+}
+
 template <bool RHO>
 void launch_p2m(int npacks, hipStream_t st, const LevelArgs& la, const Tables& tab) {
     if (npacks <= 0) return;
@@ -1572,13 +1579,26 @@ void launch_p2m(int npacks, hipStream_t st, const LevelArgs& la, const Tables& t
         hipLaunchKernelGGL((p2m_kernel<RHO, false>), dim3(npacks), dim3(256), 0, st, la);
 }
 
+// Leaf items of n <= kLeafLevels levels in one launch (theta 0.5).
+template <bool RHO>
+void launch_leaf_cube(const LevelArgs* la, int n, hipStream_t st) {
+    // the window's parity planes; the staged results take less
+    constexpr size_t lds = sizeof(double) * 8 * kWinPlane;
+    static_assert(8 * kWinPlane >= (128 * 20 + 16) + (256 * 3 + 16) + 2 * (256 * 2 + 16));
+    LeafGroup g;
+    int nitems = 0;
+    for (int i = 0; i < kLeafLevels; ++i) {
+        g.a[i] = la[i < n ? i : 0];
+        g.n[i] = i < n ? la[i].nitems : 0;
+        nitems += g.n[i];
+    }
+    if (nitems > 0) hipLaunchKernelGGL(leaf_cube_kernel<RHO>, dim3(nitems), dim3(256), lds, st, g);
+}
+
 template <bool RHO>
 void launch_leaf(int nitems, hipStream_t st, const LevelArgs& la, const Tables& tab) {
     if (tab.p2p_cube) {
-        // the window's parity planes; the staged results take less
-        constexpr size_t lds = sizeof(double) * 8 * kWinPlane;
-        static_assert(8 * kWinPlane >= (128 * 20 + 16) + (256 * 3 + 16) + 2 * (256 * 2 + 16));
-        hipLaunchKernelGGL(leaf_cube_kernel<RHO>, dim3(nitems), dim3(256), lds, st, la);
+        launch_leaf_cube<RHO>(&la, 1, st);
     } else {
         const int W = kInx + 2 * tab.p2p_halo;
         hipLaunchKernelGGL(leaf_kernel<RHO>, dim3(nitems), dim3(512), sizeof(double) * W * W * W, st, la);
@@ -1647,16 +1667,20 @@ __global__ __launch_bounds__(64 * SPLIT) __attribute__((amdgpu_waves_per_eu(3)))
 // (theta 0.5 / 0.34): 1 target 25.3 / 74.6 -> 10.7 / 15.1 us, 8 targets 26.0 /
 // 75.2 -> 16.5 / 29.3 us, 18 targets 26.4 / 76.2 -> 21.5 / 47.3 us.
 template <bool RHO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void level_kernel_wide(LevelArgs a) {
-    __shared__ int s_nbr[27];
-    __shared__ int s_kind[27];
-    __shared__ double2 s_stage[4 * kDirWave];
-    const int v = xcd_item(blockIdx.x, gridDim.x);
+__device__ __forceinline__ void wide_part(const LevelArgs& a, int v, int* s_nbr, int* s_kind, double2* s_stage) {
     const int block = v / a.parts, part = v - block * a.parts;
     const int2 it = a.items[a.item0 + (block >> 3)];
     if (it.y & kItemNear) near_tables(a, it.x, s_nbr, s_kind);   // uniform per workgroup
     m2l_item_direct<RHO, 4, false, true>(a, it.x, it.y, s_nbr, s_kind, block & 7, s_stage, (int)(threadIdx.x >> 6), part,
         a.wide_sums + (size_t)v * (kFolded * 64));
+}
+
+template <bool RHO>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void level_kernel_wide(LevelArgs a) {
+    __shared__ int s_nbr[27];
+    __shared__ int s_kind[27];
+    __shared__ double2 s_stage[4 * kDirWave];
+    wide_part<RHO>(a, xcd_item(blockIdx.x, gridDim.x), s_nbr, s_kind, s_stage);
 }
 
 // Sums the parts of one coarse block of a target (one wave, lane = cell) in
@@ -1709,14 +1733,13 @@ void launch_wide_reduce(int nitems, hipStream_t st, const LevelArgs& la, bool rh
 }
 
 // In a whole-tree solve the levels of up to 96 targets (three workgroups a CU)
-// run sums first: level_kernel_wide needs only the level's records, so the
-// sums of the coarse levels, the root's among them, run side by side, and of
-// the chain from level to level only level_reduce with its downward pass is
-// left (329-sub-grid tree: 160 -> 125 us a solve, 10,697: 1338 -> 1307; the sums
-// of a level of 8 targets take 11 us beside those of 32 and the reduction 6,
-// where the level kernels took 22 and 30 one after the other).  Larger levels
-// fill the chip by themselves, and their sums would cost as much traffic as
-// their results.  Workgroups per coarse block of such a level, 0 for a larger
+// run sums first: their sums need only the level's records, so those of the
+// coarse levels run side by side with the root's pairs, and of the chain from
+// level to level only level_reduce with its downward pass (5 to 6 us) is left,
+// where the level kernels of 8 and 32 targets took 22 and 30 us one after the
+// other (329-sub-grid tree: 160 -> 125 us a solve, 10,697: 1338 -> 1307).  Larger
+// levels fill the chip by themselves, and their sums would cost as much traffic
+// as their results.  Workgroups per coarse block of such a level, 0 for a larger
 // one.
 int sums_first_parts(int n, const Tables& tab) {
     if (n <= 0 || n > 96) return 0;
@@ -1836,33 +1859,85 @@ void launch_level(int variant, int nitems, hipStream_t st, const LevelArgs& la, 
 }
 
 // Root sub-grid: every pair of its 512 cells except self and near offsets
-// (kokkos_kernel.hpp:324-471).  Workgroup q takes partners [q*per, (q+1)*per);
-// all lanes read the same partner, one target cell per lane.
+// (kokkos_kernel.hpp:324-471).  Workgroup b takes half b & 1 of the cells, one
+// per lane, over chunk b >> 1 of the partners, a row of 8 along z, whose records
+// all lanes read from LDS.
 template <bool RHO>
-__global__ __launch_bounds__(512) void root_kernel(RootArgs a) {
-    const int t = threadIdx.x;
+__device__ __forceinline__ void root_part(const RootArgs& a, int b, double2* s_rec) {
+    const int chunk = b >> 1, t = (b & 1) * 256 + (int)threadIdx.x;
+    const int px = chunk >> 3, py = chunk & 7;
+    if (threadIdx.x < 96) {
+        const int j = (int)threadIdx.x / 12, i = (int)threadIdx.x - 12 * j;
+        s_rec[threadIdx.x] = reinterpret_cast<const double2*>(a.rec + (size_t)record_of_cell(px, py, j) * kRecDoubles)[i];
+    }
     const int tx = t >> 6, ty = (t >> 3) & 7, tz = t & 7;
     const double* trec = a.rec + (size_t)record_of_cell(tx, ty, tz) * kRecDoubles;
     const double X0 = trec[kRecY], X1 = trec[kRecY + 1], X2 = trec[kRecY + 2];
+    const int dx = px - tx, dy = py - ty;
+    unsigned skip = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int dz = j - tz;
+        const bool inbox = dx >= -5 && dx <= 5 && dy >= -5 && dy <= 5 && dz >= -5 && dz <= 5;
+        if (inbox && a.tab->root_excluded[(dx + 5) * 121 + (dy + 5) * 11 + (dz + 5)]) skip |= 1u << j;
+    }
+    __syncthreads();
     Acc<RHO> s;
     acc_clear(s);
-    const int p0 = blockIdx.x * a.per_chunk;
-    for (int p = p0; p < p0 + a.per_chunk; ++p) {
-        const int px = p >> 6, py = (p >> 3) & 7, pz = p & 7;
-        const int dx = px - tx, dy = py - ty, dz = pz - tz;
-        const bool inbox = dx >= -5 && dx <= 5 && dy >= -5 && dy <= 5 && dz >= -5 && dz <= 5;
-        if (inbox && a.tab->root_excluded[(dx + 5) * 121 + (dy + 5) * 11 + (dz + 5)]) continue;
-        m2l_far<RHO>(a.rec + (size_t)record_of_cell(px, py, pz) * kRecDoubles, X0, X1, X2, s);
+#pragma unroll 1
+    for (int j = 0; j < 8; ++j) {
+        if ((skip >> j) & 1u) continue;
+        Rec r;
+#pragma unroll
+        for (int i = 0; i < 12; ++i) r.v[i] = s_rec[j * 12 + i];
+        m2l_far_rec<RHO>(r, X0, X1, X2, s);
     }
     double f[kFolded], L[20], C[3];
     acc_fold<RHO>(s, trec, f);
     acc_finish<RHO>(f, L, C);
-    double* o = a.partial + ((size_t)blockIdx.x * kCells + t) * kRecDoubles;
+    double* o = a.partial + ((size_t)chunk * kCells + t) * kRecDoubles;
 #pragma unroll
     for (int i = 0; i < 20; ++i) o[i] = L[i];
     o[20] = C[0];
     o[21] = C[1];
     o[22] = C[2];
+}
+
+template <bool RHO>
+__global__ __launch_bounds__(256) void root_kernel(RootArgs a) {
+    __shared__ double2 s_rec[96];
+    root_part<RHO>(a, blockIdx.x, s_rec);
+}
+
+// What a whole-tree solve does between the staging of its coarsest levels and
+// the chain of reductions from level to level, in one launch: the sums of the
+// sums-first levels, the finest first, their p2m, and the root's pairs.  As
+// kernels on branches of a graph they took 11, 27, 15 and 19 us, but ~8 us for
+// each branch and join; in one launch 39 us.  With the small leaf levels in one
+// launch as well a 329-sub-grid tree takes 95 us a solve in place of 124.
+template <bool RHO, bool FULL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void tree_sums_kernel(TreeSums g) {
+    __shared__ int s_nbr[27];
+    __shared__ int s_kind[27];
+    __shared__ double2 s_stage[4 * kDirWave];
+    int b = blockIdx.x;
+    for (int i = kStageLevels - 1; i >= 0; --i) {   // uniform
+        const int n = g.sums[i];
+        if (b < n) {
+            wide_part<RHO>(g.a[i], xcd_item(b, n), s_nbr, s_kind, s_stage);
+            return;
+        }
+        b -= n;
+    }
+    for (int i = kStageLevels - 1; i >= 0; --i) {
+        const int n = g.packs[i];
+        if (b < n) {
+            p2m_pack<RHO, FULL>(g.a[i], xcd_item(b, n), s_stage);
+            return;
+        }
+        b -= n;
+    }
+    root_part<RHO>(g.root, b, s_stage);
 }
 
 // One thread per output value (cell, component); the chunks are summed in
@@ -2664,12 +2739,10 @@ octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace& w, Pac
         ra.rec = w.rec;
         ra.tab = c->d_tab;
         ra.partial = w.partial;
-        ra.per_chunk = kCells / kRootChunks;
-        ra.nchunks = kRootChunks;
         if (rho)
-            hipLaunchKernelGGL(root_kernel<true>, dim3(kRootChunks), dim3(512), 0, st, ra);
+            hipLaunchKernelGGL(root_kernel<true>, dim3(kRootChunks * 2), dim3(256), 0, st, ra);
         else
-            hipLaunchKernelGGL(root_kernel<false>, dim3(kRootChunks), dim3(512), 0, st, ra);
+            hipLaunchKernelGGL(root_kernel<false>, dim3(kRootChunks * 2), dim3(256), 0, st, ra);
         HIPC(c, hipGetLastError());
         RootReduceArgs rr;
         rr.partial = w.partial;
@@ -2696,6 +2769,7 @@ octofmm_status launch_subgrid(octofmm_context* c, const SubgridWorkspace& w, Pac
     la.wide_sums = w.wide;
     la.mon = w.mon;
     la.p2m_out = w.p2m;
+    la.leaf0 = 0;
     la.p2m_hdr = w.packs;
     la.p2m_units = w.packs + 16;
     la.p2m_idx = w.packs + kPackHead;
@@ -2959,6 +3033,65 @@ static octofmm_status launch_stage(octofmm_context* c, hipStream_t st, octofmm_p
     return OCTOFMM_OK;
 }
 
+static LevelArgs level_args(const octofmm_plan* p) {
+    LevelArgs la;
+    la.rec = p->d_rec;
+    la.com = p->d_com;
+    la.L = p->d_L;
+    la.Lc = p->d_Lc;
+    la.nbr = p->d_nbr;
+    la.kind = p->d_kind;
+    la.items = p->d_items;
+    la.tab = p->ctx->d_tab;
+    la.mixbits = p->d_mixbits;
+    la.recm = p->d_recm;
+    la.mixorder = p->d_mixorder;
+    la.mix_n64 = p->mix_n64;
+    la.queue = p->d_queue;
+    la.parts = p->wide_parts;
+    la.wide_sums = p->d_wide;
+    la.mon = p->d_mon;
+    la.p2m_out = p->d_p2m_out;
+    la.parent = p->t_parent;
+    la.octant = p->t_octant;
+    la.pL = p->t_pL;
+    la.pLc = p->t_pLc;
+    la.pcom = p->t_pcom;
+    la.g = p->t_g;
+    la.G = p->t_G;
+    la.l2l = p->l2l ? 1 : 0;
+    la.correct_am = p->t_correct_am;
+    la.leaf_rows = p->leaf_rows;
+    la.overwrite = 0;
+    la.xbase = p->d_fxbase;
+    la.dx = p->dx;
+    la.inv_dx = 1.0 / p->dx;
+    la.neg_inv_dx = -1.0 / p->dx;
+    la.nitems = p->n_m2l;
+    la.item0 = 0;
+    la.leaf0 = p->n_m2l;
+    la.p2m_hdr = p->d_packs;
+    la.p2m_units = p->d_packs + p->packs_units;
+    la.p2m_idx = p->d_packs + p->packs_idx;
+    la.p2m_di = p->d_packs + p->packs_di;
+    return la;
+}
+
+static LevelArgs leaf_args(const octofmm_plan* p) {
+    LevelArgs la = level_args(p);
+    la.nitems = p->nitems - p->n_m2l;
+    la.item0 = p->n_m2l;
+    return la;
+}
+
+static RootArgs root_args(const octofmm_plan* p) {
+    RootArgs ra;
+    ra.rec = p->d_rec;
+    ra.tab = p->ctx->d_tab;
+    ra.partial = p->d_partial;
+    return ra;
+}
+
 // stage_mask bit 0: stage the partner records; bit 1: the root kernel, or the
 // level kernel over the multipole-target items (a sums-first level: what
 // level_reduce does of it); bit 4: a sums-first level's level_kernel_wide,
@@ -2978,17 +3111,14 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         const octofmm_status s = launch_stage(c, st, &p, 1);
         if (s != OCTOFMM_OK) return s;
     }
-    if ((stage_mask & 2) && p->root) {
-        RootArgs ra;
-        ra.rec = p->d_rec;
-        ra.tab = c->d_tab;
-        ra.partial = p->d_partial;
-        ra.per_chunk = kCells / kRootChunks;
-        ra.nchunks = kRootChunks;
-        if (p->type == OCTOFMM_RHO)
-            hipLaunchKernelGGL(root_kernel<true>, dim3(kRootChunks), dim3(512), 0, st, ra);
-        else
-            hipLaunchKernelGGL(root_kernel<false>, dim3(kRootChunks), dim3(512), 0, st, ra);
+    if (p->root && (stage_mask & 2)) {
+        const RootArgs ra = root_args(p);
+        if (!p->sums_first) {   // else tree_sums_kernel ran its pairs
+            if (p->type == OCTOFMM_RHO)
+                hipLaunchKernelGGL(root_kernel<true>, dim3(kRootChunks * 2), dim3(256), 0, st, ra);
+            else
+                hipLaunchKernelGGL(root_kernel<false>, dim3(kRootChunks * 2), dim3(256), 0, st, ra);
+        }
         HIPC(c, hipGetLastError());
         RootReduceArgs rr;
         rr.partial = p->d_partial;
@@ -3000,43 +3130,9 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         hipLaunchKernelGGL(root_reduce, dim3((kCells * 23 + 255) / 256), dim3(256), 0, st, rr);
         HIPC(c, hipGetLastError());
     } else if (!p->root && (stage_mask & 30) && p->nitems > 0) {
-        LevelArgs la;
-        la.rec = p->d_rec;
-        la.com = p->d_com;
-        la.L = p->d_L;
-        la.Lc = p->d_Lc;
-        la.nbr = p->d_nbr;
-        la.kind = p->d_kind;
-        la.items = p->d_items;
-        la.tab = c->d_tab;
-        la.mixbits = p->d_mixbits;
-        la.recm = p->d_recm;
-        la.mixorder = p->d_mixorder;
-        la.mix_n64 = p->mix_n64;
-        la.queue = p->d_queue;
-        la.parts = p->wide_parts;
-        la.wide_sums = p->d_wide;
-        la.mon = p->d_mon;
-        la.p2m_out = p->d_p2m_out;
-        la.parent = p->t_parent;
-        la.octant = p->t_octant;
-        la.pL = p->t_pL;
-        la.pLc = p->t_pLc;
-        la.pcom = p->t_pcom;
-        la.g = p->t_g;
-        la.G = p->t_G;
-        la.l2l = p->l2l ? 1 : 0;
-        la.correct_am = p->t_correct_am;
-        la.leaf_rows = p->leaf_rows;
-        la.overwrite = 0;
-        la.xbase = p->d_fxbase;
-        la.dx = p->dx;
-        la.inv_dx = 1.0 / p->dx;
-        la.neg_inv_dx = -1.0 / p->dx;
+        LevelArgs la = level_args(p);
         const bool rho = p->type == OCTOFMM_RHO;
         if ((stage_mask & 18) && p->n_m2l > 0) {
-            la.nitems = p->n_m2l;
-            la.item0 = 0;
             if (p->sums_first) {
                 if (stage_mask & 16) launch_wide_sums(p->n_m2l, st, la, rho);
                 if (stage_mask & 2) launch_wide_reduce(p->n_m2l, st, la, rho);
@@ -3048,12 +3144,6 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
         }
         if ((stage_mask & 8) && p->n_p2m > 0) {
             // the leaf items with p2m lead the leaf items
-            la.nitems = p->n_p2m;
-            la.item0 = p->n_m2l;
-            la.p2m_hdr = p->d_packs;
-            la.p2m_units = p->d_packs + p->packs_units;
-            la.p2m_idx = p->d_packs + p->packs_idx;
-            la.p2m_di = p->d_packs + p->packs_di;
             if (rho)
                 launch_p2m<true>(p->n_packs, st, la, c->tab);
             else
@@ -3061,8 +3151,7 @@ static octofmm_status plan_launch(octofmm_plan* p, hipStream_t st, int stage_mas
             HIPC(c, hipGetLastError());
         }
         if ((stage_mask & 4) && p->nitems > p->n_m2l) {
-            la.nitems = p->nitems - p->n_m2l;
-            la.item0 = p->n_m2l;
+            la = leaf_args(p);
             if (rho)
                 launch_leaf<true>(la.nitems, st, la, c->tab);
             else
@@ -3477,6 +3566,7 @@ static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* 
         plan_free(p);
         return fail(c, s, "%s", what);
     };
+    if (root && in_tree) p->sums_first = true;
     if (!root && p->precision == OCTOFMM_PRECISION_FP64) {
         // (a forced variant runs its plain form in a tree, too)
         if (in_tree && !std::getenv("OCTOFMM_VARIANT")) {
@@ -3774,12 +3864,10 @@ struct octofmm_tree_plan {
     octofmm_tree_stats stats;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
-    // the interactions phase forks onto three more streams: one stages the
-    // partner records of every level, coarsest first; of the other two [0] runs
-    // the leaf kernels and [1] p2m, and both the sums of sums-first levels; the
-    // level kernels stay on the caller's stream
-    hipStream_t side_stage = nullptr, side_leaf[2] = {nullptr, nullptr};
-    hipEvent_t ev_up = nullptr, ev_join_stage = nullptr, ev_join_leaf[2] = {nullptr, nullptr};
+    // the interactions phase forks onto two more streams: [0] stages the larger
+    // levels, [1] runs their p2m and the leaf kernels
+    hipStream_t side[2] = {nullptr, nullptr};
+    hipEvent_t ev_up = nullptr, ev_join[2] = {nullptr, nullptr};
     std::vector<hipEvent_t> ev_stage, ev_level, ev_sums, ev_p2m;
 };
 
@@ -3789,7 +3877,7 @@ void tree_free(octofmm_tree_plan* t) {
     if (!t) return;
     if (t->gexec) (void)hipGraphExecDestroy(t->gexec);
     if (t->graph) (void)hipGraphDestroy(t->graph);
-    for (hipEvent_t e : {t->ev_up, t->ev_join_stage, t->ev_join_leaf[0], t->ev_join_leaf[1]})
+    for (hipEvent_t e : {t->ev_up, t->ev_join[0], t->ev_join[1]})
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : t->ev_stage)
         if (e) (void)hipEventDestroy(e);
@@ -3799,14 +3887,61 @@ void tree_free(octofmm_tree_plan* t) {
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : t->ev_p2m)
         if (e) (void)hipEventDestroy(e);
-    if (t->side_stage) (void)hipStreamDestroy(t->side_stage);
-    for (hipStream_t s : t->side_leaf)
+    for (hipStream_t s : t->side)
         if (s) (void)hipStreamDestroy(s);
     for (auto& l : t->lv) {
         plan_free(l.plan);
         (void)hipFree(l.d_xbase);   // and the tables behind it
     }
     delete t;
+}
+
+// The sums, p2m and root pairs of the n coarsest levels.
+void launch_tree_sums(octofmm_plan* const* plans, int n, hipStream_t st, bool rho, const Tables& tab) {
+    TreeSums g;
+    int blocks = 0;
+    std::memset(&g, 0, sizeof(g));
+    for (int i = 0; i < n; ++i) {
+        const octofmm_plan* p = plans[i];
+        if (p->root) {
+            g.root = root_args(p);
+            blocks += kRootChunks * 2;
+            continue;
+        }
+        g.a[i] = level_args(p);
+        g.sums[i] = p->sums_first ? p->n_m2l * 8 * p->wide_parts : 0;
+        g.packs[i] = p->n_packs;
+        blocks += g.sums[i] + g.packs[i];
+    }
+    if (blocks == 0) return;
+    if (rho && tab.p2p_cube)
+        hipLaunchKernelGGL((tree_sums_kernel<true, true>), dim3(blocks), dim3(256), 0, st, g);
+    else if (rho)
+        hipLaunchKernelGGL((tree_sums_kernel<true, false>), dim3(blocks), dim3(256), 0, st, g);
+    else if (tab.p2p_cube)
+        hipLaunchKernelGGL((tree_sums_kernel<false, true>), dim3(blocks), dim3(256), 0, st, g);
+    else
+        hipLaunchKernelGGL((tree_sums_kernel<false, false>), dim3(blocks), dim3(256), 0, st, g);
+}
+
+// The leaf items of n levels (one, but at theta 0.5).
+octofmm_status launch_leaves(octofmm_tree_plan* t, const int* levels, int n, hipStream_t st) {
+    octofmm_context* c = t->ctx;
+    const bool rho = t->type == OCTOFMM_RHO;
+    LevelArgs la[kLeafLevels];
+    for (int i = 0; i < n; ++i) la[i] = leaf_args(t->lv[levels[i]].plan);
+    if (!c->tab.p2p_cube) {
+        if (rho)
+            launch_leaf<true>(la[0].nitems, st, la[0], c->tab);
+        else
+            launch_leaf<false>(la[0].nitems, st, la[0], c->tab);
+    } else if (rho) {
+        launch_leaf_cube<true>(la, n, st);
+    } else {
+        launch_leaf_cube<false>(la, n, st);
+    }
+    HIPC(c, hipGetLastError());
+    return OCTOFMM_OK;
 }
 
 // phase bit 0: upward pass; bit 1: interactions with the fused downward pass
@@ -3836,68 +3971,89 @@ octofmm_status tree_launch(octofmm_tree_plan* t, hipStream_t st, int phases) {
                 hipLaunchKernelGGL(m2m_kernel<false>, grid, dim3(256), 0, st, a);
             HIPC(c, hipGetLastError());
         }
-    // Interactions of every level, root first.  Each level's kernels also
-    // write the final expansions (the downward pass is fused into them), so
-    // both kernels of level l read the finished non-leaf sub-grids of level
-    // l - 1, which only the level kernel of l - 1 writes: the leaf kernel of
-    // level l waits for that kernel and for its own p2m, and overlaps the level
-    // kernels that follow.  Staging depends only on the upward pass, p2m and
-    // the small levels' sums (sums_first_parts) only on staging: they fill the
-    // chip while the coarse levels, too small for that, pass one after another.
+    // Interactions of every level.  Each level's kernels also write the final
+    // expansions (the downward pass is fused into them), so both kernels of
+    // level l read the finished non-leaf sub-grids of level l - 1, which only
+    // the level kernel of l - 1 writes.
+    //
+    // The coarsest levels, as many as one round of workgroups stages, are a
+    // chain of few and small launches on the caller's stream: their staging in
+    // one, their sums and p2m and the root's pairs in one (tree_sums_kernel), a
+    // reduction per level, and small leaf levels with the next one's.  One
+    // launch follows another there within a microsecond, where a branch and its
+    // join cost about eight.  Larger levels are staged on a second stream; on a third
+    // their p2m runs ahead of all that waits for a coarser level, and the leaf
+    // kernels overlap the level kernels of their own levels.  (A graph puts its
+    // branches on 4 queues in an order of its own, following that of the capture:
+    // with the larger levels captured before the chain, the chain queued behind
+    // their p2m, 1255 us a solve instead of 1211.)
     if (phases & 2) {
-        hipStream_t ss = t->side_stage;
+        bool used[2] = {};
+        hipStream_t ss = t->side[0], sp = t->side[1];
         HIPC(c, hipEventRecord(t->ev_up, st));
-        HIPC(c, hipStreamWaitEvent(ss, t->ev_up, 0));
-        for (hipStream_t sl : t->side_leaf) HIPC(c, hipStreamWaitEvent(sl, t->ev_up, 0));
-        for (int l = 0; l < nl;) {
-            // levels that one round of workgroups stages go in one launch
-            octofmm_plan* group[kStageLevels];
-            int n = 0, slots = 0;
-            while (n < kStageLevels && l + n < nl &&
-                (n == 0 || slots + t->lv[l + n].plan->stage_slots() <= kStageTogether)) {
-                group[n] = t->lv[l + n].plan;
-                slots += group[n++]->stage_slots();
-            }
-            const octofmm_status s = launch_stage(c, ss, group, n);
-            if (s != OCTOFMM_OK) return s;
-            for (; n > 0; --n, ++l) HIPC(c, hipEventRecord(t->ev_stage[l], ss));
+        octofmm_plan* group[kStageLevels];
+        int ng = 0;   // levels of the chain
+        for (int slots = 0; ng < kStageLevels && ng < nl; ++ng) {
+            slots += t->lv[ng].plan->stage_slots();
+            if (ng > 0 && slots > kStageTogether) break;
+            group[ng] = t->lv[ng].plan;
         }
-        // what needs only a level's records: the sums of the small levels and
-        // every level's p2m, ahead of all that waits for a level above
-        for (int l = 0; l < nl; ++l) {
+        octofmm_status s = launch_stage(c, st, group, ng);
+        if (s != OCTOFMM_OK) return s;
+        launch_tree_sums(group, ng, st, t->type == OCTOFMM_RHO, c->tab);
+        HIPC(c, hipGetLastError());
+        for (int l = ng; l < nl; ++l) {
+            if (t->lv[l].plan->stage_slots() == 0) continue;
+            if (!used[0]) HIPC(c, hipStreamWaitEvent(ss, t->ev_up, 0));
+            used[0] = true;
+            s = launch_stage(c, ss, &t->lv[l].plan, 1);
+            if (s != OCTOFMM_OK) return s;
+            HIPC(c, hipEventRecord(t->ev_stage[l], ss));
+        }
+        for (int l = ng; l < nl; ++l) {
             octofmm_plan* p = t->lv[l].plan;
+            if (!p->sums_first && p->n_p2m == 0) continue;
+            HIPC(c, hipStreamWaitEvent(sp, t->ev_stage[l], 0));
+            used[1] = true;
             if (p->sums_first) {
-                hipStream_t sl = t->side_leaf[l & 1];
-                HIPC(c, hipStreamWaitEvent(sl, t->ev_stage[l], 0));
-                const octofmm_status s = plan_launch(p, sl, 16);
+                s = plan_launch(p, sp, 16);
                 if (s != OCTOFMM_OK) return s;
-                HIPC(c, hipEventRecord(t->ev_sums[l], sl));
+                HIPC(c, hipEventRecord(t->ev_sums[l], sp));
             }
             if (p->n_p2m == 0) continue;
-            HIPC(c, hipStreamWaitEvent(t->side_leaf[1], t->ev_stage[l], 0));
-            const octofmm_status s = plan_launch(p, t->side_leaf[1], 8);
+            s = plan_launch(p, sp, 8);
             if (s != OCTOFMM_OK) return s;
-            HIPC(c, hipEventRecord(t->ev_p2m[l], t->side_leaf[1]));
+            HIPC(c, hipEventRecord(t->ev_p2m[l], sp));
         }
+        int leaves[kLeafLevels], nleaves = 0;   // leaf levels not launched yet
         for (int l = 0; l < nl; ++l) {
             octofmm_plan* p = t->lv[l].plan;
-            HIPC(c, hipStreamWaitEvent(st, p->sums_first ? t->ev_sums[l] : t->ev_stage[l], 0));
-            octofmm_status s = plan_launch(p, st, 2);
+            if (l >= ng && p->n_m2l > 0) HIPC(c, hipStreamWaitEvent(st, p->sums_first ? t->ev_sums[l] : t->ev_stage[l], 0));
+            s = plan_launch(p, st, 2);
             if (s != OCTOFMM_OK) return s;
             HIPC(c, hipEventRecord(t->ev_level[l], st));
-            if (!p->root && p->nitems > p->n_m2l) {
-                hipStream_t sl = t->side_leaf[0];
-                if (p->n_p2m > 0) HIPC(c, hipStreamWaitEvent(sl, t->ev_p2m[l], 0));
-                if (l > 0) HIPC(c, hipStreamWaitEvent(sl, t->ev_level[l - 1], 0));
-                s = plan_launch(p, sl, 4);
-                if (s != OCTOFMM_OK) return s;
+            if (p->root || p->nitems == p->n_m2l) continue;
+            // levels of few leaves wait for the next level's launch
+            leaves[nleaves++] = l;
+            const bool more = l + 1 < nl && t->lv[l + 1].plan->nitems > t->lv[l + 1].plan->n_m2l;
+            if (more && c->tab.p2p_cube && p->nitems - p->n_m2l <= kStageTogether && nleaves < kLeafLevels) continue;
+            hipStream_t q = st;
+            if (p->n_m2l > 0) {   // beside this level's multipole targets
+                q = sp;
+                used[1] = true;
+                HIPC(c, hipStreamWaitEvent(sp, t->ev_level[l - 1], 0));
             }
+            for (int k = 0; k < nleaves; ++k)
+                if (leaves[k] >= ng && t->lv[leaves[k]].plan->n_p2m > 0 && q != sp)
+                    HIPC(c, hipStreamWaitEvent(q, t->ev_p2m[leaves[k]], 0));
+            s = launch_leaves(t, leaves, nleaves, q);
+            if (s != OCTOFMM_OK) return s;
+            nleaves = 0;
         }
-        HIPC(c, hipEventRecord(t->ev_join_stage, ss));
-        HIPC(c, hipStreamWaitEvent(st, t->ev_join_stage, 0));
         for (int k = 0; k < 2; ++k) {
-            HIPC(c, hipEventRecord(t->ev_join_leaf[k], t->side_leaf[k]));
-            HIPC(c, hipStreamWaitEvent(st, t->ev_join_leaf[k], 0));
+            if (!used[k]) continue;
+            HIPC(c, hipEventRecord(t->ev_join[k], t->side[k]));
+            HIPC(c, hipStreamWaitEvent(st, t->ev_join[k], 0));
         }
     }
     return OCTOFMM_OK;
@@ -3978,10 +4134,9 @@ octofmm_status octofmm_tree_plan_create(octofmm_context* c, const octofmm_tree* 
         return fail(c, s, "%s", what);
     };
     {
-        bool ok = hipStreamCreateWithFlags(&t->side_stage, hipStreamNonBlocking) == hipSuccess &&
-                  hipStreamCreateWithFlags(&t->side_leaf[0], hipStreamNonBlocking) == hipSuccess &&
-                  hipStreamCreateWithFlags(&t->side_leaf[1], hipStreamNonBlocking) == hipSuccess;
-        for (hipEvent_t* e : {&t->ev_up, &t->ev_join_stage, &t->ev_join_leaf[0], &t->ev_join_leaf[1]})
+        bool ok = hipStreamCreateWithFlags(&t->side[0], hipStreamNonBlocking) == hipSuccess &&
+                  hipStreamCreateWithFlags(&t->side[1], hipStreamNonBlocking) == hipSuccess;
+        for (hipEvent_t* e : {&t->ev_up, &t->ev_join[0], &t->ev_join[1]})
             ok = ok && hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess;
         for (int l = 0; l < nl; ++l)
             ok = ok && hipEventCreateWithFlags(&t->ev_stage[l], hipEventDisableTiming) == hipSuccess &&

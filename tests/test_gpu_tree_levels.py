@@ -1,8 +1,10 @@
 """Whole-tree solves whose small levels run sums first (up to 96 targets, in 1
-to 7 workgroups per coarse block) against the plain form of the same kernels
+to 7 workgroups per coarse block), in the launches that the coarsest levels
+share or beyond them, against the plain form of the same kernels
 (OCTOFMM_VARIANT), with levels of 1 to 97 targets, leaves and refined
-neighbours on every side; RHO and DRHODT, with and without a graph, with and
-without the leaves' rows; a repeated solve gives the same bits.
+neighbours on every side, small leaf levels that go with the next one's launch;
+RHO and DRHODT, with and without a graph, with and without the leaves' rows; a
+repeated solve gives the same bits.
 
 Tolerance: the two forms differ in the order of the sums over partners only,
 1e-12 as elsewhere.
@@ -50,20 +52,30 @@ def solve(t, theta, type_, flags):
     return out[-1]
 
 
-@pytest.mark.parametrize("sizes", [(0, 0, 0), (1, 0, 0), (8, 3, 0), (8, 64, 96), (8, 64, 97)])
-@pytest.mark.parametrize("theta", [0.5, 0.34])
-@pytest.mark.parametrize("type_", [_abi.RHO, _abi.DRHODT])
-def test_sums_first_matches_plain(monkeypatch, type_, theta, sizes):
-    t = tree_with(*sizes)
+def compare(monkeypatch, t, theta, type_, flags):
     print([int((lv.kind == _abi.SLOT_NONLEAF).sum()) for lv in t.levels], flush=True)
-    flags = _abi.PLAN_USE_GRAPH if sizes[1] else 0
-    if sizes[0] == 1:
-        flags |= _abi.TREE_LEAF_G_ONLY
     got = solve(t, theta, type_, flags)
     monkeypatch.setenv("OCTOFMM_VARIANT", "702")
     ref = solve(t, theta, type_, flags)
-    for lv, g, r in zip(t.levels, got, ref):
+    for g, r in zip(got, ref):
         for k in g:
             assert np.isfinite(g[k]).all()
             if np.abs(r[k]).max() > 0.0:
                 assert normwise(g[k], r[k]) <= TOL
+
+
+@pytest.mark.parametrize("sizes", [(0, 0, 0), (1, 0, 0), (8, 3, 0), (8, 64, 96), (8, 64, 97)])
+@pytest.mark.parametrize("theta", [0.5, 0.34])
+@pytest.mark.parametrize("type_", [_abi.RHO, _abi.DRHODT])
+def test_sums_first_matches_plain(monkeypatch, type_, theta, sizes):
+    flags = _abi.PLAN_USE_GRAPH if sizes[1] else 0
+    if sizes[0] == 1:
+        flags |= _abi.TREE_LEAF_G_ONLY
+    compare(monkeypatch, tree_with(*sizes), theta, type_, flags)
+
+
+def test_small_leaf_level_after_large_ones(monkeypatch):
+    t = tree_with(8, 64, 280)
+    leaves = [int((lv.kind == _abi.SLOT_LEAF).sum()) for lv in t.levels]
+    assert sum(lv.nnodes for lv in t.levels[:4]) > 256 and 0 < leaves[3] <= 256 < leaves[4]
+    compare(monkeypatch, t, 0.5, _abi.RHO, _abi.PLAN_USE_GRAPH)

@@ -1740,10 +1740,12 @@ void launch_wide_reduce(int nitems, hipStream_t st, const LevelArgs& la, bool rh
 // other (329-sub-grid tree: 160 -> 125 us a solve, 10,697: 1338 -> 1307).  Larger
 // levels fill the chip by themselves, and their sums would cost as much traffic
 // as their results.  Workgroups per coarse block of such a level, 0 for a larger
-// one.
+// one: the levels fill the chip together, so a split as fine as wide_parts makes
+// of a level by itself only adds sums (95.7 us, against 90.0 with at least 8
+// entries, two images a wave, to a part and two workgroups a CU from one level).
 int sums_first_parts(int n, const Tables& tab) {
     if (n <= 0 || n > 96) return 0;
-    return std::max(1, std::min((tab.nsched + 3) / 4, 96 / n));
+    return std::max(1, std::min(tab.nsched / 8, 64 / n));
 }
 
 // Persistent form of the mapping-7 kernel (variants 804, 802): a grid of

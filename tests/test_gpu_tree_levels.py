@@ -1,5 +1,5 @@
-"""Whole-tree solves whose small levels run sums first (up to 96 targets, in 1
-to 7 workgroups per coarse block), in the launches that the coarsest levels
+"""Whole-tree solves whose small levels run sums first (up to 96 targets, in one
+to several workgroups per coarse block), in the launches that the coarsest levels
 share or beyond them, against the plain form of the same kernels
 (OCTOFMM_VARIANT), with levels of 1 to 97 targets, leaves and refined
 neighbours on every side, small leaf levels that go with the next one's launch;

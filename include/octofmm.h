@@ -234,7 +234,8 @@ typedef struct octofmm_level {
  * 804, 802), fixes that variant
  * for every plan created while it is set, in place of the default or the
  * autotuner's choice.  All variants give the same results to rounding; it
- * exists for measurement.
+ * exists for measurement.  Without it whole-tree plans run FP64 levels of up to
+ * 96 multipole targets in a form of variant 704 of their own, untimed.
  * With OCTOFMM_PLAN_AUTOTUNE the choice is cached by level shape (device
  * architecture and CU count, solve type, precision, opening angle, counts of
  * multipole-target items with and without leaf neighbours, fused downward pass

@@ -534,8 +534,8 @@ __device__ __forceinline__ void near_pairs(const LevelArgs& a, const LaneGeom& g
         if (__builtin_amdgcn_ballot_w64(nb != 0) == 0) continue;
         // the 8 partners' loads in flight together: one after another the
         // waits for them were most of what a block beside leaves took longer
-        // (a 2048-slot level of mixed kinds takes 730 us in place of 760, a
-        // 105-slot one at theta 0.34 226 in place of 238)
+        // (a 2048-slot level of mixed kinds takes 755 us in place of 790, a
+        // 105-slot one at theta 0.34 227 in place of 244)
         double q[8][4];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {

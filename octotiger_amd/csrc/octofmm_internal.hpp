@@ -38,7 +38,7 @@ struct Tables {
     int8_t delta[kMaxDelta][4];       // coarse offsets (x, y, z, 0)
     uint64_t farbits[kMaxDelta];      // byte k: bit j set if (delta, j, k) is far
     uint64_t nearbits[kMaxDelta];     // byte k: bit j set if (delta, j, k) is near (self excluded)
-    uint64_t allrows[kMaxDelta];      // farbits | nearbits transposed: byte j, bit k
+    uint64_t allrows[kMaxDelta];      // farbits | nearbits transposed: byte j, bit k (host checks)
     int32_t nfar_delta;               // coarse offsets with a far pair for some child class,
     int32_t far_delta[kMaxDelta];     // in delta order (delta 0 has none: it is all near / self)
     // Far schedule of the direct-staging kernels: one staged image of 8
@@ -109,7 +109,7 @@ struct Tables {
 //   mapping 0: a wave owns a 2x2x2 block of coarse cells, lane = (coarse cell,
 //              child); the 8 lanes of a coarse cell share every partner load
 //              (8, 4, 2 waves per workgroup).  The per-sub-grid drop-ins run
-//              variant 8.
+//              mapping 7's split form for one target (level_kernel_wide).
 //   mapping 3: the partner records of each coarse offset staged once per wave
 //              in LDS by direct global->LDS loads and read back as 8-lane
 //              broadcasts; 4 or 2 waves per workgroup so that 3 waves per
@@ -118,9 +118,9 @@ struct Tables {
 //              waves (variant 504), for levels with few sub-grids.
 //   mapping 7: mapping 3's staging with the coarse offsets of a block split
 //              over 4, 2 or 8 waves (variants 704, 702, 708); the partial sums
-//              meet in the waves' images.  On small FP64 levels 704
-//              splits each block further over several workgroups (wide_parts).  The 8-wave split (one workgroup per
-//              CU by its LDS) is for levels with very few sub-grids.
+//              meet in the waves' images.  On small FP64 levels 704 splits
+//              each block further over several workgroups (wide_parts).  The
+//              8-wave split has one workgroup per CU by its LDS.
 //   mapping 8: mapping 7 as one persistent grid over per-XCD work counters
 //              (variants 804, 802).
 // Mappings 1, 2 and 4 were measured and are not built (slower than mapping 3

@@ -2284,6 +2284,25 @@ constexpr int kRootChunks = 64;
 struct P2mPacks {
     std::vector<int32_t> hdr, units, idx, di;
     int npacks() const { return (int)hdr.size() / 2; }
+    // while they are made: one coarse cell of one item with n entries from
+    // `first` on in rec and off, and the order of the units in the packs
+    struct Unit {
+        int32_t id, first, n;
+    };
+    std::vector<Unit> unit;
+    std::vector<int32_t> rec, off, order;
+    // room for any one item, so that a call with one makes them without allocating
+    void reserve_one() {
+        const size_t entries = (size_t)64 * kMaxDelta;
+        hdr.reserve(2 * 8);
+        units.reserve(64);
+        idx.reserve(entries);
+        di.reserve(entries);
+        unit.reserve(64);
+        rec.reserve(entries);
+        off.reserve(entries);
+        order.reserve(64);
+    }
 };
 
 // The coarse cells of a sub-grid that reach into its neighbour in direction
@@ -2314,11 +2333,11 @@ void build_p2m_reach(const Tables& T, P2mReach& r) {
 // equal, so a pack's 8 units are of like length and near each other.
 template <typename F>
 void build_p2m_packs(const P2mReach& reach, int nitems, F&& refined, P2mPacks& out) {
-    struct Unit {
-        int32_t id, first, n;
-    };
-    std::vector<Unit> units;
-    std::vector<int32_t> rec, di;   // the units' entries, one unit after another
+    std::vector<P2mPacks::Unit>& units = out.unit;
+    std::vector<int32_t>&rec = out.rec, &di = out.off, &order = out.order;
+    units.clear();
+    rec.clear();
+    di.clear();
     for (int o = 0; o < nitems; ++o) {
         int slot[27], count[64] = {}, at[64];
         for (int raw = 0; raw < 27; ++raw) {
@@ -2343,9 +2362,9 @@ void build_p2m_packs(const P2mReach& reach, int nitems, F&& refined, P2mPacks& o
         }
     }
     int end_of[kMaxDelta + 2] = {};   // counting sort: units of n entries lie before end_of[n]
-    for (const Unit& u : units) ++end_of[u.n];
+    for (const P2mPacks::Unit& u : units) ++end_of[u.n];
     for (int n = kMaxDelta; n >= 0; --n) end_of[n] += end_of[n + 1];
-    std::vector<int32_t> order(units.size());
+    order.resize(units.size());
     for (size_t u = units.size(); u-- > 0;) order[--end_of[units[u].n]] = (int32_t)u;
     const size_t npacks = (units.size() + 7) / 8;
     out.hdr.resize(2 * npacks);
@@ -2358,7 +2377,7 @@ void build_p2m_packs(const P2mReach& reach, int nitems, F&& refined, P2mPacks& o
     out.idx.assign((size_t)rows * 8, -1);
     out.di.assign((size_t)rows * 8, 0);
     for (size_t q = 0; q < order.size(); ++q) {
-        const Unit& u = units[order[q]];
+        const P2mPacks::Unit& u = units[order[q]];
         out.units[q] = u.id;
         const size_t first = (size_t)out.hdr[2 * (q / 8)] * 8 + q % 8;
         for (int e = 0; e < u.n; ++e) {
@@ -2474,6 +2493,7 @@ struct octofmm_context {
     double* h_pin = nullptr;       // results [512][20], [512][3], the packed inputs, p2m work lists
     int reach = 0;                 // cells of a neighbour within the stencil's reach, per axis
     P2mReach p2m_reach;
+    P2mPacks p2m_packs;            // work lists of a call
 };
 
 // doubles of the results at the front of the pinned memory, and the cells its
@@ -2707,7 +2727,7 @@ void pack_subgrid(octofmm_context* c, const octofmm_subgrid* in, bool leaf_targe
 // The p2m work lists of a packed leaf target, into the pinned memory behind
 // the inputs: hdr, units, idx, di.  Returns the number of packs.
 int pack_p2m(octofmm_context* c, PackedArgs& pa) {
-    P2mPacks pk;
+    P2mPacks& pk = c->p2m_packs;
     build_p2m_packs(c->p2m_reach, 1,
         [&](int, int raw) { return pa.kind[packed_slot(raw)] == OCTOFMM_SLOT_NONLEAF ? packed_slot(raw) : -1; }, pk);
     int32_t* dst = reinterpret_cast<int32_t*>(c->h_pin + kPinOut + pin_cells(c->tab) * 23);
@@ -2876,6 +2896,7 @@ octofmm_status octofmm_create(const octofmm_config* cfg, octofmm_context** out) 
     }
     c->reach = 2 * c->tab.max_delta;
     build_p2m_reach(c->tab, c->p2m_reach);
+    c->p2m_packs.reserve_one();
     c->d_scratch = scratch_address(c->device);
     if (!c->d_scratch) {
         octofmm_destroy(c);

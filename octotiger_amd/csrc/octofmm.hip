@@ -1704,13 +1704,18 @@ __global__ __launch_bounds__(64) void level_reduce(LevelArgs a) {
 
 // Workgroups per coarse block of variant 704 on a level of n targets (0: the
 // plain form).  The sums' way through memory and the second kernel cost ~5 us,
-// about what two images take: with the 26 images of theta 0.5 the split pays
-// up to 1.75 workgroups per CU (27 targets: 26.3 us plain, 27.3 in two parts),
-// with the 92 of theta 0.34 up to three (36 targets: 109 -> 89 us, 45: 111 ->
-// 94 us, 64 in two parts: 122 -> 125 us).  At most one image per wave.
+// about what two images take, and a second workgroup on some CUs takes back part
+// of what a split saves.  With the 26 entries of theta 0.5 two parts take three
+// images off a wave: 20 targets 26.3 us plain, 26.1 in two parts, 22 targets
+// 26.4 and 26.4, 24 targets 26.3 and 27.0, 28 targets 26.4 and 27.5, so they end
+// at 22.  With the 32 of theta 0.45 they take off four: 28 targets 31.0 and 29.3,
+// and the split ends at 1.75 workgroups per CU.  With the 92 of theta 0.34 it
+// pays up to three (36 targets: 109 and 88 us, 48: 110 and 93 us, 49: 110 and
+// 117 us).  At most one image per wave.
 int wide_parts(int n, const Tables& tab) {
     if (n <= 0) return 0;
     const int parts = std::min((tab.nsched + 3) / 4, (tab.nsched < 48 ? 448 : 768) / (8 * n));
+    if (parts == 2 && n > 22 && tab.nsched < 32) return 0;
     return parts >= 2 ? parts : 0;
 }
 

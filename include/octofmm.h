@@ -241,7 +241,8 @@ typedef struct octofmm_level {
  * multipole-target items with and without leaf neighbours, fused downward pass
  * or not): a plan of a shape seen before in the process takes the cached
  * variant without timing.  When the environment variable OCTOFMM_TUNE_CACHE
- * names a file, the cache is read from it and each new choice appended to it. */
+ * names a file, the cache is read from it and each new choice appended to it;
+ * choices that a library built from other kernel sources wrote are passed over. */
 /* The level is the root sub-grid alone (nslots = ntargets = 1, non-leaf):
  * every pair of its cells except self and near offsets, the root stencil of
  * octotiger/multipole_interactions/kernel/kokkos_kernel.hpp:324-471, 637-764.

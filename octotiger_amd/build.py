@@ -3,7 +3,9 @@
     python -m octotiger_amd.build          # library
     python -m octotiger_amd.build --asm    # also dump the gfx950 assembly to _build/
 """
+import hashlib
 import os
+import re
 import subprocess
 import sys
 
@@ -28,6 +30,26 @@ def hipcc():
     return os.path.join(rocm, "bin", "hipcc")
 
 
+def source_id(texts):
+    """12 hex digits that name the code in the given C++ texts: comments and
+    blank space do not count."""
+    h = hashlib.sha256()
+    for t in texts:
+        t = re.sub(r"//[^\n]*|/\*.*?\*/", " ", t, flags=re.S)
+        h.update(" ".join(t.split()).encode() + b"\0")
+    return h.hexdigest()[:12]
+
+
+def kernel_id():
+    """Names the kernels this tree builds: the library's sources and the flags
+    they are compiled with."""
+    texts = []
+    for f in SOURCES + HEADERS:
+        with open(os.path.join(CSRC, f)) as src:
+            texts.append(src.read())
+    return source_id(texts + [" ".join(HIP_FLAGS)])
+
+
 def build(verbose=True, asm=False):
     inc = ["-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
     objs = []
@@ -36,7 +58,8 @@ def build(verbose=True, asm=False):
     for src in SOURCES:
         obj = os.path.join(bdir, src + ".o")
         lang = ["-x", "hip"]
-        cmd = [hipcc()] + HIP_FLAGS + inc + lang + ["-c", os.path.join(CSRC, src), "-o", obj]
+        cmd = [hipcc()] + HIP_FLAGS + inc + lang + [f'-DOCTOFMM_KERNEL_ID="{kernel_id()}"', "-c",
+                                                    os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.run(cmd, check=True)

@@ -3245,12 +3245,17 @@ static void set_mixed_count(octofmm_plan* p) {
 
 // Tuning cache: the variant the autotuner chose, keyed by level shape (device
 // architecture, solve type, precision, opening angle, counts of multipole-target
-// items with and without a near pass, fused downward pass or not).  A plan of a
+// items with and without a near pass, fused downward pass or not) and by the
+// kernels the choice was timed on: the build gives their sources an id, so that
+// entries a file holds from other kernels are passed over.  A plan of a
 // shape seen before takes the cached choice without timing anything, so plans
 // of one shape run the same kernel, and give the same bits, within a process.
 // When the environment variable OCTOFMM_TUNE_CACHE names a file, the cache is
 // read from it at the first lookup and every new choice is appended to it
 // (one "key variant" line each), so the choices also hold across processes.
+#ifndef OCTOFMM_KERNEL_ID
+#define OCTOFMM_KERNEL_ID "0"
+#endif
 namespace {
 std::mutex g_tune_mu;
 std::vector<std::pair<std::string, int>> g_tune;
@@ -3263,10 +3268,10 @@ std::string tune_key(const octofmm_plan* p) {
     for (const int2& it : p->h_items)
         if (!(it.y & kItemLeaf) && (it.y & kItemNear)) ++near;
     char buf[256];
-    std::snprintf(buf, sizeof(buf), "%s/cu%d/t%d/p%d/d%d/th%.17g/m%d/n%d/l%d", arch,
+    std::snprintf(buf, sizeof(buf), "%s/cu%d/t%d/p%d/d%d/th%.17g/m%d/n%d/l%d/k%s", arch,
         hipGetDeviceProperties(&prop, p->ctx->device) == hipSuccess ? prop.multiProcessorCount : 0, p->type,
         p->precision, p->precision == OCTOFMM_PRECISION_MIXED ? p->mixed_far_d2 : 0, p->ctx->theta, p->n_m2l, near,
-        p->l2l ? 1 : 0);
+        p->l2l ? 1 : 0, OCTOFMM_KERNEL_ID);
     for (char* q = buf; *q; ++q)
         if (*q == ' ') *q = '_';
     return buf;

@@ -34,8 +34,10 @@ sys.path.insert(0, ROOT)
 METRIC = "cell-interactions/s FP64 vs mixed-prec, % VALU peak, rel. force err vs FP64"
 FP64_VALU_PEAK_TFLOPS = 78.6     # MI355X FP64 vector, dense
 HBM_PEAK_TBS = 8.0               # MI355X HBM3E
-FLOPS_PER_PAIR = {"rho": 407, "drhodt": 273}
-EXECUTED_FLOPS_PER_PAIR = 189   # of the RHO kernels
+FLOPS_PER_PAIR = {"rho": 407, "drhodt": 273}   # nominal: the operations of the reference's source
+# FP64 operations a far pair of the RHO kernels executes (76 FMA, 33 MUL and 4 ADD
+# in the gfx950 assembly, FMA = 2): what a share of a hardware rate is taken of
+EXECUTED_FLOPS_PER_PAIR = 189
 CPU_THREADS_MAX = 16             # host threads one GPU's share of the box gives a process
 
 
@@ -59,6 +61,23 @@ def staging_bytes(lv, stats):
     uniform level: per cell 184 bytes read (M, com) and a 192-byte record
     written."""
     return lv.nslots * 512 * (184 + 192)
+
+
+def executed_tflops(far_pairs, ms):
+    """FP64 rate of an RHO interaction kernel over far pairs alone."""
+    return far_pairs * EXECUTED_FLOPS_PER_PAIR / (ms * 1e-3) / 1e12
+
+
+def measured_traffic(level, variant, kernels, where=os.path.join(ROOT, "profiles")):
+    """HBM bytes per launch of a level's kernel variant, from the calibrated
+    FETCH_SIZE / WRITE_SIZE counter runs kept beside the profiles, or None where
+    no run measured these kernels (`kernels`: octotiger_amd.build.kernel_id)."""
+    path = os.path.join(where, f"traffic_{level}_v{variant}.json")
+    if not os.path.exists(path):
+        return None
+    with open(path) as f:
+        run = json.load(f)
+    return run["hbm_bytes_per_launch"] if run.get("kernel_id") == kernels else None
 
 
 def kernel_name(variant, rho=True):
@@ -286,7 +305,7 @@ def run_tree(ctx, args, hip, _abi, np):
         "fp64": {"ms_per_solve": res["fp64"]["ms_per_solve"], "phases_ms": res["fp64"]["phases_ms"],
                  "leaf_g_only_ms_per_solve": res["fp64"]["leaf_g_only_ms_per_solve"],
                  "cell_interactions_per_s": pairs / (res["fp64"]["ms_per_solve"] * 1e-3),
-                 "interaction_valu_frac": st["flops"] / (inter * 1e-3) / 1e12 / FP64_VALU_PEAK_TFLOPS,
+                 "interaction_nominal_tflops": st["flops"] / (inter * 1e-3) / 1e12,
                  "plan_create_s": res["fp64"]["plan_create_s"],
                  "production_step": res["fp64"]["production_step"]},
         "mixed": {"ms_per_solve": res["mixed"]["ms_per_solve"], "phases_ms": res["mixed"]["phases_ms"],
@@ -382,7 +401,7 @@ def main():
         sys.exit(2)
     import numpy as np
 
-    from octotiger_amd import _abi, hip, native, workloads
+    from octotiger_amd import _abi, build, hip, native, workloads
 
     sys.path.insert(0, os.path.join(ROOT, "tests"))
 
@@ -416,15 +435,8 @@ def main():
     ms_step = c4["fp64"]["ms_per_step"]
     value = pairs / (ms_step * 1e-3)
     k_ms = c4["fp64"]["stage_ms"][1]
-    achieved = st["flops"] / (k_ms * 1e-3) / 1e12
-
-    traffic = None
-    # HBM bytes per launch of this kernel variant, from the calibrated
-    # FETCH_SIZE / WRITE_SIZE counter runs kept beside the profiles
-    tpath = os.path.join(ROOT, "profiles", f"traffic_{lv.name}_v{int(st['variant'])}.json")
-    if os.path.exists(tpath):
-        with open(tpath) as f:
-            traffic = json.load(f).get("hbm_bytes_per_launch")
+    achieved = executed_tflops(st["far_pairs"], k_ms)
+    traffic = measured_traffic(lv.name, int(st["variant"]), build.kernel_id())
 
     cpu = cpu_baseline(lv, pairs // len(lv.targets), args) if args.cpu_repeats > 0 else None
 
@@ -473,7 +485,7 @@ def main():
             "value": p2 / (c2["fp64"]["ms_per_step"] * 1e-3), "ms_per_step": c2["fp64"]["ms_per_step"],
             "kernel_ms": k2, "staging_ms": c2["fp64"]["stage_ms"][0], "kernel_variant": int(s2["variant"]),
             "kernel": kernel_name(int(s2["variant"])),
-            "valu_frac": s2["flops"] / (k2 * 1e-3) / 1e12 / FP64_VALU_PEAK_TFLOPS,
+            "valu_frac": executed_tflops(s2["far_pairs"], k2) / FP64_VALU_PEAK_TFLOPS,
             "mixed": {"ms_per_step": c2["mixed"]["ms_per_step"], "kernel_ms": c2["mixed"]["stage_ms"][1],
                       "speedup_vs_fp64": c2["fp64"]["ms_per_step"] / c2["mixed"]["ms_per_step"],
                       "kernel_variant": int(c2["mixed"]["stats"]["variant"]),
@@ -492,7 +504,7 @@ def main():
                  "ms_per_step": ms3, "kernel_ms": c3["fp64"]["stage_ms"][1],
                  "cell_interactions_per_s": p3 / (ms3 * 1e-3),
                  "pairs": {k: int(s3[k]) for k in ("far_pairs", "near_pairs", "p2p_pairs", "p2m_pairs")},
-                 "valu_frac": s3["flops"] / (c3["fp64"]["stage_ms"][1] * 1e-3) / 1e12 / FP64_VALU_PEAK_TFLOPS,
+                 "nominal_tflops": s3["flops"] / (c3["fp64"]["stage_ms"][1] * 1e-3) / 1e12,
                  "kernel_variant": int(s3["variant"]), "production_step": c3["production_step"]}
 
     # dense vector FMA rates of this device: FP64, and FP32 as all device code
@@ -535,11 +547,11 @@ def main():
             "peak": FP64_VALU_PEAK_TFLOPS,
             "unit": "TFLOP/s",
             "frac": achieved / FP64_VALU_PEAK_TFLOPS,
-            # achieved counts the reference's source operations (407 a pair);
-            # the kernel executes fewer: 76 FMA, 33 MUL and 4 ADD
             "executed_flops_per_pair": EXECUTED_FLOPS_PER_PAIR,
-            "achieved_executed": achieved * EXECUTED_FLOPS_PER_PAIR / FLOPS_PER_PAIR["rho"],
-            "frac_executed": achieved * EXECUTED_FLOPS_PER_PAIR / FLOPS_PER_PAIR["rho"] / FP64_VALU_PEAK_TFLOPS,
+            # the rate in the reference's source operations, of which the kernel
+            # executes fewer: no share of a hardware rate
+            "nominal_flops_per_pair": FLOPS_PER_PAIR["rho"],
+            "nominal_tflops": st["flops"] / (k_ms * 1e-3) / 1e12,
             "traffic": traffic,
             "kernel_ms": k_ms,
             "staging_ms": c4["fp64"]["stage_ms"][0],

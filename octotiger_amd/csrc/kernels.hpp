@@ -1,12 +1,12 @@
 // kernels.hpp -- gfx950 device code of liboctofmm: FP64 pair arithmetic, the
-// AoS->record staging kernel, the level interaction kernel and the root kernel.
+// FP32 pairs of mixed precision, kernel arguments and the tree passes' shifts.
 //
-// Pair arithmetic follows Octo-Tiger's templates
+// Pair arithmetic gives what Octo-Tiger's templates give
 // (octotiger/multipole_interactions/kernel/compute_kernel_templates.hpp:67-391,
 //  octotiger/monopole_interactions/kernel/monopole_kernel_templates.hpp:16-239):
-// the same derivative tensor D of -1/r, the same order-3 contraction with
-// multiplicity factors, and the same angular-momentum correction from the
-// order-4 tensor.  Only the summation order over pairs differs.
+// the order-3 contraction of a partner's moments with the derivatives of -1/r,
+// and the angular-momentum correction from the order-4 ones.  The FP64 pairs
+// form no derivative tensor for it (see below); the FP32 pairs do.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -381,13 +381,6 @@ __device__ __forceinline__ double cell_centre(double xb, int i, double dx) {
     return xb + (double)i * dx;
 }
 
-// Result of one target cell.  Level plans accumulate L (ncomp components:
-// 20 for M2L targets, 4 for leaves) and overwrite L_c when the kernel forms
-// it (write_c).  In a whole-tree solve the cell's final expansion is written
-// directly: interactions + the parent cell's expansion re-expanded about the
-// cell's centre of mass (taylor::operator<<=, grid::compute_expansions,
-// src/grid_fmm.cpp:1524-1637), L_c + the parent's L_c, and for leaf cells
-// phi = G L0 and g = -G (L_1..3 + L_c).
 // The final expansion of a cell in a whole-tree solve: its interactions plus
 // the parent cell's expansion re-expanded about the cell's centre of mass, and
 // L_c plus the parent's L_c.
@@ -2962,11 +2955,11 @@ octofmm_status octofmm_compute_multipole_interactions(octofmm_context* c, const 
 }
 
 // The same call with the workspace in `scratch` instead of the context's
-// allocation: the same kernels and copies, no device allocation.  Every
-// region the kernels read is written by this call first (the target and
-// handed-over neighbour slots, partial halos zeroed before their scatter, the
-// metadata; empty directions are marked absent and never read), so what a
-// previous call left in the scratch does not enter the result.
+// allocation: the same kernels, no device allocation.  What enters the result
+// is written by this call first: the target, of each neighbour handed over the
+// cells within the stencil's reach (partial halos expanded by the host, zeros
+// in the cells they do not list) and the metadata; empty directions are marked
+// absent, so what a previous call left in the scratch does not enter the result.
 octofmm_status octofmm_compute_multipole_interactions_noalloc(octofmm_context* c, const octofmm_subgrid* in,
     double* L, double* L_c) {
     if (!c) return OCTOFMM_ERR_INVALID_ARGUMENT;
@@ -3601,7 +3594,7 @@ static octofmm_status level_plan_build(octofmm_context* c, const octofmm_level* 
     };
     if (root && in_tree) p->sums_first = true;
     if (!root && p->precision == OCTOFMM_PRECISION_FP64) {
-        // (a forced variant runs its plain form in a tree, too)
+        // (a forced variant runs in a tree as it does in a level plan)
         if (in_tree && !std::getenv("OCTOFMM_VARIANT")) {
             p->wide_parts = sums_first_parts(n_m2l, T);
             p->sums_first = p->wide_parts > 0;

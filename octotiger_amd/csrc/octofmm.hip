@@ -1701,14 +1701,17 @@ __global__ __launch_bounds__(64) void level_reduce(LevelArgs a) {
 // of what a split saves.  With the 26 entries of theta 0.5 two parts take three
 // images off a wave: 20 targets 26.3 us plain, 26.1 in two parts, 22 targets
 // 26.4 and 26.4, 24 targets 26.3 and 27.0, 28 targets 26.4 and 27.5, so they end
-// at 22.  With the 32 of theta 0.45 they take off four: 28 targets 31.0 and 29.3,
-// and the split ends at 1.75 workgroups per CU.  With the 92 of theta 0.34 it
-// pays up to three (36 targets: 109 and 88 us, 48: 110 and 93 us, 49: 110 and
-// 117 us).  At most one image per wave.
+// at 22; shorter schedules (theta above 0.577) save less and end at 16 (theta
+// 0.6: 16 targets 21.0 and 18.0 us, 20 targets 21.1 and 22.8; theta 0.75: 8
+// targets 11.3 and 10.7, 16 targets 11.4 and 11.5, 22 targets 11.6 and 13.9).
+// With the 32 of theta 0.45 they take off four: 28 targets 31.0 and 29.3 us, and
+// the split ends at 1.75 workgroups per CU.  With the 92 of theta 0.34 it pays up
+// to three (36 targets: 109 and 88 us, 48: 110 and 93, 49: 110 and 117).  At most
+// one image per wave.
 int wide_parts(int n, const Tables& tab) {
     if (n <= 0) return 0;
     const int parts = std::min((tab.nsched + 3) / 4, (tab.nsched < 48 ? 448 : 768) / (8 * n));
-    if (parts == 2 && n > 22 && tab.nsched < 32) return 0;
+    if (parts == 2 && tab.nsched < 32 && n > (tab.nsched < 26 ? 16 : 22)) return 0;
     return parts >= 2 ? parts : 0;
 }
 

@@ -1,10 +1,10 @@
 """Where variant 704 stops splitting the coarse blocks of a small level over several
-workgroups: the largest level it splits and the smallest it does not, at the three
+workgroups: the largest level it splits and the smallest it does not, at the
 lengths of the far schedule, with leaf neighbours (near pairs), against the oracle
 and against variant 702.  An unsplit level runs the same sums as the persistent form
 804, 4 waves a block in wave order, so the two give the same bits: at theta 0.5 two
 parts are slower than the plain form from 24 targets on (27.0 us against 26.3) and
-must not be taken there.
+must not be taken there, at theta 0.6 and 0.75 from fewer on.
 
 Tolerance: only the order of the sums over pairs differs, 1e-12 as elsewhere.
 """
@@ -47,6 +47,7 @@ def one_pass(dl, ctx, s, type_):
     (0.5, 22, True), (0.5, 23, False), (0.5, 28, False), (0.5, 29, False),
     (0.45, 28, True), (0.45, 29, False),
     (0.34, 36, True), (0.34, 48, True), (0.34, 49, False),
+    (0.6, 18, True), (0.6, 19, False), (0.75, 16, True), (0.75, 17, False),
 ])
 def test_split_ends_where_it_stops_paying(theta, n, split, monkeypatch):
     lv = strip(n)
